@@ -1150,9 +1150,7 @@ static bool decode_tiled_grouped_pays(int x_bits, int w_bits, int M, int N, int 
     if (M > 128)
         return false;
     const int t = act ? 2 : 1;
-    const int mrows = decode_tiled_grouped_rows(16, t, M, K, x_bits);
-    if (mrows == 0)
-        return false;
+    const int mrows = 16;
     const double blocks = (M + mrows - 1) / mrows;
     const double w_mb = (double)N * K * w_bits / 8e6;
     const double x_mb = (double)((N + 16 * t - 1) / (16 * t)) * mrows * K * x_bits / 8e6;
@@ -1174,7 +1172,6 @@ static bool decode_tiled_grouped_fits(const abq_gemm_state *st, int group_size, 
     const abq_tile_config &c = st->cfg;
     const KernelTable *t = find_table(registry().decode_tiled_grouped, c.x_bits, c.w_bits, c.is_signed);
     return t && t->count > 0 && st->auto_chosen && (group_size == 128 || group_size == 64) && (!act || st->N % 32 == 0) &&
-           decode_tiled_grouped_rows(16, act ? 2 : 1, st->M, st->K, c.x_bits, group_size) != 0 &&
            decode_tiled_grouped_pays(c.x_bits, c.w_bits, st->M, st->N, st->K, act, group_size);
 }
 
@@ -1937,7 +1934,6 @@ int abq_prepared_decode_pays(int x_bits, int w_bits, int is_signed, int M, int N
     if (group_size) {
         const KernelTable *t = find_table(reg.decode_tiled_grouped, x_bits, w_bits, is_signed);
         return t && t->count > 0 && (group_size == 128 || group_size == 64) && (!act || N % 32 == 0) &&
-                       decode_tiled_grouped_rows(16, act ? 2 : 1, M, K, x_bits, group_size) != 0 &&
                        decode_tiled_grouped_pays(x_bits, w_bits, M, N, K, act, group_size)
                    ? 1
                    : 0;

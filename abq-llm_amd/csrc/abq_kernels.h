@@ -93,22 +93,17 @@ inline int decode_tiled_rows(int nw, int t, int M, int K, int q)
     return decode_tiled_lds(nw, t, mrows, K, q) <= 160 * 1024 ? mrows : 0;
 }
 
-// The same kernel with group scales (groups of 128 = one K tile): fp32 partial tiles, and after the activations the
-// tile's weight scales and zero points ([group][16 rows] each, T tiles) and the activation group sums
-// ([group][16 rows]), every array padded to whole wave loads of four bytes per lane.
-// (group: 128, or 64 = two scale groups per K tile)
-inline size_t decode_tiled_grouped_lds(int nw, int t, int mrows, int K, int q, int group = 128)
+// Decode kernel with group scales on K-tiled operands (abq_gemm_decode_tiled_grouped.hip): a wave owns blocks of four K
+// tiles, so the waves of a workgroup follow from K (and
+// the weights' width and group size): up to eight waves of one or two blocks, beyond that up to
+// sixteen, evened out (K = 4096: 8 waves of one block; 5120: 5 of two; 11008: 11 of two; 13824: 14 of two).  8-bit
+// weights and groups of 64 need the registers of an eight-wave workgroup.
+inline int decode_grouped_tiled_waves(int K, int w_bits, int group_size)
 {
-    const size_t groups = (size_t)K / group;
-    const size_t per_tile = (groups * 16 + 63) / 64 * 256; // bytes of one [group][16] float array
-    return decode_tiled_lds(nw, t, mrows, K, q) + (2 * t + 1) * per_tile + 1024;
-}
-inline int decode_tiled_grouped_rows(int nw, int t, int M, int K, int q, int group = 128)
-{
-    int mrows = M < 16 ? M : 16;
-    while (mrows > 1 && decode_tiled_grouped_lds(nw, t, mrows, K, q, group) > 150 * 1024)
-        mrows = (mrows + 1) / 2;
-    return decode_tiled_grouped_lds(nw, t, mrows, K, q, group) <= 160 * 1024 ? mrows : 0;
+    const int nblocks = (K / 128 + 3) / 4;
+    const int most = nblocks <= 16 || w_bits == 8 || group_size == 64 ? 8 : 16;
+    const int per_wave = (nblocks + most - 1) / most;
+    return (nblocks + per_wave - 1) / per_wave;
 }
 
 // Workgroup id -> output tile.  XCD x = id % 8 owns n blocks [x * npx, (x + 1) * npx); inside an XCD the
