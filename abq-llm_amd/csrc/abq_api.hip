@@ -1031,6 +1031,9 @@ static bool biased_w(const abq_gemm_state *st) { return (st->reserved[4] & 2) !=
 // (abq_relayout_planes_padded), which is how the decode kernel on prepared operands reads activations of 3, 5, 6 or
 // 7 bits (abq_gemm_set_padded_activations)
 static bool padded_x(const abq_gemm_state *st) { return (st->reserved[4] & 4) != 0; }
+// reserved[4] bit 3: a group-scale state whose tile is the library's choice by its rules (no tile asked for, none measured):
+// the kernel that streams the weights once (abq_gemm_rows_grouped.hip) runs in the tile's place where it is ahead
+constexpr int kRowsKernel = 8;
 static bool one_field(int bits) { return bits == 2 || bits == 4 || bits == 8; }
 // Width of the activation records the decode kernel on prepared operands reads for a pair.
 static int decode_tiled_x_bits(int x_bits) { return abq_padded_bits(x_bits); }
@@ -1135,6 +1138,27 @@ static abq_status switch_to_decode_tiled(abq_gemm_state *st, bool one_tile = fal
     return ABQ_OK;
 }
 
+// Whether the kernel that streams the weights once for up to 64 rows (abq_gemm_rows_grouped.hip) is ahead of the prefill
+// tiles.  It wins while its workgroups cover most of the compute units (rows_grouped_covers) and its work, counted in
+// 16 x 16 tiles of the result, stays below what the prefill tiles do in their fixed time (W4A8, zero points, us):
+//   4096 x 4096     43 rows (768 tiles)  7.9 against 13.4, 128 rows (2048) 10.1 against 13.2, 192 rows (3072) 14.4 against 13.4
+//   4096 x 11008    43 rows 15.0 against 26.4, 128 rows 17.9 against 26.7
+//   12288 x 4096    32 rows (1536) 10.7 against 13.4, 43 rows (2304) 12.9 against 13.7, 64 rows (3072) 14.7 against 13.8
+//   15360 x 5120    43 rows (2880) 18.0 against 19.8
+// Outputs too wide for one round of 64x64 tiles, up to 48 rows (64 rows have no instance of six tiles): 22016 x 4096, gate
+// fused, 43 rows (4128) 19.8 against 26.6, 64 rows (5504) 32.0 against 27.7; 27648 x 5120, 32 rows (3456) 27.7 against
+// 32.3, 43 rows (5184) 33.1 against 33.5.  8-bit weights hold half the tiles in registers: 5120 x 5120, 96 rows (1920) 14.8
+// against 14.8; 12288 x 4096, 17 rows (1536) 14.5 against 14.0.
+static bool rows_grouped_pays(int x_bits, int w_bits, int is_signed, int M, int N, int K, int group_size, int act)
+{
+    if (!is_signed || !rows_grouped_runs(M, N, K, x_bits, w_bits, group_size, act) || K < 1024 || !rows_grouped_covers(M, N))
+        return false;
+    const long tiles = (N + 15) / 16, work = tiles * ((M + 15) / 16);
+    if (w_bits == 8)
+        return work <= 2048 && tiles <= 512;
+    return work <= 2900 || (tiles > 1024 && M <= 48 && work <= 4300);
+}
+
 // Group scales on a decode-sized GEMM whose operands are (or are about to be declared) both prepared: whether the
 // decode kernel of that layout has a group-scale variant for the pair that fits this shape.
 // The same weighing for the group-scale variant (one tile per workgroup, two with the SiLU gate), against the
@@ -1146,6 +1170,10 @@ static abq_status switch_to_decode_tiled(abq_gemm_state *st, bool one_tile = fal
 static bool decode_tiled_grouped_pays(int x_bits, int w_bits, int M, int N, int K, int act, int group_size)
 {
     if (M <= 16)
+        return true;
+    // (4-bit weights: folded records would be twice as wide, and the kernel that streams the weights once runs on either
+    // width: W4A8 with zero points, 43 x 22016 x 4096 19.8 us on 4-bit records, 34.5 on the folded ones)
+    if (w_bits == 4 && rows_grouped_pays(x_bits, w_bits, 1, M, N, K, group_size, act))
         return true;
     if (M > 128)
         return false;
@@ -1188,6 +1216,7 @@ static abq_status pick_grouped_tiled(abq_gemm_state *state)
             return rc;
     }
     const abq_tile_config &c = state->cfg;
+    state->reserved[4] &= ~kRowsKernel;
     const KernelTable *tg = find_table(registry().tiled_grouped, c.x_bits, c.w_bits, c.is_signed);
     if (!tg)
         return ABQ_ERR_UNSUPPORTED;
@@ -1241,14 +1270,18 @@ static abq_status pick_grouped_tiled(abq_gemm_state *state)
                 if (usable(tg->entries[i]) && tg->entries[i].lds != 0 && block_m(tg->entries[i]) == 64 && block_n(tg->entries[i]) == 64 &&
                     tg->entries[i].wk == 2)
                     pick = i;
+        // (the tile picked here stays the state's: it runs where the kernel for few rows does not)
+        state->reserved[4] |= kRowsKernel;
         // a measured best tile for this shape and group size comes before the rules above
         TunedTile t;
         if (tuning_find(c.x_bits, c.w_bits, c.is_signed, state->M, state->N, state->K, state->group_size, 1 << ABQ_LAYOUT_TILED, &t) &&
             t.cfg.nstage == 4 && t.cfg.warp_k > 0)
             for (int i = 0; i < tg->count; ++i)
                 if (usable(tg->entries[i]) && block_m(tg->entries[i]) == t.cfg.block_m && block_n(tg->entries[i]) == t.cfg.block_n &&
-                    tg->entries[i].mi * tg->entries[i].tm == t.cfg.warp_m && tg->entries[i].wk == t.cfg.block_k / t.cfg.warp_k)
+                    tg->entries[i].mi * tg->entries[i].tm == t.cfg.warp_m && tg->entries[i].wk == t.cfg.block_k / t.cfg.warp_k) {
                     pick = i;
+                    state->reserved[4] &= ~kRowsKernel;
+                }
     } else {
         const int wk = c.warp_k > 0 ? c.block_k / c.warp_k : 1;
         for (int i = 0; i < tg->count; ++i)
@@ -1886,7 +1919,13 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
                     return ABQ_ERR_NOT_INITIALIZED;
             }
         }
-        e = t->entries[variant].launch(a, (hipStream_t)stream);
+        if (st->strategy == ABQ_STRATEGY_TILED && (st->reserved[4] & kRowsKernel) &&
+            rows_grouped_pays(c.x_bits, c.w_bits, c.is_signed, st->M, st->N, st->K, st->group_size, st->act))
+            e = c.w_bits == 2   ? launch_rows_grouped_8<2>(a, (hipStream_t)stream)
+                : c.w_bits == 4 ? launch_rows_grouped_8<4>(a, (hipStream_t)stream)
+                                : launch_rows_grouped_8<8>(a, (hipStream_t)stream);
+        else
+            e = t->entries[variant].launch(a, (hipStream_t)stream);
     } else {
         if (st->group_size && st->strategy != ABQ_STRATEGY_DECODE)
             return ABQ_ERR_NOT_INITIALIZED; // group scales live on the decode and tiled kernels only
