@@ -10,6 +10,8 @@
 // a quad assemble the bytes into one word per plane with DPP moves.  Input bytes are read
 // once, every load is 16 bytes wide and consecutive lanes touch consecutive memory.
 #include <climits>
+#include <type_traits>
+
 #include "abq_kernels.h"
 #include "abq_quant.h"
 
@@ -604,30 +606,33 @@ __device__ __forceinline__ void emit_tiled(const int (&v)[8], uint32_t *tiled, i
 
 // Eight codes of magnitude at most 16 (this lane's unit: elements 8 u .. 8 u + 7 of `row`, u = 4 w + quad_lane) ->
 // their share of the row's FP6 record; the four lanes of a quad assemble one word-set of 192 bits.
-__device__ __forceinline__ void emit_fp6(const int (&v)[8], uint32_t *records, int rows, int row, int w, int quad_lane, bool active)
+// Position p = 4 s + c of the word-set's string holds element 31 - (8c + s), i.e. element 7 - s of lane 3 - c: the four
+// codes of one s are neighbours, 24 bits.  The quad transposes its codes as bytes, so that lane i ends up with the four of
+// s = i and the four of s = 4 + i, squeezes each into 24 bits, and lanes 0 .. 2 put the strings together from their own and
+// their neighbour's.  (Codes OR-ed into six dwords across the quad one by one were two hundred instructions per unit, and
+// the packing kernels were bound by them.)
+__device__ __forceinline__ uint32_t fp6_codes(uint32_t x) // four two's complement bytes -> (sign << 5) | magnitude
 {
-    // position p = 4 s + c of the word-set's 192-bit string holds element 31 - (8c + s): this lane's
-    // element j goes to position 4 (7 - j) + 3 - quad_lane as the code (sign << 5) | magnitude
-    uint32_t o[6] = { 0u, 0u, 0u, 0u, 0u, 0u };
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const uint32_t code = v[j] < 0 ? (32u | (uint32_t)(-v[j])) : (uint32_t)v[j];
-        constexpr int kBase[8] = { 168, 144, 120, 96, 72, 48, 24, 0 }; // 24 (7 - j)
-        const int d0 = kBase[j] >> 5;                                   // first dword the code can touch
-        const uint64_t wide = (uint64_t)code << ((kBase[j] & 31) + 6 * (3 - quad_lane));
-        o[d0] |= (uint32_t)wide;
-        if (d0 + 1 < 6)
-            o[d0 + 1] |= (uint32_t)(wide >> 32);
-    }
-#pragma unroll
-    for (int d = 0; d < 6; ++d)
-        o[d] = quad_or(o[d]);
-    if (active && quad_lane == 0) {
-        const int ws = w & 3;
-        uint32_t *rec = records + ((size_t)(w >> 2) * rows + row) * 24 + 12 * (ws & 1) + 6 * (ws >> 1);
-        *reinterpret_cast<uint2 *>(rec) = make_uint2(o[0], o[1]);
-        *reinterpret_cast<uint2 *>(rec + 2) = make_uint2(o[2], o[3]);
-        *reinterpret_cast<uint2 *>(rec + 4) = make_uint2(o[4], o[5]);
+    const uint32_t m = (x >> 7) & 0x01010101u; // a byte's sign; m * 255 is the mask of its bits
+    return ((x ^ ((m << 8) - m)) + m) | (m << 5);
+}
+__device__ __forceinline__ uint32_t fp6_squeeze(uint32_t x) // four codes of six bits, a byte each -> 24 bits
+{
+    const uint32_t t = (x & 0x003F003Fu) | ((x >> 2) & 0x0FC00FC0u);
+    return (t & 0xFFFu) | ((t >> 4) & 0xFFF000u);
+}
+__device__ __forceinline__ void emit_fp6(const int (&v)[8], uint32_t *records, int rows, int row, int w, int quad_lane, bool active,
+                                         uint32_t sel_pair, uint32_t sel_half)
+{
+    const uint32_t lo = fp6_squeeze(quad_transpose_bytes(fp6_codes(pack_low_bytes(v[7], v[6], v[5], v[4])), sel_pair, sel_half));
+    const uint32_t hi = fp6_squeeze(quad_transpose_bytes(fp6_codes(pack_low_bytes(v[3], v[2], v[1], v[0])), sel_pair, sel_half));
+    const uint32_t lo_next = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, 0xF9, 0xF, 0xF, true); // quad_perm [1,2,3,3]
+    const uint32_t hi_next = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, 0xF9, 0xF, 0xF, true);
+    if (active && quad_lane < 3) {
+        const int ws = w & 3, down = 8 * quad_lane, up = 24 - down;
+        uint32_t *rec = records + ((size_t)(w >> 2) * rows + row) * 24 + 12 * (ws & 1) + 6 * (ws >> 1) + quad_lane;
+        rec[0] = (lo >> down) | (lo_next << up);
+        rec[3] = (hi >> down) | (hi_next << up);
     }
 }
 
@@ -637,51 +642,67 @@ __device__ __forceinline__ void emit_fp6(const int (&v)[8], uint32_t *records, i
 // FP6: the same values written as FP6 records (codes of at most 5 bits signed / 4 unsigned): the low `bits` bits of
 // the truncated product, read as the signed or unsigned code they are in the planes (values beyond the range alias
 // there as well: the reference packs the low bits and does not clamp).
-template <bool FP6>
+// A thread takes UNITS units, 256 apart, whose loads are all in flight before the first is used: two once the grid has several
+// waves for every SIMD (FP6 records, with the assembly above and 32-bit indexes: 2048 x 4096 8.3 -> 7.1 us, 2048 x 11008 17.4
+// -> 15.5), one below, where a second unit only lengthens the chain (128 x 4096 2.4, with two 2.7).
+template <bool FP6, typename Index, int UNITS>
 __global__ __launch_bounds__(256) void pack_f16_tiled_kernel(const uint4 *__restrict__ in, const float *__restrict__ scale,
-                                                             uint32_t *__restrict__ tiled, int rows, int units, int bits,
-                                                             int is_signed)
+                                                             uint32_t *__restrict__ tiled, int rows, uint32_t units, int bits,
+                                                             int is_signed, Index n_units)
 {
     const _Float16 hs = (_Float16)scale[0];
-    const size_t n_units = (size_t)rows * units; // units per row: a multiple of 16, so a quad is active as one
-    const size_t rounded = (n_units + 255) / 256 * 256;
+    // (the units of a row are a multiple of 16 and the stride of 256, so a quad is active as one)
     uint32_t sel_pair, sel_half;
     quad_transpose_selectors(threadIdx.x & 3, sel_pair, sel_half);
-    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < rounded; t += (size_t)gridDim.x * 256) {
-        const bool active = t < n_units;
-        int v[8] = { 0, 0, 0, 0, 0, 0, 0, 0 };
-        if (active) {
-            union {
-                uint4 u;
-                _Float16 h[8];
-            } raw;
-            raw.u = in[t];
+    for (Index base = (Index)blockIdx.x * (256 * UNITS); base < n_units; base += (Index)gridDim.x * (256 * UNITS)) {
+        union {
+            uint4 u;
+            _Float16 h[8];
+        } raw[UNITS];
+        bool active[UNITS];
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const _Float16 p = raw.h[c] * hs; // fp16 product, rounded to nearest even
-                v[c] = (int)p;                    // truncation
-            }
+        for (int i = 0; i < UNITS; ++i) {
+            const Index t = base + 256 * i + threadIdx.x;
+            active[i] = t < n_units;
+            raw[i].u = in[active[i] ? t : base];
         }
-        const int row = (int)(t / units), u = (int)(t % units);
-        if constexpr (FP6) {
+#pragma unroll
+        for (int i = 0; i < UNITS; ++i) {
+            const Index t = base + 256 * i + threadIdx.x;
+            const int row = (int)(t / units), u = (int)(t - (Index)row * units);
+            int v[8];
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
-                const int low = v[c] & ((1 << bits) - 1);
-                v[c] = (is_signed && (low >> (bits - 1))) ? low - (1 << bits) : low;
+                const _Float16 p = raw[i].h[c] * hs; // fp16 product, rounded to nearest even
+                v[c] = (int)p;                       // truncation
             }
-            emit_fp6(v, tiled, rows, active ? row : 0, u >> 2, u & 3, active);
-        } else {
-            emit_tiled(v, tiled, rows, active ? row : 0, u >> 2, u & 3, bits, active, sel_pair, sel_half);
+            if constexpr (FP6) {
+#pragma unroll
+                for (int c = 0; c < 8; ++c) {
+                    const int low = v[c] & ((1 << bits) - 1);
+                    v[c] = (is_signed && (low >> (bits - 1))) ? low - (1 << bits) : low;
+                }
+                emit_fp6(v, tiled, rows, active[i] ? row : 0, u >> 2, u & 3, active[i], sel_pair, sel_half);
+            } else {
+                emit_tiled(v, tiled, rows, active[i] ? row : 0, u >> 2, u & 3, bits, active[i], sel_pair, sel_half);
+            }
         }
     }
 }
 
+// the wave's maximum in every lane: quads, halves of a row of sixteen lanes and rows by row operations, then the four rows
+// through scalar registers.  (Six butterflies through the LDS crossbar are a hundred cycles each.)
 __device__ __forceinline__ float wave_max(float v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        v = fmaxf(v, __shfl_xor(v, o));
-    return v;
+    auto dpp = [&](auto ctrl) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xF, 0xF, false));
+    };
+    v = fmaxf(v, dpp(std::integral_constant<int, 0xB1>{}));  // quad_perm [1,0,3,2]
+    v = fmaxf(v, dpp(std::integral_constant<int, 0x4E>{}));  // quad_perm [2,3,0,1]
+    v = fmaxf(v, dpp(std::integral_constant<int, 0x141>{})); // row_half_mirror
+    v = fmaxf(v, dpp(std::integral_constant<int, 0x140>{})); // row_mirror
+    auto row = [&](int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); };
+    return fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
 }
 
 // Quantises the eight fp16 values of unit u (elements 8u .. 8u + 7) of `row` and writes their share of the
@@ -719,7 +740,7 @@ __device__ __forceinline__ void quant_emit_unit(const uint4 &rawq, bool active, 
     }
     const int quad_lane = u & 3, w = u >> 2; // w: word-set (32 elements) within the row
     if (LAYOUT == 2) {
-        emit_fp6(v, planes, M, row, w, quad_lane, active);
+        emit_fp6(v, planes, M, row, w, quad_lane, active, sel_pair, sel_half);
     } else if (LAYOUT == 1) {
         emit_tiled(v, planes, M, row, w, quad_lane, bits, active, sel_pair, sel_half);
     } else {
@@ -745,12 +766,12 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 // prefill, where one wave per row leaves a SIMD with one or two waves and the time is a wave's own chain of
 // instructions (914 at K = 4096, 2359 at K = 11008) behind the latency of its loads.
 template <int LAYOUT, int NU, int BITS, int WPR = 1>
-__global__ __launch_bounds__(256) void quant_pack_wave_rows_kernel(const uint4 *__restrict__ x, uint32_t *__restrict__ planes,
+__global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void quant_pack_wave_rows_kernel(const uint4 *__restrict__ x, uint32_t *__restrict__ planes,
                                                                    float *__restrict__ scale_out, float *__restrict__ zero_out,
                                                                    int *__restrict__ group_sums, int M, int K, int bits,
                                                                    int symmetric, int group_size)
 {
-    static_assert(WPR == 1 || WPR == 4, "one wave or the whole workgroup per row");
+    static_assert(WPR == 1 || WPR == 4 || WPR == 8 || WPR == 16, "one wave or the whole workgroup per row");
     const int lane = threadIdx.x & 63;
     const int wsub = WPR == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); // the wave's place in its row
     const int row = WPR == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
@@ -954,22 +975,33 @@ hipError_t launch_quant_pack_rows(const void *x, uint32_t *planes, float *scale,
     // 1024 16.4 -> 11.9, 16384 177 -> 142.
     const int split_rows = nu <= 2 ? 256 : nu <= 8 ? 1024 : nu <= 12 ? 2048 : nu <= 16 ? 4096 : nu <= 24 ? 8192 : INT_MAX;
     if (nu <= 32 && M <= split_rows) {
-        const dim3 grid(M), block(256);
+        const dim3 grid(M);
         const int nu4 = (nu + 3) / 4;
-#define ABQ_QP_SPLIT(L, NU)                                                                                                 \
+        // Up to one row per compute unit more waves shorten a wave's chain further, eight per row above K = 2048, sixteen above
+        // 8192 (four -> more, us: 16 x 4096 3.0 -> 2.9, 256 x 4096 3.4 -> 3.3, 16 x 11008 4.4 -> 4.0, into FP6 records 5.9 -> 4.4;
+        // past one round it turns: 777 x 11008 10.2 -> 12.3).
+        const bool wide = M <= 256;
+#define ABQ_QP_SPLIT(L, NU)  ABQ_QP_SPLIT_W(L, NU, 4)
+#define ABQ_QP_SPLIT_W(L, NU, W)                                                                                                 \
     do {                                                                                                                    \
         if (L == 1 && bits == 8)                                                                                            \
-            hipLaunchKernelGGL((quant_pack_wave_rows_kernel<L, NU, (L == 1 ? 8 : 0), 4>), grid, block, 0, stream,              \
+            hipLaunchKernelGGL((quant_pack_wave_rows_kernel<L, NU, (L == 1 ? 8 : 0), W>), grid, dim3(64 * W), 0, stream,              \
                                reinterpret_cast<const uint4 *>(x), planes, scale, zero, group_sums, M, K, bits, symmetric,  \
                                group_size);                                                                                 \
         else                                                                                                                \
-            hipLaunchKernelGGL((quant_pack_wave_rows_kernel<L, NU, 0, 4>), grid, block, 0, stream,                            \
+            hipLaunchKernelGGL((quant_pack_wave_rows_kernel<L, NU, 0, W>), grid, dim3(64 * W), 0, stream,                            \
                                reinterpret_cast<const uint4 *>(x), planes, scale, zero, group_sums, M, K, bits, symmetric,  \
                                group_size);                                                                                 \
     } while (0)
 #define ABQ_QP_SPLIT_NU(L)       \
     do {                         \
-        if (nu4 <= 1)            \
+        if (wide && nu > 16)     \
+            ABQ_QP_SPLIT_W(L, 2, 16); \
+        else if (wide && nu > 8) \
+            ABQ_QP_SPLIT_W(L, 2, 8); \
+        else if (wide && nu > 4) \
+            ABQ_QP_SPLIT_W(L, 1, 8); \
+        else if (nu4 <= 1)       \
             ABQ_QP_SPLIT(L, 1);  \
         else if (nu4 <= 2)       \
             ABQ_QP_SPLIT(L, 2);  \
@@ -988,6 +1020,7 @@ hipError_t launch_quant_pack_rows(const void *x, uint32_t *planes, float *scale,
             ABQ_QP_SPLIT_NU(0);
 #undef ABQ_QP_SPLIT_NU
 #undef ABQ_QP_SPLIT
+#undef ABQ_QP_SPLIT_W
         return hipGetLastError();
     }
     // More rows than that: one wave per row, the row in registers (up to 12288 elements).
@@ -1103,22 +1136,37 @@ hipError_t launch_pack_i32(const int32_t *in, uint32_t *planes, int rows, int k,
     return hipGetLastError();
 }
 
+template <bool FP6>
+static hipError_t launch_pack_f16_records(const void *in, const float *scale, uint32_t *records, int rows, int k, int bits, int is_signed,
+                                          hipStream_t stream)
+{
+    const size_t n_units = (size_t)rows * k / 8;
+    auto go = [&](auto n, auto per_thread) {
+        using Index = decltype(n);
+        constexpr int UNITS = decltype(per_thread)::value;
+        hipLaunchKernelGGL((pack_f16_tiled_kernel<FP6, Index, UNITS>), dim3(grid_for((n_units + UNITS - 1) / UNITS)), dim3(256), 0, stream,
+                           reinterpret_cast<const uint4 *>(in), scale, records, rows, (uint32_t)(k / 8), bits, is_signed, n);
+    };
+    // (32-bit indexes while the last stride stays within them)
+    if (n_units >= (1ull << 31))
+        go((uint64_t)n_units, std::integral_constant<int, 2>{});
+    else if (n_units >= 256 * 1024)
+        go((uint32_t)n_units, std::integral_constant<int, 2>{});
+    else
+        go((uint32_t)n_units, std::integral_constant<int, 1>{});
+    return hipGetLastError();
+}
+
 hipError_t launch_pack_f16_tiled(const void *in, const float *scale, uint32_t *tiled, int rows, int k, int bits,
                                  hipStream_t stream)
 {
-    const size_t n_units = (size_t)rows * k / 8;
-    hipLaunchKernelGGL(pack_f16_tiled_kernel<false>, dim3(grid_for(n_units)), dim3(256), 0, stream,
-                       reinterpret_cast<const uint4 *>(in), scale, tiled, rows, k / 8, bits, 0);
-    return hipGetLastError();
+    return launch_pack_f16_records<false>(in, scale, tiled, rows, k, bits, 0, stream);
 }
 
 hipError_t launch_pack_f16_fp6(const void *in, const float *scale, uint32_t *records, int rows, int k, int bits, int is_signed,
                                hipStream_t stream)
 {
-    const size_t n_units = (size_t)rows * k / 8;
-    hipLaunchKernelGGL(pack_f16_tiled_kernel<true>, dim3(grid_for(n_units)), dim3(256), 0, stream,
-                       reinterpret_cast<const uint4 *>(in), scale, records, rows, k / 8, bits, is_signed);
-    return hipGetLastError();
+    return launch_pack_f16_records<true>(in, scale, records, rows, k, bits, is_signed, stream);
 }
 
 hipError_t launch_pack_f16(const void *in, const float *scale, uint32_t *planes, int rows, int k,
