@@ -16,7 +16,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("p", [2, 4, 8])
 @pytest.mark.parametrize("M,N,K,act", [(17, 40, 1024, False), (32, 4128, 1152, True), (33, 8216, 1152, False), (43, 16416, 1280, True),
                                        (48, 12312, 1024, False), (49, 4104, 4224, False), (64, 12320, 1024, True), (65, 72, 8320, False),
-                                       (96, 4112, 1024, False), (110, 96, 1664, True), (128, 24, 1152, False)])
+                                       (96, 4112, 1024, False), (110, 96, 1664, True), (128, 24, 1152, False),
+                                       # (the fewest workgroups that take the kernel, in two blocks of rows; K of one to five tiles: one
+                                       # and two waves, blocks of one and three tiles)
+                                       (65, 2056, 8320, False), (128, 1544, 1152, False), (32, 4096, 128, False), (20, 4128, 384, True),
+                                       (64, 4100, 640, False)])
 def test_rows_blocks_and_tiles(abq, oracle, p, M, N, K, act):
     rng = np.random.default_rng(M + N + K + p)
     xt, wt, kw, want = operands(abq, oracle, rng, M, N, K, 8, p, 128, act)
