@@ -43,13 +43,19 @@ constexpr int rows_ahead(int p, int t, int mb) { return 4 * t * (p + mb) <= 150 
 constexpr int rows_ring(int p, int t, int mb) { return mb <= 2 && rows_ahead(p, t, mb) == 4 ? 3 : 2; }
 // instances that are built: what registers and LDS hold
 constexpr bool rows_built(int p, int t, int mb) { return t * p <= 24 && t * mb <= 18; }
-// LDS: the activation rings (the partial tiles meet there at the end) | scales, zero points and group sums per wave | the
-// rows' scales and zero points, the tiles' zero-point terms
+// LDS: the activation rings, then scales, zero points and group sums per wave (the waves' partial tiles take the place of all
+// of these at the end) | the rows' scales and zero points, the tiles' zero-point terms
 constexpr int rows_scale_loads(int t, int mb, bool zp) { return zp ? 2 * t + mb : t; }
-constexpr size_t rows_lds(int nw, int p, int t, int mb, bool zp)
+constexpr size_t rows_lds_of_loop(int nw, int p, int t, int mb, bool zp)
 {
-    return (size_t)nw * rows_ring(p, t, mb) * mb * 2048 + (size_t)nw * rows_scale_loads(t, mb, zp) * 256 + 512 + 512;
+    return (size_t)nw * (rows_ring(p, t, mb) * mb * 2048 + rows_scale_loads(t, mb, zp) * 256);
 }
+constexpr size_t rows_lds_of_sum(int nw, int t, int mb) { return (size_t)nw * t * mb * 1024; }
+constexpr size_t rows_lds_for_rows(int nw, int p, int t, int mb, bool zp) // where the rows' scales lie
+{
+    return rows_lds_of_loop(nw, p, t, mb, zp) > rows_lds_of_sum(nw, t, mb) ? rows_lds_of_loop(nw, p, t, mb, zp) : rows_lds_of_sum(nw, t, mb);
+}
+constexpr size_t rows_lds(int nw, int p, int t, int mb, bool zp) { return rows_lds_for_rows(nw, p, t, mb, zp) + 512 + 512; }
 
 // 16 bytes per lane from base + off straight into LDS: lane l lands at lds_addr + 16 l
 __device__ __forceinline__ void rows_dma16(const void *base, uint32_t off, unsigned lds_addr)
@@ -66,9 +72,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmA
     constexpr int LW = T * DtgShare<P>::kLoads; // ... weights
     constexpr int LS = rows_scale_loads(T, MB, ZP); // ... of a block: scales, zero points, group sums (into LDS)
     constexpr int XB = MB * 2048;              // bytes of a step's activations
-    constexpr int TC = T <= 2 * R ? T : 2;     // tiles whose partial sums meet in LDS at a time
     static_assert(4 % D == 0 && R <= D && R < 4, "the rings' places follow from the step of the block");
-    static_assert(TC % 2 == 0 || TC == T, "a gate tile and its up tile stay together");
     extern __shared__ __align__(16) unsigned char smem[];
 
     const int tid = threadIdx.x;
@@ -95,7 +99,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmA
     float *sws = reinterpret_cast<float *>(smem + NW * (R * XB) + wid * (LS * 256)); // [T][16 rows][4 groups]
     float *zws = sws + T * 64;                                                       // [T][16 rows][4 groups]
     int *sxs = reinterpret_cast<int *>(zws + T * 64);                                // [MB][4 groups][16 rows]
-    float *par = reinterpret_cast<float *>(smem + NW * (R * XB) + NW * (LS * 256));  // [2][64]: scales, zero points of the rows
+    float *par = reinterpret_cast<float *>(smem + rows_lds_for_rows(NW, P, T, MB, ZP)); // [2][64]: scales, zero points of the rows
     float *terms = par + 128;                                                        // [128]
 
     // ---- byte offsets of the lane's share ---------------------------------------------------------------------------
@@ -276,47 +280,45 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmA
     // after the other.
     v4f *red = reinterpret_cast<v4f *>(smem);
     _Float16 *out = reinterpret_cast<_Float16 *>(a.D);
+    // (All tiles at once: two at a time, a pair of barriers for each, 22016 x 4096 took 21.2 us in a trace instead of 19.9.)
+    __syncthreads(); // every wave is through with its ring and its scales
 #pragma unroll
-    for (int t0 = 0; t0 < T; t0 += TC) {
-        __syncthreads(); // every wave is through with the rings (t0 > 0: with the tiles before)
+    for (int t = 0; t < T; ++t)
 #pragma unroll
-        for (int t = t0; t < t0 + TC; ++t)
-#pragma unroll
-            for (int b = 0; b < MB; ++b)
-                red[((wid * TC + t - t0) * MB + b) * 64 + r * 4 + g] = facc[t][b];
-        __syncthreads();
-        for (int o = tid; o < TC * MB * 64; o += (int)blockDim.x) {
-            const int t = o / (MB * 64), rem = o % (MB * 64), b = rem >> 6, gg = (rem >> 4) & 3, c = rem & 15;
-            const int n = (tile0 + t0 + t) * 16 + c, mr = b * 16 + gg * 4;
-            if (n >= N || mr >= Mb || (a.act && (t & 1)))
-                continue;
-            auto total = [&](int tt) {
-                v4f v = v4f{ 0.f, 0.f, 0.f, 0.f };
+        for (int b = 0; b < MB; ++b)
+            red[((wid * T + t) * MB + b) * 64 + r * 4 + g] = facc[t][b];
+    __syncthreads();
+    for (int o = tid; o < T * MB * 64; o += (int)blockDim.x) {
+        const int t = o / (MB * 64), rem = o % (MB * 64), b = rem >> 6, gg = (rem >> 4) & 3, c = rem & 15;
+        const int n = (tile0 + t) * 16 + c, mr = b * 16 + gg * 4;
+        if (n >= N || mr >= Mb || (a.act && (t & 1)))
+            continue;
+        auto total = [&](int tt) {
+            v4f v = v4f{ 0.f, 0.f, 0.f, 0.f };
 #pragma unroll 8
-                for (int w = 0; w < NW; ++w)
-                    v += red[((w * TC + tt) * MB + b) * 64 + c * 4 + gg];
+            for (int w = 0; w < NW; ++w)
+                v += red[((w * T + tt) * MB + b) * 64 + c * 4 + gg];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float f = v[e] * (1.0f / kShift);
-                    if (row_zero)
-                        f = __builtin_fmaf(-par[64 + mr + e], terms[(t0 + tt) * 16 + c], f);
-                    v[e] = f * par[mr + e];
-                }
-                return v;
-            };
-            const v4f v = total(t);
-            if (T > 1 && a.act) { // this tile holds gate rows, the next one their up rows
-                const v4f up = total(T > 1 ? t + 1 : t);
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (mr + e < Mb)
-                        out[(size_t)(m0 + mr + e) * (N / 2) + (n >> 5) * 16 + c] = (_Float16)(silu(v[e]) * up[e]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (mr + e < Mb)
-                        out[(size_t)(m0 + mr + e) * N + n] = (_Float16)v[e];
+            for (int e = 0; e < 4; ++e) {
+                float f = v[e] * (1.0f / kShift);
+                if (row_zero)
+                    f = __builtin_fmaf(-par[64 + mr + e], terms[tt * 16 + c], f);
+                v[e] = f * par[mr + e];
             }
+            return v;
+        };
+        const v4f v = total(t);
+        if (T > 1 && a.act) { // this tile holds gate rows, the next one their up rows
+            const v4f up = total(T > 1 ? t + 1 : t);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (mr + e < Mb)
+                    out[(size_t)(m0 + mr + e) * (N / 2) + (n >> 5) * 16 + c] = (_Float16)(silu(v[e]) * up[e]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (mr + e < Mb)
+                    out[(size_t)(m0 + mr + e) * N + n] = (_Float16)v[e];
         }
     }
 }
