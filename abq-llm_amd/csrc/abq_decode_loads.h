@@ -4,6 +4,7 @@
 // counted wait.
 #pragma once
 #include "abq_kernels.h"
+#include "abq_lds_dma.h"
 #include "abq_bits.h"
 
 namespace abq {
@@ -14,14 +15,6 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 constexpr bool decode_tiled_width(int b) { return b == 2 || b == 4 || b == 8; }
 // single-field widths, activations at least as wide as the weights
 constexpr bool decode_tiled_built(int q, int p) { return decode_tiled_width(q) && decode_tiled_width(p) && q >= p; }
-
-__device__ __forceinline__ void dt_load_to_lds(const void *src, unsigned lds_addr)
-{
-    // lane l of the wave lands at lds_addr + 16 * l.  (M0 cannot be named as clobbered: the compiler reserves it and
-    // sets it up itself right before each of its own uses, it keeps no value there across other instructions.)
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(src)
-                 : "memory");
-}
 
 __device__ __forceinline__ v4u dt_load16(const char *base, uint32_t off)
 {
@@ -96,13 +89,6 @@ template <int BITS, bool SIGNED> __device__ __forceinline__ void dt_unpack(const
 }
 
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ void dt_dma_dword(const void *base, uint32_t off, unsigned lds_addr)
-{
-    // the dword at base + off (off per lane) of lane l lands at lds_addr + 4 * l
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(off), "s"(base)
-                 : "memory");
-}
 
 // a lane's share of one weight record (32 elements): P dwords
 template <int P> struct DtgShare {

@@ -19,6 +19,7 @@
 // with a multiply-add per unit.  The LPR partial sums meet through DPP row operations (and one or two
 // cross-row shuffles): no LDS traffic for the reduction.
 #include "abq_kernels.h"
+#include "abq_lds_dma.h"
 
 #ifndef ABQ_Q
 #error "compile with -DABQ_Q=<x_bits> -DABQ_P=<w_bits>"
@@ -29,13 +30,6 @@ namespace abq {
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kBcntWaves = 8;
-
-__device__ __forceinline__ void bc_load_to_lds(const void *src, unsigned lds_addr)
-{
-    // lane l of the wave lands at lds_addr + 16 * l (M0 cannot be named as clobbered: the compiler reserves it)
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(src)
-                 : "memory");
-}
 
 __device__ __forceinline__ v4u bc_load16(const char *base, uint32_t off)
 {
@@ -113,13 +107,13 @@ __global__ __launch_bounds__(64 * kBcntWaves) void gemm_bcnt(const GemmArgs a)
     if (Mb == M) { // all planes are one contiguous block
         for (int pb = wid * 64; pb < xchunks; pb += NT) {
             const int p = min(pb + lane, xchunks - 1);
-            bc_load_to_lds(Xg + (uint32_t)p * 16u, xs_addr + (unsigned)pb * 16u);
+            lds_dma16(Xg + (uint32_t)p * 16u, xs_addr + (unsigned)pb * 16u);
         }
     } else {
         for (int pb = wid * 64; pb < xchunks; pb += NT) {
             const int p = min(pb + lane, xchunks - 1);
             const int i = p / per_plane, c = p - i * per_plane;
-            bc_load_to_lds(Xg + ((size_t)(i * M + m0) * KW) * 4 + (size_t)c * 16, xs_addr + (unsigned)pb * 16u);
+            lds_dma16(Xg + ((size_t)(i * M + m0) * KW) * 4 + (size_t)c * 16, xs_addr + (unsigned)pb * 16u);
         }
     }
 

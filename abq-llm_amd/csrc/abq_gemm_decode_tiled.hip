@@ -125,13 +125,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_tiled(const GemmArgs a, i
             if (pb < xchunks) {
                 const int p = pb + lane;
                 const int src = min(p ^ ((p >> QLOG) & (Q - 1)), xchunks - 1);
-                dt_load_to_lds(Xt + (uint32_t)src * 16u, xs_addr + (unsigned)pb * 16u);
+                lds_dma16(Xt + (uint32_t)src * 16u, xs_addr + (unsigned)pb * 16u);
             }
         }
         for (int pb = wid * 64 + XC * NT; pb < xchunks; pb += NT) {
             const int p = pb + lane;
             const int src = min(p ^ ((p >> QLOG) & (Q - 1)), xchunks - 1);
-            dt_load_to_lds(Xt + (uint32_t)src * 16u, xs_addr + (unsigned)pb * 16u);
+            lds_dma16(Xt + (uint32_t)src * 16u, xs_addr + (unsigned)pb * 16u);
         }
     } else { // several blocks of rows: a K tile's rows are Mb * Q chunks out of M * Q
         const int per = Mb * Q;
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_tiled(const GemmArgs a, i
             const int p = min(pb + lane, xchunks - 1);
             const int q = p ^ ((p >> QLOG) & (Q - 1));
             const int kt = q / per, rem = q - kt * per;
-            dt_load_to_lds(Xt + ((size_t)(kt * M + m0) * Q + rem) * 16u, xs_addr + (unsigned)pb * 16u);
+            lds_dma16(Xt + ((size_t)(kt * M + m0) * Q + rem) * 16u, xs_addr + (unsigned)pb * 16u);
         }
     }
 
@@ -370,13 +370,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_fields(const GemmArgs a, 
             if (pb < xchunks) {
                 const int p = pb + lane;
                 const int src = min(p ^ ((p >> QLOG) & (QP - 1)), xchunks - 1);
-                dt_load_to_lds(Xt + (uint32_t)src * 16u, xs_addr + (unsigned)pb * 16u);
+                lds_dma16(Xt + (uint32_t)src * 16u, xs_addr + (unsigned)pb * 16u);
             }
         }
         for (int pb = wid * 64 + XC * NT; pb < xchunks; pb += NT) {
             const int p = pb + lane;
             const int src = min(p ^ ((p >> QLOG) & (QP - 1)), xchunks - 1);
-            dt_load_to_lds(Xt + (uint32_t)src * 16u, xs_addr + (unsigned)pb * 16u);
+            lds_dma16(Xt + (uint32_t)src * 16u, xs_addr + (unsigned)pb * 16u);
         }
     } else {
         const int per = Mb * QP;
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_fields(const GemmArgs a, 
             const int p = min(pb + lane, xchunks - 1);
             const int q = p ^ ((p >> QLOG) & (QP - 1));
             const int kt = q / per, rem = q - kt * per;
-            dt_load_to_lds(Xt + ((size_t)(kt * M + m0) * QP + rem) * 16u, xs_addr + (unsigned)pb * 16u);
+            lds_dma16(Xt + ((size_t)(kt * M + m0) * QP + rem) * 16u, xs_addr + (unsigned)pb * 16u);
         }
     }
 

@@ -142,14 +142,14 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
     // what the final sum needs per row and column goes to LDS now (the oldest loads of their waves): fetched behind the K
     // loop it would put one more memory latency at the end
     if (XM == 0 && wid == 0) {
-        dt_dma_dword(a.x_scale, (uint32_t)(m0 + min(r, Mb - 1)) * 4u, (unsigned)(size_t)par); // (lanes 0 .. 15 are read)
+        lds_dma4(a.x_scale, (uint32_t)(m0 + min(r, Mb - 1)) * 4u, (unsigned)(size_t)par); // (lanes 0 .. 15 are read)
         if (row_zero)
-            dt_dma_dword(a.x_zero, (uint32_t)(m0 + min(r, Mb - 1)) * 4u, (unsigned)(size_t)(par + 64));
+            lds_dma4(a.x_zero, (uint32_t)(m0 + min(r, Mb - 1)) * 4u, (unsigned)(size_t)(par + 64));
     }
     if (row_zero && wid == NW - 1) {
 #pragma unroll
         for (int i = 0; i < (T + 3) / 4; ++i)
-            dt_dma_dword(a.w_zero_term, (uint32_t)min(tile0 * 16 + i * 64 + lane, N - 1) * 4u, (unsigned)(size_t)(terms + i * 64));
+            lds_dma4(a.w_zero_term, (uint32_t)min(tile0 * 16 + i * 64 + lane, N - 1) * 4u, (unsigned)(size_t)(terms + i * 64));
     }
 
     const int upr = a.K >> 3; // XM: units of eight halves per row
@@ -193,12 +193,12 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
 #pragma unroll
                 for (int t = 0; t < T; ++t) {
                     const uint32_t off = (soff[t] + grp) * 4u;
-                    dt_dma_dword(a.w_scale, off, (unsigned)(size_t)(sws + (b * T + t) * SC + i * 64));
+                    lds_dma4(a.w_scale, off, (unsigned)(size_t)(sws + (b * T + t) * SC + i * 64));
                     if (zp)
-                        dt_dma_dword(a.w_zero, off, (unsigned)(size_t)(zws + (b * T + t) * SC + i * 64));
+                        lds_dma4(a.w_zero, off, (unsigned)(size_t)(zws + (b * T + t) * SC + i * 64));
                 }
                 if (XM == 0 && zp)
-                    dt_dma_dword(a.x_group_sums, (sumoff + (uint32_t)min(first + g, NG - 1)) * 4u, (unsigned)(size_t)(sxs + b * SC + i * 64));
+                    lds_dma4(a.x_group_sums, (sumoff + (uint32_t)min(first + g, NG - 1)) * 4u, (unsigned)(size_t)(sxs + b * SC + i * 64));
             }
         // ---- a step's weights and the next one's activations (steps past the end of K repeat the last one) ---------------
         auto k_tile = [&](int i) { return min(4 * block_of(i >> 2) + (i & 3), KT - 1); };

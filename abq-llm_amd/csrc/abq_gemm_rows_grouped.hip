@@ -57,13 +57,6 @@ constexpr size_t rows_lds_for_rows(int nw, int p, int t, int mb, bool zp) // whe
 }
 constexpr size_t rows_lds(int nw, int p, int t, int mb, bool zp) { return rows_lds_for_rows(nw, p, t, mb, zp) + 512 + 512; }
 
-// 16 bytes per lane from base + off straight into LDS: lane l lands at lds_addr + 16 l
-__device__ __forceinline__ void rows_dma16(const void *base, uint32_t off, unsigned lds_addr)
-{
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(off), "s"(base)
-                 : "memory");
-}
-
 template <int P, int T, int MB, bool ZP>
 __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmArgs a, int m_blocks)
 {
@@ -132,14 +125,14 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmA
     // What the final sum needs per row and column: the oldest loads of their waves.
     if (wid == 0) {
         const uint32_t row = (uint32_t)(m0 + min(lane, Mb - 1)) * 4u;
-        dt_dma_dword(a.x_scale, row, (unsigned)(size_t)par);
+        lds_dma4(a.x_scale, row, (unsigned)(size_t)par);
         if (row_zero)
-            dt_dma_dword(a.x_zero, row, (unsigned)(size_t)(par + 64));
+            lds_dma4(a.x_zero, row, (unsigned)(size_t)(par + 64));
     }
     if (row_zero && wid == NW - 1) {
 #pragma unroll
         for (int i = 0; i < (T + 3) / 4; ++i)
-            dt_dma_dword(a.w_zero_term, (uint32_t)min(tile0 * 16 + i * 64 + lane, N - 1) * 4u, (unsigned)(size_t)(terms + i * 64));
+            lds_dma4(a.w_zero_term, (uint32_t)min(tile0 * 16 + i * 64 + lane, N - 1) * 4u, (unsigned)(size_t)(terms + i * 64));
     }
 
     // Step s of the wave: K tile s % 4 of its block s / 4 (steps past the end of K repeat the last tile and count nothing).
@@ -156,7 +149,7 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmA
         const unsigned to = (unsigned)(size_t)ring + (unsigned)buf * XB;
 #pragma unroll
         for (int c = 0; c < LX; ++c)
-            rows_dma16(xp, xoff[c], to + c * 1024u);
+            lds_dma16(xp, xoff[c], to + c * 1024u);
     };
     // a block's scales: sixteen rows times four groups per instruction, neighbouring lanes on neighbouring groups
     auto request_scales = [&](int blk) {
@@ -165,14 +158,14 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmA
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             const uint32_t off = (soff[t] + grp) * 4u;
-            dt_dma_dword(a.w_scale, off, (unsigned)(size_t)(sws + t * 64));
+            lds_dma4(a.w_scale, off, (unsigned)(size_t)(sws + t * 64));
             if constexpr (ZP)
-                dt_dma_dword(a.w_zero, off, (unsigned)(size_t)(zws + t * 64));
+                lds_dma4(a.w_zero, off, (unsigned)(size_t)(zws + t * 64));
         }
         if constexpr (ZP) {
 #pragma unroll
             for (int b = 0; b < MB; ++b)
-                dt_dma_dword(a.x_group_sums, (sumoff[b] + (uint32_t)min(first + g, KT - 1)) * 4u, (unsigned)(size_t)(sxs + b * 64));
+                lds_dma4(a.x_group_sums, (sumoff[b] + (uint32_t)min(first + g, KT - 1)) * 4u, (unsigned)(size_t)(sxs + b * 64));
         }
     };
 

@@ -109,25 +109,6 @@ template <int N> __device__ __forceinline__ void staged_wait_loads()
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// `base` is the same in every lane (a scalar register pair), `offset` the lane's byte offset from it.
-__device__ __forceinline__ void staged_load_to_lds(const void *base, uint32_t offset, unsigned lds_addr)
-{
-    // the LDS address is the same in every lane; readfirstlane tells the compiler so
-    // (M0 cannot be named as clobbered: the compiler reserves it, rejects it in a clobber list, and sets it up itself
-    // right before each of its own uses; it keeps no value there across other instructions.)
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(offset),
-                 "s"(base)
-                 : "memory");
-}
-
-// The same with four bytes per lane (lane l lands at M0 + 4 * l): the group scales.
-__device__ __forceinline__ void staged_load_dword_to_lds(const void *base, uint32_t offset, unsigned lds_addr)
-{
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(offset),
-                 "s"(base)
-                 : "memory");
-}
-
 // LDS of a launch that writes fp16: the stages, or the waves' output tiles if those are larger and still fit beside
 // the other workgroup of the compute unit (two for the four-wave tiles with at most four MFMA tiles a wave).
 template <int TM, int TN, int WM, int WN, int STAGE_BYTES> struct StagedOutputLds {
@@ -297,7 +278,7 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     int kq = 0;
     auto request = [&](int stage, int i) {
         if (GROUPED && i == NPR) {
-            staged_load_dword_to_lds(sq, goff[i], lds0 + wk * BUF_BYTES + stage + SC_OFF + sc_block * 256);
+            lds_dma4(sq, goff[i], lds0 + wk * BUF_BYTES + stage + SC_OFF + sc_block * 256);
             return;
         }
         int q = wid + NW * i;
@@ -305,7 +286,7 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
             q -= NW;
         // (which operand request i is for does not depend on the wave when the waves divide both operands' loads)
         const bool activations = (NIA % NW == 0 && NI % NW == 0) ? NW * i < NIA : q < NIA;
-        staged_load_to_lds(activations ? (const void *)xq : (const void *)wq, goff[i], lds_wave + stage + (q - wid) * 1024);
+        lds_dma16(activations ? (const void *)xq : (const void *)wq, goff[i], lds_wave + stage + (q - wid) * 1024);
     };
     auto next_tile = [&]() {
         if ((kq + 1) * WK + wk < ktot) {

@@ -8,6 +8,7 @@
 // algorithm/quantize/quantizer.py:111-179 of the reference.
 #pragma once
 #include "abq_kernels.h"
+#include "abq_lds_dma.h"
 
 namespace abq {
 
@@ -161,15 +162,6 @@ __device__ __forceinline__ void zero_point_product(const int (&sx)[TM][8], const
             }
 }
 
-// A wave's 64 x 16 bytes from global memory straight into LDS at lds_addr + 16 * lane (`base` the same in every lane,
-// `offset` the lane's byte offset from it).
-__device__ __forceinline__ void epilogue_load_to_lds(const void *base, uint32_t offset, unsigned lds_addr)
-{
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(offset),
-                 "s"(base)
-                 : "memory");
-}
-
 // Half h of a chunk that the workgroup has staged in LDS (see group_scale_epilogue): the lane's eight groups of its TM
 // activation rows and TN weight rows.  A staged row is 128 bytes at row_at(row), its 16-byte pieces permuted by the
 // row number.
@@ -306,7 +298,7 @@ __device__ __forceinline__ void group_scale_epilogue(const GemmArgs &a, v16f (&f
                     for (int u = wave; u < UNITS; u += WM * WN) { // wave-uniform
                         const void *base;
                         const uint32_t off = zero_point_unit_offset<RA, RB>(a, u, lane, m0, n0, M, N, groups, first, &base);
-                        epilogue_load_to_lds(base, off, lds0 + u * 1024);
+                        lds_dma16(base, off, lds0 + u * 1024);
                     }
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                     __syncthreads();
