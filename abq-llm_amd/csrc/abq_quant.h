@@ -1,9 +1,11 @@
 // Per-token dynamic quantisation of fp16 activations: what a row's codes follow from once its extrema are known.
 // Shared by the quantise-and-pack kernels (abq_pack.hip) and the decode kernel that quantises its activations
-// itself (abq_gemm_decode_tiled.hip), so that both produce the same codes bit for bit.
+// itself (abq_gemm_decode_tiled_grouped.hip), so that both produce the same codes bit for bit.
 // Semantics: algorithm/quantize/quantizer.py:111-179 of the reference (per_token_dynamic_calibration, fake_quant).
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include "abq_recip.h"
 
 namespace abq {
 
@@ -35,17 +37,12 @@ __device__ __forceinline__ QuantRow quant_row_params(float mx, float mn, int bit
     QuantRow q;
     q.scale = scale;
     // x / scale in three operations instead of the dozen of a full division, with the same bits: recip is the
-    // correctly rounded reciprocal (the fp64 quotient is never close enough to an fp32 midpoint for the second
-    // rounding to cross it), t = x recip is within an ulp of the quotient, the residual x - t scale is exact in
+    // correctly rounded reciprocal (abq_recip.h), t = x recip is within an ulp of the quotient, the residual x - t scale is exact in
     // an fma, and t + residual recip then rounds to the quotient itself (checked against the division on a CPU
     // for every finite fp16 value and 600 000 scales of the forms above; a zero may come out with the other
     // sign, which the rounding to an integer code forgets).  div_fixup restores what a division makes of an
     // infinite x.
-    // (The reciprocal: the hardware's estimate, 1 ulp, and a Newton step whose residual is exact in an fma.  Equal to the
-    // rounded fp64 quotient for all 2^23 mantissas at every exponent from -17 to 13, checked on the GPU.  The fp64
-    // division it replaces was a chain of some forty instructions in front of every row's codes.)
-    const float r0 = __builtin_amdgcn_rcpf(scale);
-    q.recip = __builtin_fmaf(__builtin_fmaf(-scale, r0, 1.0f), r0, r0);
+    q.recip = rounded_reciprocal(scale, __builtin_amdgcn_rcpf(scale));
     // rint(q) + zp, clamped to [lo, hi], minus the offset of the stored code: the offset is taken off before the
     // clamp instead (all three are small integers, so the sums are the same numbers)
     const float code_offset = symmetric ? 0.f : (float)half_range;
