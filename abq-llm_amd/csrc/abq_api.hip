@@ -633,9 +633,10 @@ static int native_config(int x_bits, int w_bits, int is_signed, int index, abq_t
         const KernelEntry &e = tm->entries[index - (n - tm->count)];
         entry_to_config(e, e.mi == 16 ? ABQ_STRATEGY_MFMA16 : ABQ_STRATEGY_MFMA32, x_bits, w_bits, is_signed, 0, cfg);
     }
-    // (entries that want row sums handed in stand behind the kernel of the same tuple, at the end: no tuples of their own)
+    // (entries that want row sums handed in stand behind the kernel of the same tuple, at the end: no tuples of their own;
+    // neither do unlisted ones count)
     int tt_count = tt->count;
-    while (tt_count > 0 && (tt->entries[tt_count - 1].flags & kNeedsRowSums))
+    while (tt_count > 0 && (tt->entries[tt_count - 1].flags & (kNeedsRowSums | kUnlisted)))
         --tt_count;
     if (in(tt_count))
         entry_to_config(tt->entries[index - (n - tt_count)], ABQ_STRATEGY_TILED, x_bits, w_bits, is_signed, 0, cfg);
@@ -790,6 +791,8 @@ static int large_tiles_int8(int x_bits, int w_bits, int is_signed, const LargeTi
     return 0;
 }
 
+static bool row_sums_at_hand(const abq_gemm_state *st);
+
 // Picks the tiled-kernel tile for a shape.  Pairs with a cost model (large_tiles_int8) weigh their large
 // tiles against 128x128 once the shape has 200 tiles of 128x128; everything else goes by the thresholds
 // below (measured on MI355X, LLaMA shapes): smaller tiles win by filling the chip.
@@ -885,6 +888,26 @@ static abq_status switch_to_tiled(abq_gemm_state *st)
             if (e.lds != 0 && e.tm == want[0] && e.tn == want[1] && e.wm == want[2] && e.wn == want[3] && e.wk == want[4] && e.kb == 128)
                 pick = i;
         }
+    }
+    {
+        // Long K on a 64x64 grid that leaves compute units free: that tile with four groups of waves.  A K tile there is the chain of
+        // one wave per SIMD, and four share it; on short K the two further partial tiles cost what the shorter loop gains.  Two
+        // groups -> four, weights from memory and activations converted in the call, us: 128 x 5120 x 13824 W4A8 30.0 -> 28.9,
+        // W4A4 24.0 -> 23.3, W2A4 25.3 -> 23.3, W2A2 24.8 -> 22.7; 256 x 2048 x 16384 33.1 -> 31.1, 27.9 -> 26.2, 29.3 -> 27.0,
+        // 28.4 -> 25.7; 128 x 6144 x 8192 (192 workgroups) 21.1 -> 21.2, 17.4 -> 17.4, 18.0 -> 17.3, 17.5 -> 16.8.  W2A8 gains up to
+        // 112 workgroups only: 400 x 1024 x 11008 22.7 -> 22.0, but 128 x 4096 x 11008 21.4 -> 22.8, 192 x 4096 x 8192 17.9 -> 19.2.
+        // Unsigned 8-bit operands have no tile of two groups; one -> four where their row sums are to be had (without them another
+        // kernel runs): W2A8 128 x 5120 x 13824 34.7 -> 26.9, 128 x 5120 x 5120 16.4 -> 13.6, W4A8 33.3 -> 29.2, 16.6 -> 16.4.
+        const KernelEntry &p = tt->entries[pick];
+        const bool flip = !c.is_signed && (c.x_bits == 8 || c.w_bits == 8);
+        if (p.tm == 1 && p.tn == 1 && p.wm == 2 && p.wn == 2 && p.kb == 128 && (flip ? row_sums_at_hand(st) : p.wk == 2) &&
+            st->K >= (flip ? 4096 : 8192) &&
+            (long)((st->M + 63) / 64) * ((st->N + 63) / 64) <= (!flip && c.x_bits == 8 && c.w_bits == 2 ? 112 : 192))
+            for (int i = 0; i < tt->count; ++i) {
+                const KernelEntry &e = tt->entries[i];
+                if (e.tm == 1 && e.tn == 1 && e.wm == 2 && e.wn == 2 && e.wk == 4 && e.kb == 128)
+                    pick = i;
+            }
     }
     abq_tile_config cfg;
     entry_to_config(tt->entries[pick], ABQ_STRATEGY_TILED, c.x_bits, c.w_bits, c.is_signed, 0, &cfg);
@@ -1549,6 +1572,24 @@ static RowSumPlan row_sum_plan(const abq_gemm_state *st, size_t converted)
     return p;
 }
 
+// Whether the sums an unsigned 8-bit operand needs on the prefill kernel are set or can be taken, as the state stands.
+static bool row_sums_at_hand(const abq_gemm_state *st)
+{
+    const size_t xb = st->x_layout == ABQ_LAYOUT_TILED ? 0 : planes_bytes(st->M, st->K, st->cfg.x_bits);
+    const size_t wb = st->w_layout == ABQ_LAYOUT_TILED ? 0 : planes_bytes(st->N, st->K, st->cfg.w_bits);
+    abq_gemm_state tiled = *st;
+    tiled.strategy = ABQ_STRATEGY_TILED;
+    return row_sum_plan(&tiled, xb + wb).ok;
+}
+
+// The tile of an unsigned 8-bit operand depends on whether the sums are at hand: picked again once layouts, sums or workspace
+// have changed.
+static void repick_unsigned_tile(abq_gemm_state *st)
+{
+    if (st->strategy == ABQ_STRATEGY_TILED && st->auto_chosen && !st->group_size && !st->cfg.is_signed && (st->cfg.x_bits == 8 || st->cfg.w_bits == 8))
+        (void)switch_to_tiled(st);
+}
+
 // Whether the state's kernel is one that wants row sums handed in.
 static bool wants_row_sums(const abq_gemm_state *st)
 {
@@ -1596,6 +1637,7 @@ static void reconsider_decode_tiled(abq_gemm_state *st)
     if (st->strategy == ABQ_STRATEGY_TILED && st->auto_chosen && !st->group_size && !st->act && st->x_layout == ABQ_LAYOUT_TILED &&
         st->w_layout == ABQ_LAYOUT_TILED && decode_tiled_pays(st->cfg.x_bits, st->cfg.w_bits, st->M, st->N, st->K))
         (void)switch_to_decode_tiled(st);
+    repick_unsigned_tile(st);
     apply_tuned(st);
 }
 
@@ -1911,8 +1953,9 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
                 const KernelEntry &want = t->entries[st->variant];
                 for (int i = 0; i < st->variant; ++i) {
                     const KernelEntry &o = t->entries[i];
+                    // (an unlisted tile has no such kernel: the one whose waves do not split K)
                     if (!(o.flags & kNeedsRowSums) && o.tm == want.tm && o.tn == want.tn && o.wm == want.wm && o.wn == want.wn &&
-                        o.wk == want.wk && o.kb == want.kb)
+                        o.wk == ((want.flags & kUnlisted) ? 1 : want.wk) && o.kb == want.kb)
                         variant = i;
                 }
                 if (variant < 0)
@@ -2053,6 +2096,8 @@ abq_status abq_gemm_set_operand_layout(abq_gemm_state *st, int x_layout, int w_l
         if (switch_to_tiled(&alt) == ABQ_OK)
             next = alt;
     }
+    if (rc == ABQ_OK)
+        repick_unsigned_tile(&next);
     if (rc == ABQ_OK)
         apply_tuned(&next); // a measured best tile for this shape on these layouts, if the table holds one
     // activation records declared padded are read by the decode kernel on prepared operands only
@@ -2198,6 +2243,7 @@ abq_status abq_gemm_set_workspace(abq_gemm_state *st, void *workspace, size_t by
         if (switch_to_decode_tiled(&tmp) == ABQ_OK && decode_tiled_x_ok(&tmp) && bytes >= abq_gemm_workspace_bytes(&tmp))
             *st = tmp;
     }
+    repick_unsigned_tile(st);
     apply_tuned(st); // (a tile that converts plane activations can be taken now that there is room for them)
     return ABQ_OK;
 }

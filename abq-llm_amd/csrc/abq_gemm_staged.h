@@ -632,16 +632,6 @@ template <int QB, int PB, bool FP6, int TM, int TN, int WM, int WN, bool GROUPED
     static_assert(3 * kBuf <= 160 * 1024, "three stages fit a compute unit's LDS");
 };
 
-// Four groups of waves that split K on the 64x64 tile, where a launch leaves compute units free anyway: a K tile then is the
-// chain of one wave per SIMD (0.28 us; two groups 0.15; deeper pipelines change nothing), and four share it.  On short K the two
-// further partial tiles cost what the shorter loop gains, and W8A8 is bound by its LDS traffic (128 x 4096 x 4096 10.1 us with
-// three groups against 8.9 with one).  128 rows, two groups -> four, us: W2A8 5120 x 13824 19.5 -> 17.6, W4A8 24.7 -> 23.2, W2A4
-// 21.6 -> 19.2, W2A2 4096 x 11008 18.2 -> 16.7, but W2A8 4096 x 4096 9.3 -> 9.7; one group -> four: W4A8 5120 x 5120 11.0 -> 10.4.
-template <int QB, int PB, bool FP6, int TM, int TN, int WM, int WN, bool GROUPED, int WK> constexpr bool staged_four_k_groups()
-{
-    return TM == 1 && TN == 1 && WM == 2 && WN == 2 && WK < 4 && !GROUPED && !FP6 && QB + PB < 16;
-}
-
 template <int QB, int PB, bool SIGNED, bool FP6, int TM, int TN, int WM, int WN, bool GROUPED = false, int WK = 1>
 static hipError_t launch_mfma_staged(const GemmArgs &a, hipStream_t stream)
 {
@@ -649,10 +639,6 @@ static hipError_t launch_mfma_staged(const GemmArgs &a, hipStream_t stream)
     if (GROUPED && a.group_size != 128)
         return hipErrorInvalidValue; // one scale per K tile
     const int m_blocks = (a.M + BM - 1) / BM, n_blocks = (a.N + BN - 1) / BN;
-    if constexpr (staged_four_k_groups<QB, PB, FP6, TM, TN, WM, WN, GROUPED, WK>()) {
-        if ((long)m_blocks * n_blocks <= 192 && a.K >= (WK == 1 ? 4096 : 8192))
-            return launch_mfma_staged<QB, PB, SIGNED, FP6, TM, TN, WM, WN, GROUPED, 4>(a, stream);
-    }
     using Stages = StagedStages<QB, PB, FP6, TM, TN, WM, WN, GROUPED, WK>;
     constexpr int S = Stages::value;
     const int npx = (n_blocks + 7) / 8;

@@ -500,6 +500,16 @@ static hipError_t launch_mfma_tiled(const GemmArgs &a, hipStream_t stream)
 #else
 #define ABQ_STAGED_KSPLIT(SG) ABQ_SENTRY_K(SG, 1, 1, 2, 2, 2) ABQ_SENTRY_K(SG, 2, 1, 2, 2, 2) ABQ_SENTRY_K(SG, 2, 2, 2, 2, 2)
 #endif
+// The 64 x 64 tile with four groups that split K, for small grids on long K (the host's rule, with figures: switch_to_tiled).
+// Not W8A8, which is bound by its LDS traffic (128 x 4096 x 4096 10.1 us with three groups against 8.9 with one).
+#define ABQ_SENTRY_K4(SG, FLAGS)                                                                       \
+    { 32, 1, 1, 2, 2, 4, 4, &launch_mfma_staged<ABQ_Q, ABQ_P, SG, false, 1, 1, 2, 2, false, 4>, 128,   \
+      StagedStages<ABQ_Q, ABQ_P, false, 1, 1, 2, 2, false, 4>::kLds, FLAGS },
+#if ABQ_Q == 8 && ABQ_P == 8
+#define ABQ_STAGED_K4(SG, FLAGS)
+#else
+#define ABQ_STAGED_K4(SG, FLAGS) ABQ_SENTRY_K4(SG, FLAGS)
+#endif
 // Activations wider than the weights: a 128 x 256 tile (eight waves of 64 x 64, 2 along M, 4 along N) moves fewer
 // bytes per MFMA than 256 x 128, since a row of activations is the longer record.
 #if ABQ_Q > ABQ_P
@@ -521,12 +531,12 @@ static hipError_t launch_mfma_tiled(const GemmArgs &a, hipStream_t stream)
 static const KernelEntry kSigned[] = { ABQ_ENTRY_T(4, 4) ABQ_ENTRY_T(2, 4) ABQ_SENTRY(true, 2, 2, 2, 2) ABQ_SENTRY(true, 2, 1, 2, 2)
                                        ABQ_SENTRY(true, 1, 1, 2, 2) ABQ_TILED_HALF_VARIANTS(ABQ_HENTRY_T)
                                        ABQ_SENTRY(true, 2, 2, 4, 2) ABQ_WENTRY_T(2, 2, 4, 4) ABQ_STAGED_256(true)
-                                       ABQ_STAGED_WIDE_N(true) ABQ_STAGED_KSPLIT(true) };
+                                       ABQ_STAGED_WIDE_N(true) ABQ_STAGED_KSPLIT(true) ABQ_STAGED_K4(true, kUnlisted) };
 #if ABQ_Q < 8 && ABQ_P < 8
 static const KernelEntry kUnsigned[] = { ABQ_ENTRY_F(4, 4) ABQ_ENTRY_F(2, 4) ABQ_SENTRY(false, 2, 2, 2, 2) ABQ_SENTRY(false, 2, 1, 2, 2)
                                          ABQ_SENTRY(false, 1, 1, 2, 2) ABQ_TILED_HALF_VARIANTS(ABQ_HENTRY_F)
                                          ABQ_SENTRY(false, 2, 2, 4, 2) ABQ_WENTRY_F(2, 2, 4, 4) ABQ_STAGED_256(false)
-                                         ABQ_STAGED_WIDE_N(false) ABQ_STAGED_KSPLIT(false) };
+                                         ABQ_STAGED_WIDE_N(false) ABQ_STAGED_KSPLIT(false) ABQ_STAGED_K4(false, kUnlisted) };
 #else
 // Pairs with an unsigned 8-bit operand: the kernel above under every tuple, which takes the row sums of the
 // correction itself, and behind it, under the same tuples, the staged kernel for the tiles it is built for, which
@@ -542,7 +552,8 @@ static const KernelEntry kUnsigned[] = { ABQ_ENTRY_F(4, 4) ABQ_ENTRY_F(2, 4) ABQ
 static const KernelEntry kUnsigned[] = { ABQ_TILED_VARIANTS(ABQ_ENTRY_F) ABQ_TILED_HALF_VARIANTS(ABQ_HENTRY_F)
                                          ABQ_TILED_WIDE_VARIANTS(ABQ_WENTRY_F)
                                          ABQ_SENTRY_U8(2, 2, 2, 2) ABQ_SENTRY_U8(2, 1, 2, 2) ABQ_SENTRY_U8(1, 1, 2, 2)
-                                         ABQ_SENTRY_U8(2, 2, 4, 2) ABQ_STAGED_U8_LARGE };
+                                         ABQ_SENTRY_U8(2, 2, 4, 2) ABQ_STAGED_U8_LARGE
+                                         ABQ_STAGED_K4(false, kNeedsRowSums | kUnlisted) };
 #endif
 #else
 static const KernelEntry kSigned[] = { ABQ_TILED_VARIANTS(ABQ_ENTRY_T) ABQ_TILED_HALF_VARIANTS(ABQ_HENTRY_T)

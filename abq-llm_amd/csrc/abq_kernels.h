@@ -54,6 +54,7 @@ struct KernelEntry {
                             // in front of it in the table is the kernel that runs when the sums are not to be had
 };
 constexpr int kNeedsRowSums = 1;
+constexpr int kUnlisted = 2; // a tile for one range of shapes: named and picked like the others, but not part of the native tile space
 
 struct KernelTable {
     int x_bits, w_bits, is_signed;

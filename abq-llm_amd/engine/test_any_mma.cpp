@@ -664,15 +664,28 @@ int main(int argc, char **argv)
     // the fastest tile of each operand layout (planes, K-tiled, FP6), for --tuning-out
     double layout_tops[3] = { 0, 0, 0 };
     abq_tile_config layout_best[3];
-    const int ncfg = abq_native_config_count(x_bits, w_bits, is_signed);
+    std::vector<abq_tile_config> tiles;
+    for (int i = 0; i < abq_native_config_count(x_bits, w_bits, is_signed); ++i) {
+        abq_tile_config cfg;
+        if (abq_native_config_get(x_bits, w_bits, is_signed, i, &cfg) == ABQ_OK)
+            tiles.push_back(cfg);
+    }
+    // ... and the 64 x 64 tile whose four groups of waves split K, which the native list leaves out, where the pair has it
+    if (M > 16) {
+        const abq_tile_config four = { x_bits, w_bits, is_signed, 64, 64, 512, 32, 32, 128, 32, 32, 32, 4 };
+        abq_gemm_state probe;
+        if (abq_gemm_init(&four, 0, 0, 0, d_xp, d_xp, M, N, K, d_xp, nullptr, 0, ABQ_OUT_I32, &probe) == ABQ_OK)
+            tiles.push_back(four);
+    }
+    const int ncfg = (int)tiles.size();
     // + the library's choice (+ its choice on prepared operands (+ the same with the weights padded as well))
     const int nlines = ncfg + (M <= 16 ? (padded && wq != w_bits ? 3 : 2) : (padded_prefill ? 2 : 1));
     for (int i = 0; i < nlines; ++i) {
         abq_tile_config cfg;
         const bool library_default = i >= ncfg;
         const bool prepared = M <= 16 && i >= ncfg + 1, pad_weights = i == ncfg + (M <= 16 ? 2 : 1);
-        if (!library_default && abq_native_config_get(x_bits, w_bits, is_signed, i, &cfg) != ABQ_OK)
-            continue;
+        if (!library_default)
+            cfg = tiles[i];
         char name[160] = "library default";
         const char *how = pad_weights ? " (padded records)" : (with_sums && d_wpad) ? " (with row sums)" : "";
         if (prepared)
