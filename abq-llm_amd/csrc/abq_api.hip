@@ -10,6 +10,7 @@
 #include <mutex>
 
 #include "abq_kernels.h"
+#include "abq_rows_grouped.h"
 #include "abq_tuning.h"
 
 namespace abq {
@@ -82,6 +83,26 @@ struct Registry {
 #undef ABQ_REG
     }
 };
+
+// reserved[4] bit 4: the kernel that streams the weights once for up to 64 rows (abq_gemm_rows_grouped.hip) runs for this
+// group-scale state, by the library's rule, a measured entry or because it was asked for; grid, workgroup and LDS are then its own.
+// A state moved to another kernel loses the bit (resolve).
+constexpr int kRowsKernel = 16;
+static bool rows_kernel(const abq_gemm_state *st) { return (st->reserved[4] & kRowsKernel) != 0; }
+// its tuple (NSTAGE 7): 64 rows by 16 weight rows at the least, eight waves that own blocks of 512 elements of K
+static abq_tile_config rows_config(int x_bits, int w_bits) { return abq_tile_config{ x_bits, w_bits, 1, 64, 16, 4096, 64, 16, 512, 16, 16, 64, 7 }; }
+constexpr int kRowsStage = 7;
+
+static void set_rows_kernel(abq_gemm_state *st, bool on)
+{
+    st->reserved[4] = (st->reserved[4] & ~kRowsKernel) | (on ? kRowsKernel : 0);
+    if (!on)
+        return;
+    const RowsPlan plan = rows_grouped_plan(st->cfg.w_bits, st->M, st->N, st->K, st->act, st->w_zero != nullptr);
+    st->grid_dim = abq_dim3{ plan.grid, 1, 1 };
+    st->block_dim = abq_dim3{ (unsigned)(64 * plan.waves), 1, 1 };
+    st->shared_mem_size = plan.lds;
+}
 
 static const Registry &registry()
 {
@@ -270,6 +291,17 @@ static abq_status resolve(const abq_tile_config *cfg, int x_bits, int w_bits, in
 {
     const Registry &reg = registry();
     int strategy = cfg ? strategy_of_mma(*cfg) : ABQ_STRATEGY_AUTO;
+    st->reserved[4] &= ~kRowsKernel;
+    if (strategy == ABQ_STRATEGY_MFMA16 && cfg->nstage == kRowsStage) {
+        // the kernel for 17 rows and more asked for by name: it carries group scales only, so the state runs once they are set
+        const abq_tile_config want = rows_config(x_bits, w_bits);
+        if (memcmp(cfg, &want, sizeof want) != 0 || !rows_grouped_runs(M, N, K, x_bits, w_bits, 128, 0))
+            return ABQ_ERR_UNSUPPORTED;
+        st->strategy = ABQ_STRATEGY_TILED;
+        st->variant = -1;
+        st->cfg = want;
+        return ABQ_OK;
+    }
     if (strategy == ABQ_STRATEGY_FP6) {
         if (cfg->nstage != 5 || cfg->warp_k != 128 || cfg->block_k != 128 || cfg->warp_m <= 0 || cfg->warp_n <= 0 ||
             cfg->warp_m % 32 || cfg->warp_n % 32 || cfg->block_m % cfg->warp_m || cfg->block_n % cfg->warp_n)
@@ -1054,9 +1086,6 @@ static bool biased_w(const abq_gemm_state *st) { return (st->reserved[4] & 2) !=
 // (abq_relayout_planes_padded), which is how the decode kernel on prepared operands reads activations of 3, 5, 6 or
 // 7 bits (abq_gemm_set_padded_activations)
 static bool padded_x(const abq_gemm_state *st) { return (st->reserved[4] & 4) != 0; }
-// reserved[4] bit 3: a group-scale state whose tile is the library's choice by its rules (no tile asked for, none measured):
-// the kernel that streams the weights once (abq_gemm_rows_grouped.hip) runs in the tile's place where it is ahead
-constexpr int kRowsKernel = 8;
 static bool one_field(int bits) { return bits == 2 || bits == 4 || bits == 8; }
 // Width of the activation records the decode kernel on prepared operands reads for a pair.
 static int decode_tiled_x_bits(int x_bits) { return abq_padded_bits(x_bits); }
@@ -1218,9 +1247,34 @@ static bool decode_tiled_grouped_pays(int x_bits, int w_bits, int M, int N, int 
     return decode_us < 0.9 * tiled_us;
 }
 
+// What the table of measured tiles says of that kernel for a shape: 1 it is the fastest entry, -1 it was measured and a tile is
+// faster, 0 it was not measured (an entry of a tile alone says nothing of it).
+static int rows_grouped_by_table(const abq_gemm_state *st, int group_size)
+{
+    const abq_tile_config &c = st->cfg;
+    TunedTile best;
+    if (!rows_grouped_runs(st->M, st->N, st->K, c.x_bits, c.w_bits, group_size, st->act) || !c.is_signed ||
+        !tuning_find(c.x_bits, c.w_bits, 1, st->M, st->N, st->K, group_size, 1 << ABQ_LAYOUT_TILED, &best))
+        return 0;
+    if (best.cfg.nstage == kRowsStage)
+        return 1;
+    return tuning_measured(c.x_bits, c.w_bits, 1, st->M, st->N, st->K, group_size, kRowsStage) ? -1 : 0;
+}
+
+// A state on the decode kernel's group-scale variant with more than one block of 16 rows: the kernel that streams the weights
+// once for all of them, where it covers the chip.
+static void settle_row_blocks(abq_gemm_state *st)
+{
+    const abq_tile_config &c = st->cfg;
+    set_rows_kernel(st, c.is_signed && rows_grouped_runs(st->M, st->N, st->K, c.x_bits, c.w_bits, st->group_size, st->act) &&
+                            rows_grouped_covers(st->M, st->N));
+}
+
 static bool decode_tiled_grouped_fits(const abq_gemm_state *st, int group_size, int act)
 {
     const abq_tile_config &c = st->cfg;
+    if (rows_grouped_by_table(st, group_size) != 0)
+        return false; // a measured entry decides, where the tile is picked
     const KernelTable *t = find_table(registry().decode_tiled_grouped, c.x_bits, c.w_bits, c.is_signed);
     return t && t->count > 0 && st->auto_chosen && (group_size == 128 || group_size == 64) && (!act || st->N % 32 == 0) &&
            decode_tiled_grouped_pays(c.x_bits, c.w_bits, st->M, st->N, st->K, act, group_size);
@@ -1239,7 +1293,14 @@ static abq_status pick_grouped_tiled(abq_gemm_state *state)
             return rc;
     }
     const abq_tile_config &c = state->cfg;
-    state->reserved[4] &= ~kRowsKernel;
+    const bool rows_asked = !state->auto_chosen && c.nstage == kRowsStage;
+    if (rows_asked) {
+        if (!rows_grouped_runs(state->M, state->N, state->K, c.x_bits, c.w_bits, state->group_size, state->act))
+            return ABQ_ERR_UNSUPPORTED;
+        set_rows_kernel(state, true);
+        return ABQ_OK;
+    }
+    bool rows = false;
     const KernelTable *tg = find_table(registry().tiled_grouped, c.x_bits, c.w_bits, c.is_signed);
     if (!tg)
         return ABQ_ERR_UNSUPPORTED;
@@ -1293,18 +1354,18 @@ static abq_status pick_grouped_tiled(abq_gemm_state *state)
                 if (usable(tg->entries[i]) && tg->entries[i].lds != 0 && block_m(tg->entries[i]) == 64 && block_n(tg->entries[i]) == 64 &&
                     tg->entries[i].wk == 2)
                     pick = i;
-        // (the tile picked here stays the state's: it runs where the kernel for few rows does not)
-        state->reserved[4] |= kRowsKernel;
+        // The kernel that streams the weights once, by its rule or a measured entry (the state keeps the tile picked here as its
+        // tuple then).
+        const int by_table = rows_grouped_by_table(state, state->group_size);
+        rows = by_table ? by_table > 0 : rows_grouped_pays(c.x_bits, c.w_bits, c.is_signed, state->M, state->N, state->K, state->group_size, state->act);
         // a measured best tile for this shape and group size comes before the rules above
         TunedTile t;
         if (tuning_find(c.x_bits, c.w_bits, c.is_signed, state->M, state->N, state->K, state->group_size, 1 << ABQ_LAYOUT_TILED, &t) &&
             t.cfg.nstage == 4 && t.cfg.warp_k > 0)
             for (int i = 0; i < tg->count; ++i)
                 if (usable(tg->entries[i]) && block_m(tg->entries[i]) == t.cfg.block_m && block_n(tg->entries[i]) == t.cfg.block_n &&
-                    tg->entries[i].mi * tg->entries[i].tm == t.cfg.warp_m && tg->entries[i].wk == t.cfg.block_k / t.cfg.warp_k) {
+                    tg->entries[i].mi * tg->entries[i].tm == t.cfg.warp_m && tg->entries[i].wk == t.cfg.block_k / t.cfg.warp_k)
                     pick = i;
-                    state->reserved[4] &= ~kRowsKernel;
-                }
     } else {
         const int wk = c.warp_k > 0 ? c.block_k / c.warp_k : 1;
         for (int i = 0; i < tg->count; ++i)
@@ -1324,6 +1385,7 @@ static abq_status pick_grouped_tiled(abq_gemm_state *state)
         state->block_dim = abq_dim3{ (unsigned)(64 * e.wm * e.wn * e.wk), 1, 1 };
         state->shared_mem_size = e.lds ? e.lds : 2 * (size_t)(bm + bn) * (e.kb + 16) + (bm + bn) * 4;
     }
+    set_rows_kernel(state, rows);
     return ABQ_OK;
 }
 
@@ -1341,6 +1403,8 @@ static void apply_tuned(abq_gemm_state *st)
     TunedTile t;
     if (!tuning_find(c.x_bits, c.w_bits, c.is_signed, st->M, st->N, st->K, 0, mask, &t))
         return;
+    if (t.cfg.nstage == kRowsStage)
+        return; // (carries group scales only)
     // the decode kernel on prepared operands converts activations that arrive as planes into the workspace, like the
     // prefill kernels; it cannot be chosen before there is one
     if (t.cfg.nstage == 6 && st->x_layout != ABQ_LAYOUT_TILED &&
@@ -1390,6 +1454,8 @@ abq_status abq_gemm_set_scales(abq_gemm_state *state, const float *x_scale, cons
                                find_table(registry().decode_grouped, c.x_bits, c.w_bits, c.is_signed);
         if (decode_ok || decode_tiled_ok) {
             state->variant = 0;
+            if (decode_tiled_ok)
+                settle_row_blocks(state);
         } else {
             const abq_status rc = pick_grouped_tiled(state);
             if (rc != ABQ_OK) {
@@ -1420,6 +1486,8 @@ abq_status abq_gemm_set_zero_points(abq_gemm_state *state, const float *x_zero, 
     state->w_zero = w_zero;
     state->x_group_sums = x_group_sums;
     state->w_zero_term = w_zero_term;
+    if (rows_kernel(state)) // (the plan follows from what the workgroups have to hold)
+        set_rows_kernel(state, true);
     return ABQ_OK;
 }
 
@@ -1444,6 +1512,8 @@ abq_status abq_gemm_set_activation(abq_gemm_state *state, int act)
         }
     }
     state->act = act;
+    if (rows_kernel(state))
+        set_rows_kernel(state, true);
     return ABQ_OK;
 }
 
@@ -1835,7 +1905,8 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
                                           : st->group_size ? reg.tiled_grouped
                                                            : reg.tiled,
                                           c.x_bits, c.w_bits, c.is_signed);
-        if (!t || st->variant < 0 || st->variant >= t->count)
+        const bool rows = st->group_size && rows_kernel(st);
+        if (!t || (!rows && (st->variant < 0 || st->variant >= t->count)))
             return ABQ_ERR_NOT_INITIALIZED;
         // Activations that arrive as planes and whose row sums a branch below will take from those planes: the
         // conversion's launch takes the sums as well (further workgroups of the same grid), where that branch puts them.
@@ -1870,6 +1941,10 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
                 return hip_status(e);
             a.W = reinterpret_cast<const uint32_t *>(ws + xb);
         }
+        if (rows)
+            return hip_status(c.w_bits == 2   ? launch_rows_grouped_8<2>(a, (hipStream_t)stream)
+                              : c.w_bits == 4 ? launch_rows_grouped_8<4>(a, (hipStream_t)stream)
+                                              : launch_rows_grouped_8<8>(a, (hipStream_t)stream));
         int variant = st->variant;
         if (st->strategy == ABQ_STRATEGY_TILED && !c.is_signed && !biased && x_plane_bits(st) < c.x_bits && w_plane_bits(st) < c.w_bits) {
             // Unsigned codes that leave the top bit of their records clear are signed codes of the records' width as
@@ -1962,13 +2037,7 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
                     return ABQ_ERR_NOT_INITIALIZED;
             }
         }
-        if (st->strategy == ABQ_STRATEGY_TILED && (st->reserved[4] & kRowsKernel) &&
-            rows_grouped_pays(c.x_bits, c.w_bits, c.is_signed, st->M, st->N, st->K, st->group_size, st->act))
-            e = c.w_bits == 2   ? launch_rows_grouped_8<2>(a, (hipStream_t)stream)
-                : c.w_bits == 4 ? launch_rows_grouped_8<4>(a, (hipStream_t)stream)
-                                : launch_rows_grouped_8<8>(a, (hipStream_t)stream);
-        else
-            e = t->entries[variant].launch(a, (hipStream_t)stream);
+        e = t->entries[variant].launch(a, (hipStream_t)stream);
     } else {
         if (st->group_size && st->strategy != ABQ_STRATEGY_DECODE)
             return ABQ_ERR_NOT_INITIALIZED; // group scales live on the decode and tiled kernels only
@@ -2154,6 +2223,7 @@ static abq_status set_operand_layout_by_rules(abq_gemm_state *st, int x_layout, 
     if (x_layout == ABQ_LAYOUT_TILED && w_layout == ABQ_LAYOUT_TILED && st->group_size && st->strategy != ABQ_STRATEGY_DECODE_TILED &&
         decode_tiled_grouped_fits(st, st->group_size, st->act) && switch_to_decode_tiled(st) == ABQ_OK) {
         st->variant = 0;
+        settle_row_blocks(st);
         st->x_layout = x_layout;
         st->w_layout = w_layout;
         return ABQ_OK;

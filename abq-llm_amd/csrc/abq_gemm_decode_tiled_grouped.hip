@@ -656,11 +656,6 @@ template <int Q, int P, bool SIGNED, bool XDYN = false> static hipError_t launch
         return hipErrorInvalidValue;
     if (a.act && a.N % 32 != 0)
         return hipErrorInvalidValue;
-    if constexpr (Q == 8 && SIGNED && !XDYN) {
-        // more than one block of 16 rows: the kernel that streams the weights once for all of them
-        if (rows_grouped_runs(a.M, a.N, a.K, Q, P, a.group_size, a.act) && rows_grouped_covers(a.M, a.N))
-            return launch_rows_grouped_8<P>(a, stream);
-    }
     if constexpr (!XDYN) {
         if (a.group_size == 64)
             return launch_dtg<Q, P, SIGNED, false, true>(a, stream);

@@ -16,7 +16,7 @@
 //     once for all MB blocks of 16 rows;
 //   * the activations of a step go from L2 into a ring of R buffers of the wave's own LDS (global_load_lds, no registers);
 //     a buffer is refilled as soon as its operands are in registers, so R steps are in flight beside the products;
-//   * T is chosen so that the workgroups make as few rounds of the 256 compute units as possible (rows_pick_tiles).
+//   * T is chosen so that the workgroups make as few rounds of the 256 compute units as possible (rows_grouped_plan).
 // The order of every sum depends on K alone, so all T and MB give the same bits.
 //
 // W4A8 with zero points on both sides, 43 rows (us, against the 64x64 and 64x128 prefill tiles on the same records): 4096 x
@@ -27,35 +27,13 @@
 
 #include "abq_decode_loads.h"
 #include "abq_kernels.h"
+#include "abq_rows_grouped.h"
 
 #if !defined(ABQ_Q) || !defined(ABQ_P) || ABQ_Q != 8
 #error "compile with -DABQ_Q=8 -DABQ_P=<w_bits>"
 #endif
 
 namespace abq {
-
-constexpr int kRowsWaves = 8;
-
-// Steps whose weights are in flight beside the one multiplied: a whole block where the registers hold it beside the
-// accumulators, else two.
-constexpr int rows_ahead(int p, int t, int mb) { return 4 * t * (p + mb) <= 150 ? 4 : 2; }
-// buffers of the activation ring: three steps of 32 rows fit beside the scales, two of 48 or 64
-constexpr int rows_ring(int p, int t, int mb) { return mb <= 2 && rows_ahead(p, t, mb) == 4 ? 3 : 2; }
-// instances that are built: what registers and LDS hold
-constexpr bool rows_built(int p, int t, int mb) { return t * p <= 24 && t * mb <= 18; }
-// LDS: the activation rings, then scales, zero points and group sums per wave (the waves' partial tiles take the place of all
-// of these at the end) | the rows' scales and zero points, the tiles' zero-point terms
-constexpr int rows_scale_loads(int t, int mb, bool zp) { return zp ? 2 * t + mb : t; }
-constexpr size_t rows_lds_of_loop(int nw, int p, int t, int mb, bool zp)
-{
-    return (size_t)nw * (rows_ring(p, t, mb) * mb * 2048 + rows_scale_loads(t, mb, zp) * 256);
-}
-constexpr size_t rows_lds_of_sum(int nw, int t, int mb) { return (size_t)nw * t * mb * 1024; }
-constexpr size_t rows_lds_for_rows(int nw, int p, int t, int mb, bool zp) // where the rows' scales lie
-{
-    return rows_lds_of_loop(nw, p, t, mb, zp) > rows_lds_of_sum(nw, t, mb) ? rows_lds_of_loop(nw, p, t, mb, zp) : rows_lds_of_sum(nw, t, mb);
-}
-constexpr size_t rows_lds(int nw, int p, int t, int mb, bool zp) { return rows_lds_for_rows(nw, p, t, mb, zp) + 512 + 512; }
 
 template <int P, int T, int MB, bool ZP>
 __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmArgs a, int m_blocks)
@@ -318,42 +296,16 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmA
 
 // ---- launch -------------------------------------------------------------------------------------------------------
 
-// Tiles of 16 weight rows per workgroup.  A workgroup fills a compute unit's LDS, so workgroups run in rounds of 256; a
-// round's time is the weights of T tiles from memory plus the activations from L2, which is about three times as fast.
-template <int P> static int rows_pick_tiles(const GemmArgs &a, int mb)
-{
-    const int nw = (a.K / 128 + 3) / 4 < kRowsWaves ? (a.K / 128 + 3) / 4 : kRowsWaves;
-    const long tiles = (a.N + 15) / 16, m_blocks = (a.M + 63) / 64;
-    const int choices[5] = { 1, 2, 3, 4, 6 };
-    int best = 0;
-    double best_cost = 0;
-    for (int c : choices) {
-        if (!rows_built(P, c, mb) || (a.act && (c & 1)) || rows_lds(nw, P, c, mb, a.w_zero != nullptr) > 160 * 1024)
-            continue;
-        const double cost = (double)(((tiles + c - 1) / c * m_blocks + 255) / 256) * (3.0 * c * (P * 256 + 128) + mb * 2048.0);
-        if (best == 0 || cost < best_cost) {
-            best = c;
-            best_cost = cost;
-        }
-    }
-    return best;
-}
-
-template <int P, int T, int MB, bool ZP> static hipError_t launch_rows_instance(const GemmArgs &a, hipStream_t stream)
+template <int P, int T, int MB, bool ZP> static hipError_t launch_rows_instance(const GemmArgs &a, const RowsPlan &plan, hipStream_t stream)
 {
     if constexpr (!rows_built(P, T, MB)) {
         return hipErrorInvalidValue;
     } else {
-        const int nblocks = (a.K / 128 + 3) / 4, nw = nblocks < kRowsWaves ? nblocks : kRowsWaves;
-        const size_t lds = rows_lds(nw, P, T, MB, ZP);
         static const hipError_t attr =
             hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_rows_grouped<P, T, MB, ZP>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (attr != hipSuccess)
             return attr;
-        if (lds > 160 * 1024)
-            return hipErrorInvalidValue;
-        const int wgs = ((a.N + 15) / 16 + T - 1) / T, m_blocks = (a.M + MB * 16 - 1) / (MB * 16);
-        hipLaunchKernelGGL((gemm_rows_grouped<P, T, MB, ZP>), dim3((wgs + 7) / 8 * 8 * m_blocks), dim3(64 * nw), lds, stream, a, m_blocks);
+        hipLaunchKernelGGL((gemm_rows_grouped<P, T, MB, ZP>), dim3(plan.grid), dim3(64 * plan.waves), plan.lds, stream, a, plan.m_blocks);
         return hipGetLastError();
     }
 }
@@ -366,22 +318,24 @@ hipError_t ABQ_CAT(launch_rows_grouped_8, _, ABQ_P)(const GemmArgs &a, hipStream
     if (!rows_grouped_runs(a.M, a.N, a.K, 8, ABQ_P, a.group_size, a.act) || !a.w_scale || !a.x_scale || (a.w_zero && !a.x_group_sums) ||
         (a.x_zero && !a.w_zero_term))
         return hipErrorInvalidValue;
-    const int m_blocks = (a.M + 63) / 64, mb = ((a.M + m_blocks - 1) / m_blocks + 15) / 16;
+    const RowsPlan plan = rows_grouped_plan(ABQ_P, a.M, a.N, a.K, a.act, a.w_zero != nullptr);
     auto with_t = [&](auto bb, auto zp) -> hipError_t {
         constexpr int MB = decltype(bb)::value;
         constexpr bool ZP = decltype(zp)::value;
-        switch (rows_pick_tiles<ABQ_P>(a, MB)) {
-        case 1: return launch_rows_instance<ABQ_P, 1, MB, ZP>(a, stream);
-        case 2: return launch_rows_instance<ABQ_P, 2, MB, ZP>(a, stream);
-        case 3: return launch_rows_instance<ABQ_P, 3, MB, ZP>(a, stream);
-        case 4: return launch_rows_instance<ABQ_P, 4, MB, ZP>(a, stream);
-        case 6: return launch_rows_instance<ABQ_P, 6, MB, ZP>(a, stream);
+        switch (plan.tiles) {
+        case 1: return launch_rows_instance<ABQ_P, 1, MB, ZP>(a, plan, stream);
+        case 2: return launch_rows_instance<ABQ_P, 2, MB, ZP>(a, plan, stream);
+        case 3: return launch_rows_instance<ABQ_P, 3, MB, ZP>(a, plan, stream);
+        case 4: return launch_rows_instance<ABQ_P, 4, MB, ZP>(a, plan, stream);
+        case 6: return launch_rows_instance<ABQ_P, 6, MB, ZP>(a, plan, stream);
         default: return hipErrorInvalidValue;
         }
     };
     using std::integral_constant;
     auto with_mb = [&](auto zp) -> hipError_t {
-        return mb <= 2 ? with_t(integral_constant<int, 2>{}, zp) : mb == 3 ? with_t(integral_constant<int, 3>{}, zp) : with_t(integral_constant<int, 4>{}, zp);
+        return plan.row_blocks == 2   ? with_t(integral_constant<int, 2>{}, zp)
+               : plan.row_blocks == 3 ? with_t(integral_constant<int, 3>{}, zp)
+                                      : with_t(integral_constant<int, 4>{}, zp);
     };
     return a.w_zero ? with_mb(std::true_type{}) : with_mb(std::false_type{});
 }

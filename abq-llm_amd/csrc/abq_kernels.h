@@ -107,25 +107,6 @@ inline int decode_grouped_tiled_waves(int K, int w_bits, int group_size)
     return (nblocks + per_wave - 1) / per_wave;
 }
 
-// Kernel for 17 rows and more with group scales on K-tiled operands (abq_gemm_rows_grouped.hip): what it runs.  Its byte
-// offsets are 32 bits wide.
-inline bool rows_grouped_runs(int M, int N, int K, int x_bits, int w_bits, int group_size, int act)
-{
-    return M > 16 && x_bits == 8 && (w_bits == 2 || w_bits == 4 || w_bits == 8) && group_size == 128 && K >= 128 && (!act || N % 32 == 0) &&
-           (size_t)N * K * w_bits / 8 < (1ull << 32) && (size_t)M * K < (1ull << 32) && (size_t)N * (K / 128) * 4 < (1ull << 32);
-}
-// Whether its workgroups, one tile of 16 weight rows and up to 64 rows each at the least, cover most of the 256 compute
-// units (W4A8: 2048 x 2048 at 32 rows, 128 workgroups, 4.1 us against 4.0 on the decode kernel's blocks of rows; at 80
-// rows, 256, 4.7 against 6.4 on the prefill tiles; 1024 x 1024 at 128 rows, 128, 4.8 against 4.2, at 192 rows, 192, 4.9 against 7.5).
-inline bool rows_grouped_covers(int M, int N) { return (long)((N + 15) / 16) * ((M + 63) / 64) >= 192; }
-hipError_t launch_rows_grouped_8_2(const GemmArgs &, hipStream_t);
-hipError_t launch_rows_grouped_8_4(const GemmArgs &, hipStream_t);
-hipError_t launch_rows_grouped_8_8(const GemmArgs &, hipStream_t);
-template <int P> inline hipError_t launch_rows_grouped_8(const GemmArgs &a, hipStream_t stream)
-{
-    return P == 2 ? launch_rows_grouped_8_2(a, stream) : P == 4 ? launch_rows_grouped_8_4(a, stream) : launch_rows_grouped_8_8(a, stream);
-}
-
 // Workgroup id -> output tile.  XCD x = id % 8 owns n blocks [x * npx, (x + 1) * npx); inside an XCD the
 // workgroups run through groups of four m blocks, M fastest inside a group, then N, then the next group:
 // the 32 or 64 workgroups an XCD runs at a time then cover a patch of 4 x 8 (or 4 x 16) tiles, so every

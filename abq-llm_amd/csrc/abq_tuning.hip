@@ -11,7 +11,7 @@
 // One line per entry, '#' starts a comment:
 //     <kernel name> <M> <N> <K> <group size> <TOPS>
 // The kernel name carries bit widths, signedness and the tile tuple (abq_parse_kernel_name); the tuple says which
-// operand layout the tile runs on (NSTAGE 5: FP6 records; NSTAGE 4 and 6: K-tiled; else planes).  An entry serves
+// operand layout the tile runs on (NSTAGE 5: FP6 records; NSTAGE 4, 6 and 7: K-tiled; else planes).  An entry serves
 // the M of its bucket (1, 2, 3-4, 5-8, 9-16, 17-32, 33-64, ...) on exactly its N, K and group size.  A file may hold
 // several entries per shape, e.g. the best tile of each layout: a lookup takes the fastest among those the caller
 // can run.
@@ -106,9 +106,27 @@ int tile_operand_layout(const abq_tile_config &c)
 {
     if (c.mma_m == 32 && c.mma_n == 32 && c.mma_k == 64)
         return ABQ_LAYOUT_FP6;
-    if ((c.mma_m == 32 && c.mma_k == 32 && c.nstage == 4) || (c.mma_m == 16 && c.mma_k == 64 && c.nstage == 6))
+    if ((c.mma_m == 32 && c.mma_k == 32 && c.nstage == 4) || (c.mma_m == 16 && c.mma_k == 64 && (c.nstage == 6 || c.nstage == 7)))
         return ABQ_LAYOUT_TILED;
     return ABQ_LAYOUT_PLANES;
+}
+
+bool tuning_measured(int x_bits, int w_bits, int is_signed, int M, int N, int K, int group, int nstage)
+{
+    std::lock_guard<std::mutex> lock(g_mutex);
+    auto in = [&](const std::vector<TunedTile> &table) {
+        for (const TunedTile &t : table)
+            if (t.cfg.x_bits == x_bits && t.cfg.w_bits == w_bits && (t.cfg.is_signed != 0) == (is_signed != 0) && t.N == N && t.K == K &&
+                t.group_size == group && m_bucket(t.M) == m_bucket(M) && t.cfg.nstage == nstage)
+                return true;
+        return false;
+    };
+    if (in(g_loaded))
+        return true;
+    if (!g_builtin_enabled)
+        return false;
+    parse_builtin_locked();
+    return in(g_builtin);
 }
 
 bool tuning_find(int x_bits, int w_bits, int is_signed, int M, int N, int K, int group, int layout_mask, TunedTile *out)

@@ -250,11 +250,15 @@ int sweep_group_scales(int M, int N, int K, int x_bits, int w_bits, bool is_sign
     double best_tops = 0;
     std::string best;
     const int ncfg = abq_native_config_count(x_bits, w_bits, is_signed);
-    for (int i = 0; i <= ncfg; ++i) {
+    for (int i = 0; i <= ncfg + 1; ++i) { // (+ the kernel for 17 rows and more, which carries group scales only)
         abq_tile_config cfg;
-        const bool library_default = i == ncfg;
+        const bool library_default = i == ncfg + 1;
         if (!library_default) {
-            if (abq_native_config_get(x_bits, w_bits, is_signed, i, &cfg) != ABQ_OK || cfg.nstage != (fp6 ? 5 : 4) || cfg.warp_k != 128)
+            if (i == ncfg)
+                cfg = abq_tile_config{ x_bits, w_bits, 1, 64, 16, 4096, 64, 16, 512, 16, 16, 64, 7 };
+            else if (abq_native_config_get(x_bits, w_bits, is_signed, i, &cfg) != ABQ_OK || cfg.nstage != (fp6 ? 5 : 4) || cfg.warp_k != 128)
+                continue;
+            if (i == ncfg && (fp6 || !is_signed))
                 continue;
             char name[160];
             abq_format_kernel_name(&cfg, 0, name, sizeof name);

@@ -82,7 +82,10 @@ abq_status abq_pack_f16(const void *in_f16, const float *scale_dev, uint32_t *pl
  *   16 x 16 x 64  planes re-assembled to int8 in registers, v_mfma_i32_16x16x64_i8
  *                 (NSTAGE = 3: decode kernel, activations staged in LDS; NSTAGE = 2: every wave
  *                 expands its own activations; NSTAGE = 6: decode kernel on K-tiled operands,
- *                 BN / 16 weight tiles per workgroup, WK = K elements a wave keeps in flight)
+ *                 BN / 16 weight tiles per workgroup, WK = K elements a wave keeps in flight; NSTAGE = 7,
+ *                 64x16x4096_64x16x512: kernel for 17 rows and more on K-tiled operands with group scales
+ *                 of 128 and signed 8-bit activations; the state runs once abq_gemm_set_scales has been
+ *                 called.  Not part of the native tile space below, whose tiles run without group scales)
  *   32 x 32 x 32  the same feeding v_mfma_i32_32x32x32_i8 (NSTAGE = 4: LDS-staged kernels on K-tiled
  *                 operands, WK = 128 (or 64) = K elements per LDS stage and group of waves; BK = 2 WK:
  *                 two groups of waves share the tile and split K between them, for small grids; BK = 4 WK:
@@ -182,7 +185,9 @@ typedef struct abq_gemm_state {
     int group_size;        /* 0 = per channel          */
     int reserved[5];       /* [0] popcount kernels: log2 of the lanes per weight row; [1] see
                               abq_gemm_set_dynamic_f16_activations; [2], [3] see abq_gemm_set_value_bits; [4] bits 0, 1 see
-                              abq_gemm_set_biased_records, bit 2 abq_gemm_set_padded_activations */
+                              abq_gemm_set_biased_records, bit 2 abq_gemm_set_padded_activations, bit 4: the NSTAGE 7 kernel
+                              runs (cfg is then that of the tile it stands in for, or its own if asked for;
+                              grid_dim, block_dim and shared_mem_size are its own) */
     /* K-tiled operands (ABQ_STRATEGY_TILED) */
     int x_layout, w_layout;  /* abq_layout of X and W as handed to init                    */
     int auto_chosen;         /* 1 if the tile was the library's choice                     */

@@ -59,3 +59,48 @@ def test_unsigned_8_bit_operands_take_four_k_groups_once_their_row_sums_are_ther
     assert asked["launches"][0]["kernel"] == plain  # (the same integers without the sums)
     for r in (from_planes, mixed):
         assert r["status"] == 0 and staged64(r["launches"][-1]["kernel"]) == (8, 4, False, 4) and r["tile"] == tile64(8, 4, 0, 4), r
+
+
+ROWS = "AqBMMA_8x%dxtrue_64x16x4096_64x16x512_16x16x64_7"
+
+
+def rows_kernel(r):
+    return r["launches"][-1]["kernel"].startswith("gemm_rows_grouped<")
+
+
+@pytest.mark.parametrize("order", [["layouts", "scales", "zeros", "act"], ["scales", "layouts", "act", "zeros"], ["scales", "zeros", "act", "layouts"]])
+def test_states_of_17_rows_and_more_describe_the_kernel_that_runs(tmp_path, order):
+    shapes = [(8, 4, 43, 4096, 4096), (8, 4, 43, 12288, 4096), (8, 4, 43, 22016, 4096), (8, 2, 128, 4096, 4096), (8, 2, 32, 4096, 11008),
+              (8, 8, 96, 4096, 4096), (8, 2, 17, 4096, 1024)]
+    calls = [dict(q=q, p=p, signed=1, M=m, N=n, K=k, group=128, zeros=z, act=act, order=order)
+             for q, p, m, n, k in shapes for z in (0, 1) for act in (0, 1)]
+    for c, r in zip(calls, launches(tmp_path, calls)):
+        assert rows_kernel(r) and runs_what_it_says(r), (c, r)
+
+
+@pytest.mark.parametrize("p,m,n", [(2, 128, 4096), (4, 43, 4096), (8, 64, 4096), (4, 64, 12288)])
+def test_a_measured_tile_replaces_the_kernel_for_17_rows_only_where_that_was_measured_too(tmp_path, p, m, n):
+    k = 4096
+    tile = "AqBMMA_8x%dxtrue_128x64x128_64x32x128_32x32x32_4" % p
+    entry = lambda name, tops, group=128: "%s %d %d %d %d %s" % (name, m, n, k, group, tops)  # noqa: E731
+    rows = ROWS % p
+    by_rule, tile_only, tile_ahead, rows_ahead, no_group = launches(tmp_path, [
+        dict(q=8, p=p, signed=1, M=m, N=n, K=k, group=128, tuning=t)
+        for t in ([], [entry(tile, 500)], [entry(tile, 500), entry(rows, 400)], [entry(rows, 500), entry(tile, 400)])] +
+        [dict(q=8, p=p, signed=1, M=m, N=n, K=k, tuning=[entry(rows, 900, 0)])])
+    assert rows_kernel(by_rule) == (n == 4096)
+    assert rows_kernel(tile_only) == rows_kernel(by_rule)
+    assert rows_kernel(rows_ahead) and runs_what_it_says(rows_ahead)
+    assert not rows_kernel(tile_ahead) and tile_ahead["tile"] == tile and runs_what_it_says(tile_ahead)
+    assert no_group["status"] == 0 and not rows_kernel(no_group)  # (the entry names a kernel that needs group scales)
+
+
+def test_the_kernel_for_17_rows_runs_by_its_name(tmp_path):
+    ask = lambda p=4, **c: dict(dict(q=8, p=p, signed=1, M=300, N=4096, K=512, tile=ROWS % p, group=128), **c)  # noqa: E731
+    calls = [ask(p, M=m, zeros=z) for p in (2, 4, 8) for m in (17, 300) for z in (0, 1)]
+    for c, r in zip(calls, launches(tmp_path, calls)):
+        assert rows_kernel(r) and runs_what_it_says(r) and r["tile"] == c["tile"], (c, r)
+    # refused: 16 rows, groups of 64, no group scales, other pairs, another tuple
+    few, g64, bare, pair, other = launches(tmp_path, [ask(M=16), ask(group=64), ask(group=0), ask(tile="AqBMMA_4x4xtrue" + ROWS[len("AqBMMA_8x%dxtrue"):], q=4),
+                                                      ask(tile=(ROWS % 4).replace("64x16x4096", "64x32x4096").replace("64x16x512", "64x32x512"))])
+    assert [r["status"] for r in (few, g64, pair, other)] == [3, 3, 3, 3] and bare["status"] == 4 and not bare["launches"]
