@@ -13,16 +13,19 @@
 //
 // What bounds it: launch, one cold memory round trip and the stream of weights, scales and zero points (4 to 34 MB), so
 // everything of a wave is requested before its first wait, and no wave waits for another before the final sum:
-//   * a wave owns blocks of four K tiles (block b of K goes to wave b mod NW) for T tiles of 16 weight rows.  Every
+//   * a wave owns blocks of S = four K tiles (block b of K goes to wave b mod NW) for T tiles of 16 weight rows.  Every
 //     record of the activations, every scale and zero point is then used by exactly one wave of the workgroup, which
 //     brings it in for itself.  (Staging the rows in LDS for the whole workgroup kept 16 rows x 4096 to one workgroup per
 //     compute unit, split 16 rows x 11008 over two workgroups that each streamed the weights, and put a barrier in front
 //     of the first product.)
 //   * the four steps of a block times sixteen rows are the 64 dwords of one DMA instruction: a tile's scales cost one
 //     instruction per block.
+//   * below K = 4096 the blocks are of one to three K tiles, so that there are still up to eight waves (blocks of four throughout
+//     left one or two: W2A8 16 x 8192 x 512 5.3 -> 3.3 us, 1 x 1024 x 512 2.5 -> 2.1, 16 x 8192 x 3072 5.4 -> 4.8).
 //   * T is chosen so that the workgroups make one round of the compute units where the rows are worth it
-//     (decode_grouped_tiles): sixteen rows of activations cost a workgroup more L2 traffic than one tile's weights.
-//   * B = 2: the steps of two blocks in one unrolled round (long K).
+//     (dtg_pick_tiles): sixteen rows of activations cost a workgroup more L2 traffic than one tile's weights.
+//   * B = 2: the steps of two blocks in one unrolled round (long K); a wave's odd last block is a round of its own (as the first
+//     half of a round of two, its other half repeating the last loads, W8A8 8192 x 11008 took 25.6 us instead of 20.1).
 //   * the waves' partial tiles meet in LDS and are added in the order of the waves: which blocks a wave owns depends on
 //     K alone, so every variant below gives the same bits.
 #include <type_traits>
@@ -47,11 +50,13 @@ constexpr int dtg_threads(int p, int t, int b, int xm, bool g64)
 // flight: a compute unit's loads are served in order, and a wave that issues everything first stands at its last loads
 // until the stream has come that far, with the quantisation and the products waiting behind (22016 x 4096 at one token,
 // six tiles: half the kernel).
-// (x: bytes of activations a lane loads per step, 0 where they are quantised here)
-constexpr int dtg_ahead(int p, int t, int b, int x)
+// x: bytes of activations a lane loads per step, 0 where they are quantised here.  steps: of a round; all of them where that many
+// may be in flight, so that no request waits for the first loads to land, but one fewer where the quantisation stands in
+// between (one token through eight layers 222 us with all of them, 208 with one fewer).
+constexpr int dtg_ahead(int p, int t, int steps, int x)
 {
-    const int d = (x ? 44 : 24) / (t * p + x);
-    return d < 1 ? 1 : d > 4 * b - 1 ? 4 * b - 1 : d;
+    const int d = (x ? 44 : 24) / (t * p + x), most = (x && steps < 4) || steps == 1 ? steps : steps - 1;
+    return d < 1 ? 1 : d > most ? most : d;
 }
 
 // XM: how the activations arrive.
@@ -70,7 +75,7 @@ constexpr int dtg_ahead(int p, int t, int b, int x)
 // G64: groups of 64, two to a K tile: lane groups 0, 1 hold the elements of the first, 2, 3 those of the second, and the
 // matrix core sums over all four, so a step runs its two instructions twice: once on all lanes and once with the
 // activations of lane groups 2, 3 zeroed; the difference is the second group's dot product.
-template <int Q, int P, bool SIGNED, int T, int B, int XM, int XL, int FE, bool G64>
+template <int Q, int P, bool SIGNED, int T, int B, int S, int XM, int XL, int FE, bool G64>
 __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_tiled_grouped(const GemmArgs a)
 {
     static_assert(!XM || (Q == 8 && SIGNED && !G64), "in-kernel quantisation writes signed 8-bit records, groups of 128");
@@ -78,7 +83,8 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
     constexpr int LPS = DtgShare<P>::kLoads;       // weight loads per step and tile
     constexpr bool XS = XM == 0;
     constexpr int LPX = XS ? XL : 0;               // activation loads per step
-    constexpr int SC = 64 * GPT;                   // floats of a tile's scales per block: [GPT][16 rows][4 groups]
+    constexpr int SL = (S * GPT + 3) / 4;          // scale loads per block and tile
+    constexpr int SC = 64 * SL;                    // floats of a tile's scales per block: [SL][16 rows][4 groups]
     constexpr int XB = XS ? Q * 256 : 0;           // XS: bytes of sixteen rows' records of a step
     extern __shared__ __align__(16) unsigned char smem[];
 
@@ -90,7 +96,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
     const int M = a.M, N = a.N;
     const int KT = a.K >> 7; // K tiles = steps
     const int NG = KT * GPT; // scale groups along K
-    const int nblocks = (KT + 3) >> 2;
+    const int nblocks = (KT + S - 1) / S;
     const int tile0 = blockIdx.x * T;
     const int rows = min(M, 16);
     const int m0 = blockIdx.y * 16;
@@ -101,13 +107,13 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
     // LDS: [wave][tile][row][16] partial results | per wave: scales, zero points, group sums of its blocks in flight
     // (and its int8 records) | the rows' scales and zero points, the tiles' zero-point terms | extrema of rows quantised here
     const int blocks_of_wave = XM ? (nblocks + NW - 1) / NW : 0;
-    const unsigned own_bytes = B * (2 * T + 1) * SC * 4 + 2 * XB + (XM ? (unsigned)(blocks_of_wave * 4 * rows) * 128u : 0u);
+    const unsigned own_bytes = B * (2 * T + 1) * SC * 4 + 2 * XB + (XM ? (unsigned)(blocks_of_wave * S * rows) * 128u : 0u);
     float *red = reinterpret_cast<float *>(smem);
     unsigned char *own = smem + (unsigned)(NW * T * rows) * 64u + (unsigned)wid * own_bytes;
     float *sws = reinterpret_cast<float *>(own);           // [B][T][SC]
     float *zws = sws + B * T * SC;                         // [B][T][SC]
-    int *sxs = reinterpret_cast<int *>(zws + B * T * SC);  // [B][4 * GPT groups][16 rows]
-    unsigned char *xq = own + B * (2 * T + 1) * SC * 4;    // XM: [block of the wave][4][row][8 chunks], XS: [2][row][Q chunks]
+    int *sxs = reinterpret_cast<int *>(zws + B * T * SC);  // [B][4 * SL groups][16 rows]
+    unsigned char *xq = own + B * (2 * T + 1) * SC * 4;    // XM: [block of the wave][S][row][8 chunks], XS: [2][row][Q chunks]
     float *par = reinterpret_cast<float *>(smem + (unsigned)(NW * T * rows) * 64u + (unsigned)NW * own_bytes); // [2][64]: scales, zero points
     float *terms = par + 128;                              // [128]
     float *row_ext = terms + 128;                          // XM: [row][2][16 waves]
@@ -128,6 +134,9 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
     const char *Xt = reinterpret_cast<const char *>(a.X);
     const char *Wt = reinterpret_cast<const char *>(a.W);
     const bool row_zero = XM ? a.x_dynamic == 2 : a.x_zero != nullptr;
+    uint32_t zp_mask = zp ? ~0u : 0u;
+    if constexpr (XM != 0)
+        asm volatile("" : "+v"(zp_mask));
 
     float facc[T][FE];
 #pragma unroll
@@ -153,12 +162,13 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
     }
 
     const int upr = a.K >> 3; // XM: units of eight halves per row
-    int round = 0;
-    do {
-        if (round) // the scales of the last round have been read before new ones land on them
+    // One round: the next NB of the wave's blocks, `done` of them being behind it.
+    auto round = [&](int done, auto blocks_of_round) {
+        constexpr int NB = decltype(blocks_of_round)::value;
+        if (done) // the scales of the last round have been read before new ones land on them
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        constexpr int NS = 4 * B;                          // steps of a round
-        constexpr int D = dtg_ahead(P, T, B, 4 * LPX);              // steps whose weights are requested ahead of the one multiplied
+        constexpr int NS = S * NB;                         // steps of a round
+        constexpr int D = dtg_ahead(P, T, NS, 4 * LPX);    // steps whose weights are requested ahead of the one multiplied
         // A step's request is its weights and, in front of them, the next step's activations, so that those have landed
         // when the step's weights have.
         auto loads_of = [](int i) { return T * LPS + (i + 1 < NS ? LPX : 0); };
@@ -168,27 +178,30 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
                 n += loads_of(i);
             return n;
         };
-        DtgShare<P> wb[D + 1][T];
-        v4u xs[XS ? D + 2 : 1][XS ? XL : 1];
+        constexpr int WB = D + 1 < NS ? D + 1 : NS, XR = D + 2 < NS ? D + 2 : NS; // ring sizes
+        DtgShare<P> wb[WB][T];
+        v4u xs[XS ? XR : 1][XS ? XL : 1];
         constexpr int XH = XM == 1 || XM == 4 ? XM : 1;
-        v4u xr[XH][B];
-        auto block_of = [&](int b) { return (round * B + b) * NW + wid; };
+        v4u xr[XH][NB];
+        auto block_of = [&](int b) { return (done + b) * NW + wid; };
+        // XM: the lane's unit of a block (S < 4: the further lanes repeat the last one and write nothing)
+        auto unit_of = [&](int blk) { return min(blk * (16 * S) + (S == 4 ? lane : min(lane, 16 * S - 1)), upr - 1); };
 
         if constexpr (XM == 1 || XM == 4) {
-            // the wave's own units of the rows: unit 64 * block + lane (past the rows' end the last one once more)
+            // the wave's own units of the rows (past the rows' end the last one once more)
 #pragma unroll
             for (int m = 0; m < XH; ++m)
 #pragma unroll
-                for (int b = 0; b < B; ++b)
-                    xr[m][b] = dt_load16(Xt, (uint32_t)(min(m, Mb - 1) * upr + min(block_of(b) * 64 + lane, upr - 1)) * 16u);
+                for (int b = 0; b < NB; ++b)
+                    xr[m][b] = dt_load16(Xt, (uint32_t)(min(m, Mb - 1) * upr + unit_of(block_of(b))) * 16u);
         }
         // ---- scales, zero points and group sums of the blocks ----------------------------------------------------
 #pragma unroll
-        for (int b = 0; b < B; ++b)
+        for (int b = 0; b < NB; ++b)
 #pragma unroll
-            for (int i = 0; i < GPT; ++i) {
+            for (int i = 0; i < SL; ++i) {
                 // sixteen rows times four groups, neighbouring lanes on neighbouring groups: sixteen cache lines per instruction
-                const int first = 4 * GPT * block_of(b) + 4 * i;
+                const int first = S * GPT * block_of(b) + 4 * i;
                 const uint32_t grp = (uint32_t)min(first + (lane & 3), NG - 1);
 #pragma unroll
                 for (int t = 0; t < T; ++t) {
@@ -201,13 +214,13 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
                     lds_dma4(a.x_group_sums, (sumoff + (uint32_t)min(first + g, NG - 1)) * 4u, (unsigned)(size_t)(sxs + b * SC + i * 64));
             }
         // ---- a step's weights and the next one's activations (steps past the end of K repeat the last one) ---------------
-        auto k_tile = [&](int i) { return min(4 * block_of(i >> 2) + (i & 3), KT - 1); };
+        auto k_tile = [&](int i) { return min(S * block_of(i / S) + i % S, KT - 1); };
         auto request_acts = [&](int i) {
             const char *xp = Xt + (size_t)k_tile(i) * xstep;
             if constexpr (XS) {
-                xs[i % (D + 2)][0] = dt_load16(xp, xoff);
+                xs[i % XR][0] = dt_load16(xp, xoff);
                 if constexpr (XL > 1)
-                    xs[i % (D + 2)][1] = dt_load16(xp, xoff2);
+                    xs[i % XR][1] = dt_load16(xp, xoff2);
             }
         };
         auto request = [&](int i) {
@@ -216,7 +229,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
             const char *wp = Wt + (size_t)k_tile(i) * wstep;
 #pragma unroll
             for (int t = 0; t < T; ++t)
-                wb[i % (D + 1)][t].issue(wp, woff[t], once);
+                wb[i % WB][t].issue(wp, woff[t], once);
         };
         request_acts(0);
 #pragma unroll
@@ -224,7 +237,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
             request(i);
 
         if constexpr (XM != 0) {
-            if (XM == 8 ? round == 0 : true) {
+            if (XM == 8 ? done == 0 : true) {
                 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
                 auto dpp = [](float v, auto ctrl, auto row_mask) {
                     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v),
@@ -256,20 +269,20 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
                     return fmaxf((float)m.x, (float)m.y);
                 };
                 auto reload = [&](int m, int blk) {
-                    return *reinterpret_cast<const v4u *>(Xt + ((size_t)m * upr + min(blk * 64 + lane, upr - 1)) * 16u);
+                    return *reinterpret_cast<const v4u *>(Xt + ((size_t)m * upr + unit_of(blk)) * 16u);
                 };
                 const bool symmetric = a.x_dynamic == 1;
                 // symmetric: the maximum of |x| stands for both extrema; else the maxima of x and of -x
                 const uint32_t keep = symmetric ? 0x7FFF7FFFu : 0xFFFFFFFFu;
                 if constexpr (XM != 8) {
                     if (zp) // the halves are the oldest loads
-                        dt_wait_loads_n(loads_of_steps(0, D) + 2 * B * T);
+                        dt_wait_loads_n(loads_of_steps(0, D) + 2 * NB * SL * T);
                     else
-                        dt_wait_loads_n(loads_of_steps(0, D) + B * T);
+                        dt_wait_loads_n(loads_of_steps(0, D) + NB * SL * T);
 #pragma unroll
                     for (int m = 0; m < XH; ++m)
 #pragma unroll
-                        for (int b = 0; b < B; ++b)
+                        for (int b = 0; b < NB; ++b)
                             dt_landed(xr[m][b]);
                 }
                 auto extrema = [&](int m, auto unit, int count) {
@@ -295,7 +308,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
 #pragma unroll
                     for (int m = 0; m < XH; ++m)
                         if (m < Mb)
-                            extrema(m, [&](int b) { return xr[m][b]; }, B);
+                            extrema(m, [&](int b) { return xr[m][b]; }, NB);
                 }
                 __syncthreads();
                 uint32_t sel_pair, sel_half;
@@ -329,12 +342,15 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
                         for (int c = 0; c < 8; ++c)
                             v[c] = quant_code_bits((float)raw.h[c], qr);
                     }
-                    const uint32_t e_even = quad_transpose_bytes(pack_low_bytes(v[7], v[5], v[3], v[1]), sel_pair, sel_half);
-                    const uint32_t e_odd = quad_transpose_bytes(pack_low_bytes(v[6], v[4], v[2], v[0]), sel_pair, sel_half);
-                    const int rowi = (b * 4 + g) * rows + m;
+                    uint32_t e_even = quad_transpose_bytes(pack_low_bytes(v[7], v[5], v[3], v[1]), sel_pair, sel_half);
+                    uint32_t e_odd = quad_transpose_bytes(pack_low_bytes(v[6], v[4], v[2], v[0]), sel_pair, sel_half);
+                    if ((b * NW + wid) * (16 * S) + lane >= upr) // past the end of K
+                        e_even = e_odd = 0u;
+                    const int rowi = (b * S + g) * rows + m;
                     const int dw = 8 * ((lane >> 2) & 3) + 2 * (lane & 3); // first of the lane's two dwords in the record
                     const int chunk = (dw >> 2) ^ (rowi & 7);
-                    *reinterpret_cast<uint2 *>(xq + ((uint32_t)rowi * 8 + chunk) * 16u + (dw & 3) * 4u) = make_uint2(e_even, e_odd);
+                    if (S == 4 || g < S)
+                        *reinterpret_cast<uint2 *>(xq + ((uint32_t)rowi * 8 + chunk) * 16u + (dw & 3) * 4u) = make_uint2(e_even, e_odd);
                 };
                 if constexpr (XM == 8) {
                     for (int m = 0; m < Mb; ++m) {
@@ -348,7 +364,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
                         if (m < Mb) {
                             const QuantRow qr = params(m);
 #pragma unroll
-                            for (int b = 0; b < B; ++b)
+                            for (int b = 0; b < NB; ++b)
                                 quantise(m, b, xr[m][b], qr);
                         }
                 }
@@ -371,8 +387,9 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
             int sum[FE];              // XM
         };
         auto read_lds = [&](int i, Operands &s) {
-            const int b = i >> 2, d = i & 3;
-            const bool have = 4 * block_of(b) + d < KT; // (wave-uniform) steps past the end of K count nothing
+            const int b = i / S, d = i % S;
+            // (wave-uniform) steps past the end of K count nothing; rows quantised here have zero records there
+            const bool have = !XS || S * block_of(b) + d < KT;
 #pragma unroll
             for (int j = 0; j < GPT; ++j) {
                 const int at = (GPT * d + j) * 16, place = ((GPT * d + j) >> 2) * 64 + r * 4 + ((GPT * d + j) & 3);
@@ -380,7 +397,9 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
                 for (int t = 0; t < T; ++t) {
                     const float sw = sws[(b * T + t) * SC + place], zw = zws[(b * T + t) * SC + place];
                     s.sw[j][t] = have ? sw : 0.f;
-                    s.zw[j][t] = have && zp ? zw : 0.f;
+                    // (XM: by a mask; a select the compiler turns into a branch around the read, with a wait in it, which made one
+                    // token through eight layers 218 us instead of 209)
+                    s.zw[j][t] = XS ? (have && zp ? zw : 0.f) : __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, zw) & zp_mask);
                 }
                 if constexpr (XM == 0) {
                     if constexpr (FE == 1) {
@@ -395,7 +414,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
             }
             if constexpr (XS) {
                 // the records as they were loaded -> the wave's LDS, chunks of a row permuted -> the operand
-                auto &x = xs[i % (D + 2)];
+                auto &x = xs[i % XR];
                 unsigned char *buf = xq + (i & 1) * XB;
 #pragma unroll
                 for (int j = 0; j < XL; ++j) {
@@ -422,7 +441,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
                 }
             }
             if constexpr (XM != 0) {
-                const int rowi = ((XM == 8 ? round * B + b : b) * 4 + d) * rows + min(r, Mb - 1);
+                const int rowi = ((XM == 8 ? done + b : b) * S + d) * rows + min(r, Mb - 1);
                 const unsigned char *xrow = xq + (uint32_t)rowi * 128u;
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
@@ -447,7 +466,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 v4i bv[2];
-                dtg_operands<P, SIGNED>(wb[i % (D + 1)][t], bv);
+                dtg_operands<P, SIGNED>(wb[i % WB][t], bv);
                 v4i acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[0], bv[0], zero, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[1], bv[1], acc, 0, 0, 0);
                 if constexpr (G64) {
@@ -491,7 +510,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
             dt_wait_loads_n(loads_of_steps(i + 1, i + D < NS ? i + D + 1 : NS));
 #pragma unroll
             for (int t = 0; t < T; ++t)
-                wb[i % (D + 1)][t].landed();
+                wb[i % WB][t].landed();
             if (i + 1 < NS)
                 read_lds(i + 1, ops[(i + 1) % 3]);
             multiply(i, ops[i % 3], prod[i & 1]);
@@ -499,8 +518,18 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
                 fold(ops[(i - 1) % 3], prod[(i - 1) & 1]);
         }
         fold(ops[(NS - 1) % 3], prod[(NS - 1) & 1]);
-        ++round;
-    } while (XM != 1 && XM != 4 && round * B * NW < nblocks); // (rows held in registers: all blocks are in flight)
+    };
+    if constexpr (XM == 1 || XM == 4) {
+        round(0, std::integral_constant<int, B>{}); // (rows held in registers: all blocks are in flight)
+    } else {
+        // (block b of K is the wave's if b mod NW = wid; every wave has at least one)
+        int done = 0;
+        for (; (done + B - 1) * NW + wid < nblocks; done += B)
+            round(done, std::integral_constant<int, B>{});
+        if constexpr (B > 1) // the odd one (padded to a round of two, its repeated loads made W8A8 at K = 11008 a quarter slower)
+            if (done * NW + wid < nblocks)
+                round(done, std::integral_constant<int, 1>{});
+    }
 
     // ---- the waves' partial tiles meet in LDS, added in the order of the waves ---------------------------------------
 #pragma unroll
@@ -542,23 +571,26 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
 // ---- launch -------------------------------------------------------------------------------------------------------
 
 // LDS of a workgroup without what the quantising variants add
-static size_t dtg_lds(int nw, int t, int b, int rows, bool g64) { return (size_t)nw * t * rows * 64 + (size_t)nw * b * (2 * t + 1) * 256 * (g64 ? 2 : 1) + 1024; }
+static size_t dtg_lds(int nw, int t, int b, int s, int rows, bool g64)
+{
+    return (size_t)nw * t * rows * 64 + (size_t)nw * b * (2 * t + 1) * 256 * (g64 && s >= 3 ? 2 : 1) + 1024;
+}
 
 // instances that are built: what the registers hold
 constexpr bool dtg_built(int p, int t, int b, bool g64) { return t * b * p <= (g64 && p < 8 ? 8 : 16) && t * b <= 6 && !(g64 && b == 2 && t > 1); }
 
-template <int Q, int P, bool SIGNED, int T, int B, int XM, int XL, int FE, bool G64>
+template <int Q, int P, bool SIGNED, int T, int B, int S, int XM, int XL, int FE, bool G64>
 static hipError_t launch_dtg_instance(const GemmArgs &a, hipStream_t stream)
 {
     if constexpr (!dtg_built(P, T, B, G64)) {
         return hipErrorInvalidValue;
     } else {
         const int nw = decode_grouped_tiled_waves(a.K, P, a.group_size), rows = a.M < 16 ? a.M : 16;
-        const int nblocks = (a.K / 128 + 3) / 4;
-        size_t lds = dtg_lds(nw, T, B, rows, G64) + (!XM && XL ? (size_t)nw * 2 * Q * 256 : 0);
+        const int nblocks = (a.K / 128 + S - 1) / S;
+        size_t lds = dtg_lds(nw, T, B, S, rows, G64) + (!XM && XL ? (size_t)nw * 2 * Q * 256 : 0);
         if (XM)
-            lds += (size_t)nw * ((nblocks + nw - 1) / nw) * 4 * rows * 128 + (size_t)rows * 128;
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_decode_tiled_grouped<Q, P, SIGNED, T, B, XM, XL, FE, G64>),
+            lds += (size_t)nw * ((nblocks + nw - 1) / nw) * S * rows * 128 + (size_t)rows * 128;
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_decode_tiled_grouped<Q, P, SIGNED, T, B, S, XM, XL, FE, G64>),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (attr != hipSuccess)
             return attr;
@@ -566,28 +598,42 @@ static hipError_t launch_dtg_instance(const GemmArgs &a, hipStream_t stream)
             return hipErrorInvalidValue;
         const int tiles = (a.N + 15) / 16;
         const dim3 grid((tiles + T - 1) / T, (a.M + 15) / 16);
-        hipLaunchKernelGGL((gemm_decode_tiled_grouped<Q, P, SIGNED, T, B, XM, XL, FE, G64>), grid, dim3(64 * nw), lds, stream, a);
+        hipLaunchKernelGGL((gemm_decode_tiled_grouped<Q, P, SIGNED, T, B, S, XM, XL, FE, G64>), grid, dim3(64 * nw), lds, stream, a);
         return hipGetLastError();
     }
 }
 
 // Tiles per workgroup, or 0 if the shape has no instance with b blocks in flight.  Up to eight packed rows the fewest:
 // several workgroups on a compute unit overlap each other's phases (W2A8 12288 x 4096 at four rows 5.9 us on one tile, 6.3
-// on two; gate + up at eight rows 9.4 on two, 10.0 on six).  With more rows, or rows that every workgroup quantises for
-// itself, the fewest that make one round of the 256 compute units: 12288 x 4096 at sixteen rows 8.1 us on one tile, 6.9
-// on three; at one fp16 row 7.2 on one, 5.8 on three; gate + up at one fp16 row 9.3 on two, 8.2 on six.
-template <int P> static int dtg_pick_tiles(const GemmArgs &a, int xm, bool g64, int b)
+// on two; gate + up at eight rows 9.4 on two, 10.0 on six).  Rows that every workgroup quantises for itself: the fewest that
+// make one round of the 256 compute units (12288 x 4096 at one fp16 row 7.2 us on one, 5.8 on three; gate + up 9.3 on two, 8.2
+// on six).  More than eight packed rows: by what the rounds move (12288 x 4096 at sixteen rows 8.1 us on one tile, 6.9 on three).  Workgroups of a few
+// waves share a compute unit whatever their rows are (K < 1024: 16 x 8192 x 512 3.5 us on two tiles, 3.1 on one), those of
+// nine waves and more (long K, more than 256 tiles) have one to themselves and take two tiles at any number of rows.
+template <int P> static int dtg_pick_tiles(const GemmArgs &a, int q, int xm, bool g64, int b)
 {
     const int tiles = (a.N + 15) / 16, nw = decode_grouped_tiled_waves(a.K, P, a.group_size), rows = a.M < 16 ? a.M : 16;
+    const int one_round = !xm && decode_grouped_tiled_steps(a.K) == 1 && nw < 8 ? (nw > 2 ? 512 : 1024) : 256;
     const int choices[5] = { 1, 2, 3, 4, 6 };
     int best = 0;
+    long best_cost = 0;
     for (int c : choices) {
         // (a single row and the variants that hold several rows have instances of one and two tiles, unless they quantise)
-        if (!dtg_built(P, c, b, g64) || (a.act && (c & 1)) || dtg_lds(nw, c, b, rows, g64) > 120 * 1024 || 64 * nw > dtg_threads(P, c, b, xm, g64) ||
+        if (!dtg_built(P, c, b, g64) || (a.act && (c & 1)) || dtg_lds(nw, c, b, 4, rows, g64) > 120 * 1024 || 64 * nw > dtg_threads(P, c, b, xm, g64) ||
             (xm >= 4 && c > 2) || (xm == 8 && b > 1))
             continue;
+        const int rounds = ((tiles + c - 1) / c + one_round - 1) / one_round;
+        if (!xm && a.M > 8) {
+            // weights from memory, activations from L2, which is about three times as fast
+            const long cost = (long)rounds * (3 * c * P * 256 + rows * q * 16);
+            if (best == 0 || cost <= best_cost) {
+                best = c;
+                best_cost = cost;
+            }
+            continue;
+        }
         best = c;
-        if ((!xm && a.M <= 8) || (tiles + c - 1) / c <= 256)
+        if ((!xm && !(nw > 8 && b == 1 && c == 1)) || rounds == 1)
             break;
     }
     return best;
@@ -595,7 +641,8 @@ template <int P> static int dtg_pick_tiles(const GemmArgs &a, int xm, bool g64, 
 
 template <int Q, int P, bool SIGNED, bool XDYN, bool G64> static hipError_t launch_dtg(const GemmArgs &a, hipStream_t stream)
 {
-    const int nblocks = (a.K / 128 + 3) / 4, nw = decode_grouped_tiled_waves(a.K, P, a.group_size);
+    const int steps = decode_grouped_tiled_steps(a.K);
+    const int nblocks = (a.K / 128 + steps - 1) / steps, nw = decode_grouped_tiled_waves(a.K, P, a.group_size);
     const int per_wave = (nblocks + nw - 1) / nw;
     // two blocks of a wave in flight where it has two and there is an instance, else one after the other; rows held in
     // registers need all of a wave's blocks in flight
@@ -603,40 +650,52 @@ template <int Q, int P, bool SIGNED, bool XDYN, bool G64> static hipError_t laun
     int xm = !XDYN ? 0 : per_wave > 2 || a.M > 4 ? 8 : a.M > 1 ? 4 : 1;
     if (xm == 8)
         b = 1;
-    int t = dtg_pick_tiles<P>(a, xm, G64, b);
+    // Nor on more than two workgroups per compute unit, or more than one where the registers of two blocks (groups of 64) or
+    // their waves (more than eight) leave no room for a second workgroup beside the first: W2A8 at one row 5120 x 13824 9.9 ->
+    // 8.3 us on two tiles of one block, 8192 x 11008 9.4 -> 7.2, groups of 64 12288 x 5120 9.2 -> 7.0; at five rows 27648 x 5120
+    // 17.4 -> 13.7; at 16 rows of groups of 64 8192 x 11008 17.6 -> 12.8.
+    const int tiles = (a.N + 15) / 16;
+    if (!xm && (tiles > 512 || (tiles > 256 && (nw > 8 || G64))))
+        b = 1;
+    int t = dtg_pick_tiles<P>(a, Q, xm, G64, b);
     if (t == 0 && b == 2) {
         b = 1;
         if (XDYN)
             xm = 8;
-        t = dtg_pick_tiles<P>(a, xm, G64, b);
+        t = dtg_pick_tiles<P>(a, Q, xm, G64, b);
     }
-    auto go = [&](auto tt, auto bb) -> hipError_t {
-        constexpr int TT = decltype(tt)::value, BB = decltype(bb)::value;
+    auto go = [&](auto tt, auto bb, auto ss) -> hipError_t {
+        constexpr int TT = decltype(tt)::value, BB = decltype(bb)::value, SS = decltype(ss)::value;
         if constexpr (XDYN) {
             if (xm == 1)
-                return launch_dtg_instance<Q, P, SIGNED, TT, BB, 1, 0, 1, false>(a, stream);
+                return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 1, 0, 1, false>(a, stream);
             if constexpr (TT <= 2) {
                 if (xm == 4)
-                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, 4, 0, 4, false>(a, stream);
+                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 4, 0, 4, false>(a, stream);
                 if constexpr (BB == 1)
-                    return launch_dtg_instance<Q, P, SIGNED, TT, 1, 8, 0, 4, false>(a, stream);
+                    return launch_dtg_instance<Q, P, SIGNED, TT, 1, SS, 8, 0, 4, false>(a, stream);
             }
             return hipErrorInvalidValue;
         } else {
             if (a.M == 1) {
                 if constexpr (TT <= 2)
-                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, 0, 1, 1, G64>(a, stream);
+                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 1, 1, G64>(a, stream);
                 return hipErrorInvalidValue;
             }
             if constexpr (Q == 8) {
                 if (a.M > 8)
-                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, 0, 2, 4, G64>(a, stream);
+                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 2, 4, G64>(a, stream);
             }
-            return launch_dtg_instance<Q, P, SIGNED, TT, BB, 0, 1, 4, G64>(a, stream);
+            return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 1, 4, G64>(a, stream);
         }
     };
     using std::integral_constant;
-    auto with_b = [&](auto tt) -> hipError_t { return b == 2 ? go(tt, integral_constant<int, 2>{}) : go(tt, integral_constant<int, 1>{}); };
+    auto with_b = [&](auto tt) -> hipError_t {
+        constexpr integral_constant<int, 1> one{};
+        if (steps < 4) // (a wave then has one block)
+            return steps == 1 ? go(tt, one, one) : steps == 2 ? go(tt, one, integral_constant<int, 2>{}) : go(tt, one, integral_constant<int, 3>{});
+        return b == 2 ? go(tt, integral_constant<int, 2>{}, integral_constant<int, 4>{}) : go(tt, one, integral_constant<int, 4>{});
+    };
     switch (t) {
     case 1: return with_b(integral_constant<int, 1>{});
     case 2: return with_b(integral_constant<int, 2>{});

@@ -94,14 +94,19 @@ inline int decode_tiled_rows(int nw, int t, int M, int K, int q)
     return decode_tiled_lds(nw, t, mrows, K, q) <= 160 * 1024 ? mrows : 0;
 }
 
-// Decode kernel with group scales on K-tiled operands (abq_gemm_decode_tiled_grouped.hip): a wave owns blocks of four K
-// tiles, so the waves of a workgroup follow from K (and
-// the weights' width and group size): up to eight waves of one or two blocks, beyond that up to
-// sixteen, evened out (K = 4096: 8 waves of one block; 5120: 5 of two; 11008: 11 of two; 13824: 14 of two).  8-bit
-// weights and groups of 64 need the registers of an eight-wave workgroup.
+// Decode kernel with group scales on K-tiled operands (abq_gemm_decode_tiled_grouped.hip): a wave owns blocks of four K tiles,
+// below K = 4096 of one to three, so that there are still up to eight waves whose loads and products run beside each other.
+inline int decode_grouped_tiled_steps(int K)
+{
+    const int steps = (K / 128 + 7) / 8;
+    return steps < 4 ? steps : 4;
+}
+// The waves of a workgroup follow from K (and the weights' width and group size): up to eight waves of one or two blocks,
+// beyond that up to sixteen, evened out (K = 4096: 8 waves of one block; 5120: 5 of two; 11008: 11 of two; 13824: 14 of two).
+// 8-bit weights and groups of 64 need the registers of an eight-wave workgroup.
 inline int decode_grouped_tiled_waves(int K, int w_bits, int group_size)
 {
-    const int nblocks = (K / 128 + 3) / 4;
+    const int steps = decode_grouped_tiled_steps(K), nblocks = (K / 128 + steps - 1) / steps;
     const int most = nblocks <= 16 || w_bits == 8 || group_size == 64 ? 8 : 16;
     const int per_wave = (nblocks + most - 1) / most;
     return (nblocks + per_wave - 1) / per_wave;

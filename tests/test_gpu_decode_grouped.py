@@ -73,3 +73,29 @@ def test_rows_quantised_in_the_kernel(abq, oracle, p, symmetric, M, N, K, act):
     got = g.run()
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("q,p", [(8, 2), (8, 8), (4, 4), (2, 2)])
+@pytest.mark.parametrize("group", [128, 64])
+# blocks of two and three K tiles, the last one short; waves with an odd number of blocks, whose last is a round of its own (8-bit
+# weights and groups of 64: three and two blocks, three each); one tile and several per workgroup by the waves
+@pytest.mark.parametrize("M,N,K,act", [(9, 264, 1152, False), (16, 72, 2176, False), (5, 40, 2944, False), (16, 4128, 1408, True), (1, 24, 2048, False),
+                                       (8, 40, 8320, False), (16, 32, 9216, True), (3, 8208, 512, False), (16, 8216, 256, False), (12, 4112, 8576, False)])
+def test_short_blocks_and_odd_rounds(abq, oracle, q, p, group, M, N, K, act):
+    rng = np.random.default_rng(M + N + K + 10 * q + p)
+    xt, wt, kw, want = operands(abq, oracle, rng, M, N, K, q, p, group, act)
+    g = abq.Gemm(xt, wt, True, out_kind=abq.OUT_F16_SCALED, **kw)
+    assert g.strategy == "decode_tiled", g.strategy
+    print(q, p, group, M, N, K, act, flush=True)
+    got = g.run()
+    torch.cuda.synchronize()
+    assert_close_rel(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("p", [2, 8])
+# the same with rows quantised in the kernel: units of a block that is no whole wave, records past the end of K
+@pytest.mark.parametrize("M,N,K,act", [(1, 40, 128, False), (1, 12312, 1152, False), (3, 24, 2688, False), (4, 64, 1920, True), (16, 40, 896, False),
+                                       (1, 96, 8960, True)])
+def test_rows_quantised_in_short_blocks(abq, oracle, p, M, N, K, act):
+    test_rows_quantised_in_the_kernel(abq, oracle, p, False, M, N, K, act)
+    test_rows_quantised_in_the_kernel(abq, oracle, p, True, M, N, K, act)

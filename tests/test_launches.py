@@ -104,3 +104,13 @@ def test_the_kernel_for_17_rows_runs_by_its_name(tmp_path):
     few, g64, bare, pair, other = launches(tmp_path, [ask(M=16), ask(group=64), ask(group=0), ask(tile="AqBMMA_4x4xtrue" + ROWS[len("AqBMMA_8x%dxtrue"):], q=4),
                                                       ask(tile=(ROWS % 4).replace("64x16x4096", "64x32x4096").replace("64x16x512", "64x32x512"))])
     assert [r["status"] for r in (few, g64, pair, other)] == [3, 3, 3, 3] and bare["status"] == 4 and not bare["launches"]
+
+
+@pytest.mark.parametrize("p,group", [(2, 128), (8, 128), (4, 64)])
+def test_group_scale_decode_keeps_eight_waves_down_to_1024(tmp_path, p, group):
+    """Blocks of four K tiles throughout left one or two waves there.  Above, waves of two blocks; odd counts where no more waves fit."""
+    waves = {256: 2, 512: 4, 640: 5, 1024: 8, 1152: 5, 2048: 8, 2944: 8, 4096: 8, 5120: 5, 11008: 11 if p < 8 and group == 128 else 8}
+    calls = [dict(q=8, p=p, signed=1, M=m, N=4096, K=k, group=group, zeros=z) for k in waves for m in (1, 8, 16) for z in (0, 1)]
+    for c, r in zip(calls, launches(tmp_path, calls)):
+        (made,) = r["launches"]
+        assert made["kernel"].startswith("gemm_decode_tiled_grouped<") and made["block"] == [64 * waves[c["K"]], 1, 1], (c, made)
