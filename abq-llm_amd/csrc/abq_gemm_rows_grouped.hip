@@ -274,7 +274,11 @@ __global__ __launch_bounds__(64 * kRowsWaves) void gemm_rows_grouped(const GemmA
                 float f = v[e] * (1.0f / kShift);
                 if (row_zero)
                     f = __builtin_fmaf(-par[64 + mr + e], terms[tt * 16 + c], f);
-                v[e] = f * par[mr + e];
+                f *= par[mr + e];
+                // (rounded to fp32 here in every instance: in some of them the compiler would fuse this product into the conversion
+                // to fp16, and they would differ in a last place now and then)
+                asm("" : "+v"(f));
+                v[e] = f;
             }
             return v;
         };
