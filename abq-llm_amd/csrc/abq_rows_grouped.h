@@ -53,25 +53,29 @@ struct RowsPlan {
     int row_blocks; // of 16 rows per workgroup: 2 to 4
     int m_blocks;   // blocks of that many rows
     int waves;
+    int rounds; // of the compute units
     size_t lds;
     unsigned grid;
 };
 
-// A workgroup fills a compute unit's LDS, so workgroups run in rounds of 256; a round's time is the weights of its tiles from
-// memory plus the activations from L2, which is about three times as fast.
+// A workgroup fills a compute unit's LDS, so workgroups run in rounds of the 32 compute units of an XCD (the blocks of rows of a set
+// of weight rows share one: counted over all 256, 22 sets of eleven blocks passed for one round, but six XCDs had 33 to run); a
+// round's time is the weights of its tiles from memory plus the activations from L2, which is about three times as fast.
 inline RowsPlan rows_grouped_plan(int w_bits, int M, int N, int K, int act, bool zero_points)
 {
     const int m64 = (M + 63) / 64, mb16 = ((M + m64 - 1) / m64 + 15) / 16, mb = mb16 < 2 ? 2 : mb16;
     const int nw = (K / 128 + 3) / 4 < kRowsWaves ? (K / 128 + 3) / 4 : kRowsWaves;
     const long tiles = (N + 15) / 16;
-    RowsPlan plan{ 0, mb, (M + mb * 16 - 1) / (mb * 16), nw, 0, 0 };
+    RowsPlan plan{ 0, mb, (M + mb * 16 - 1) / (mb * 16), nw, 0, 0, 0 };
     double best_cost = 0;
     for (int c : { 1, 2, 3, 4, 6 }) {
         if (!rows_built(w_bits, c, mb) || (act && (c & 1)) || rows_lds(nw, w_bits, c, mb, zero_points) > 160 * 1024)
             continue;
-        const double cost = (double)(((tiles + c - 1) / c * m64 + 255) / 256) * (3.0 * c * (w_bits * 256 + 128) + mb * 2048.0);
+        const long per_xcd = ((tiles + c - 1) / c + 7) / 8 * plan.m_blocks, rounds = (per_xcd + 31) / 32;
+        const double cost = (double)rounds * (3.0 * c * (w_bits * 256 + 128) + mb * 2048.0);
         if (plan.tiles == 0 || cost < best_cost) {
             plan.tiles = c;
+            plan.rounds = (int)rounds;
             best_cost = cost;
         }
     }
