@@ -1194,6 +1194,7 @@ static abq_status switch_to_decode_tiled(abq_gemm_state *st, bool one_tile = fal
 // tiles.  It wins while its workgroups cover most of the compute units (rows_grouped_covers) and its work, counted in
 // 16 x 16 tiles of the result, stays below what the prefill tiles do in their fixed time (W4A8, zero points, us):
 //   4096 x 4096     43 rows (768 tiles)  7.9 against 13.4, 128 rows (2048) 10.1 against 13.2, 192 rows (3072) 14.4 against 13.4
+//   1024 x 4096     144 rows (576)  6.5 against 12.2, 256 rows (1024) 7.5 against 12.4, 512 rows (2048) 9.4 against 12.4
 //   4096 x 11008    43 rows 15.0 against 26.4, 128 rows 17.9 against 26.7
 //   12288 x 4096    32 rows (1536) 10.7 against 13.4, 43 rows (2304) 12.9 against 13.7, 64 rows (3072) 14.7 against 13.8
 //   15360 x 5120    43 rows (2880) 18.0 against 19.8
@@ -1206,6 +1207,15 @@ static bool rows_grouped_pays(int x_bits, int w_bits, int is_signed, int M, int 
     if (!is_signed || !rows_grouped_runs(M, N, K, x_bits, w_bits, group_size, act) || K < 1024 || !rows_grouped_covers(M, N))
         return false;
     const long tiles = (N + 15) / 16, work = tiles * ((M + 15) / 16);
+    // Measured up to 512 rows.  Above 128 only where the plan makes one round (700 x 1024 x 4096, two: 21.1 against 12.4), and on short
+    // K above 32 rows only with up to two tiles per workgroup: the tiles' time falls with K, the fold and the final sum do not
+    // (W4A8 512 x 1024 x 1024 6.5 against 7.1, but three tiles, 192 x 3072 x 1024, 9.1 against 7.6, 43 x 12288 x 1024 8.1
+    // against 7.7; K = 1536 8.2 against 9.1; up to 32 rows 32 x 12288 x 1024 6.8 against 7.4).
+    if (M > 512)
+        return false;
+    const RowsPlan plan = rows_grouped_plan(w_bits, M, N, K, act, true);
+    if ((M > 128 && plan.rounds > 1) || (M > 32 && K < (M > 128 ? 2048 : 1536) && plan.rounds * plan.tiles > 2))
+        return false;
     if (w_bits == 8)
         return work <= 2048 && tiles <= 512;
     return work <= 2900 || (tiles > 1024 && M <= 48 && work <= 4300);
@@ -1225,10 +1235,10 @@ static bool decode_tiled_grouped_pays(int x_bits, int w_bits, int M, int N, int 
         return true;
     // (4-bit weights: folded records would be twice as wide, and the kernel that streams the weights once runs on either
     // width: W4A8 with zero points, 43 x 22016 x 4096 19.8 us on 4-bit records, 34.5 on the folded ones)
-    if (w_bits == 4 && rows_grouped_pays(x_bits, w_bits, 1, M, N, K, group_size, act))
-        return true;
     if (M > 128)
         return false;
+    if (w_bits == 4 && rows_grouped_pays(x_bits, w_bits, 1, M, N, K, group_size, act))
+        return true;
     const int t = act ? 2 : 1;
     const int mrows = 16;
     const double blocks = (M + mrows - 1) / mrows;

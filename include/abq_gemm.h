@@ -330,9 +330,12 @@ int abq_fp6_eligible(int x_bits, int w_bits, int is_signed, int k);
 
 /* Whether a GEMM of this shape whose operands are both K-tiled runs ABQ_STRATEGY_DECODE_TILED when the tile is the
  * library's choice: always up to 16 rows where that kernel is built for the pair (and, with group scales, for
- * groups of 128), and up to 128 rows where the library estimates the kernel, run over blocks of 16 rows (from 17 rows on, with
- * 8-bit activations and groups of 128, a kernel that streams the weights once for up to 64 rows), ahead of the prefill kernel.  For callers that hold their weights in several prepared forms and have to pick one before
- * they quantise the activations (ABQGEMMWrapper::gemm_dynamic).  No counterpart in the reference. */
+ * groups of 64 and 128), and up to 128 rows where the library estimates the kernel, run over blocks of 16 rows, ahead of
+ * the prefill kernel (with 8-bit activations and groups of 128 the NSTAGE 7 kernel, which streams the weights once for up to
+ * 64 rows, takes the blocks' place where it covers the chip).  Never above 128 rows; the NSTAGE 7 kernel may still run there
+ * in a prefill tile's place, on whatever records the weights are held in.  For callers that hold their weights in
+ * several prepared forms and have to pick one before they quantise the activations (ABQGEMMWrapper::gemm_dynamic).  No
+ * counterpart in the reference. */
 int abq_prepared_decode_pays(int x_bits, int w_bits, int is_signed, int M, int N, int K, int group_size, int act);
 /* planes [bits][rows][k/32] -> fp6 [k/128][rows][24]; bits <= 4, or <= 5 if is_signed. */
 abq_status abq_relayout_planes_fp6(const uint32_t *planes, uint32_t *fp6, int rows, int k, int bits,

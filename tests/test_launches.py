@@ -114,3 +114,25 @@ def test_group_scale_decode_keeps_eight_waves_down_to_1024(tmp_path, p, group):
     for c, r in zip(calls, launches(tmp_path, calls)):
         (made,) = r["launches"]
         assert made["kernel"].startswith("gemm_decode_tiled_grouped<") and made["block"] == [64 * waves[c["K"]], 1, 1], (c, made)
+
+
+def test_the_plan_for_17_rows_counts_rounds_per_xcd(tmp_path):
+    """22 sets of three tiles by eleven blocks of rows are 242 workgroups, but six of the eight XCDs would run 33 on 32 compute units."""
+    (r,) = launches(tmp_path, [dict(q=8, p=4, signed=1, M=700, N=1024, K=4096, tile=ROWS % 4, group=128, zeros=1)])
+    assert r["launches"][0]["kernel"] == "gemm_rows_grouped<4, 4, 4, true>"
+
+
+def test_the_kernel_for_17_rows_is_bounded_in_rows(tmp_path):
+    shape = lambda m, n, k, p=4: dict(q=8, p=p, signed=1, M=m, N=n, K=k, group=128, zeros=1)  # noqa: E731
+    on = [shape(43, 4096, 4096), shape(128, 4096, 4096), shape(512, 1024, 4096), shape(32, 12288, 1024), shape(512, 1024, 1024)]
+    off = [shape(700, 1024, 4096), shape(1400, 512, 4096), shape(5000, 128, 4096), shape(192, 3072, 1024), shape(43, 12288, 1024), shape(513, 1024, 4096)]
+    for c, r in zip(on + off, launches(tmp_path, on + off)):
+        assert rows_kernel(r) == (c in on) and runs_what_it_says(r), (c, r)
+
+
+def test_no_decode_records_above_128_rows(abq):
+    for p in (2, 4, 8):
+        for n, k in ((128, 4096), (512, 4096), (1024, 4096), (4096, 4096), (4096, 11008)):
+            for m in (129, 200, 700, 1400, 5000):
+                assert not abq.prepared_decode_pays(8, p, True, m, n, k, 128)
+    assert abq.prepared_decode_pays(8, 4, True, 128, 4096, 4096, 128)
