@@ -1774,7 +1774,7 @@ abq_status abq_gemm_set_biased_records(abq_gemm_state *st, int x_biased, int w_b
         return ABQ_ERR_UNSUPPORTED;
     if (x_biased && !w_biased)
         return ABQ_ERR_INVALID_ARG;
-    st->reserved[4] = (x_biased ? 1 : 0) | (w_biased ? 2 : 0);
+    st->reserved[4] = (st->reserved[4] & ~3) | (x_biased ? 1 : 0) | (w_biased ? 2 : 0);
     if (w_biased && st->strategy == ABQ_STRATEGY_DECODE_TILED && st->auto_chosen)
         return switch_to_tiled(st); // biased records are read by the prefill kernel only
     return ABQ_OK;
@@ -2280,8 +2280,8 @@ abq_status abq_gemm_set_dynamic_f16_activations(abq_gemm_state *st, const void *
         return ABQ_ERR_INVALID_ARG;
     const abq_tile_config &c = st->cfg;
     const KernelTable *t = find_table(registry().decode_tiled_grouped_dyn, c.x_bits, c.w_bits, c.is_signed);
-    // a workgroup quantises all of its rows in registers: 16384 elements (the instance of eight waves; all rows of a
-    // call at most 16, which is what the decode kernel takes per workgroup without splitting M)
+    // a workgroup quantises all of its rows into its LDS: up to 16384 elements (up to four rows are held in registers on the way, more
+    // are read a second time); all rows of a call at most 16, what the decode kernel takes per workgroup
     if (st->strategy != ABQ_STRATEGY_DECODE_TILED || st->group_size != 128 || st->w_layout != ABQ_LAYOUT_TILED || !t || t->count == 0 ||
         st->variant != 0 || st->M > 16 || (size_t)st->M * st->K > 16384 || (st->x_zero && symmetric))
         return ABQ_ERR_UNSUPPORTED;

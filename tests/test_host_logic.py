@@ -801,3 +801,18 @@ def test_small_batches_with_plane_activations_reach_the_prepared_decode_kernel_o
         assert strategy(8, 2, 128, 11008, 4096, P, True) == "tiled" and strategy(8, 2, 300, 4096, 4096, P, True) == "tiled"
     finally:
         lib.abq_tuning_enable_builtin(1)
+
+
+def test_declaring_biased_records_leaves_the_other_declarations(abq):
+    """abq_gemm_set_biased_records sets its own two bits: padded activation records stay declared, and a group-scale state stays on
+    the kernel it runs."""
+    lib = abq.lib()
+    rc, st = _init(abq, q=3, p=2, M=4, signed=1, N=256, K=512)
+    assert rc == 0 and lib.abq_gemm_set_padded_activations(ctypes.byref(st), 1) == 0 and st.reserved[4] == 4
+    assert lib.abq_gemm_set_biased_records(ctypes.byref(st), 0, 0) == 0 and st.reserved[4] == 4
+    rc, st = _init(abq, q=8, p=4, M=43, signed=1, N=4096, K=4096, out_kind=abq.OUT_F16_SCALED)
+    T = abq.LAYOUT_TILED
+    assert rc == 0 and lib.abq_gemm_set_operand_layout(ctypes.byref(st), T, T) == 0
+    assert lib.abq_gemm_set_scales(ctypes.byref(st), 0x4000, 0x5000, 128) == 0
+    before = bytes(st)
+    assert lib.abq_gemm_set_biased_records(ctypes.byref(st), 0, 0) == 0 and bytes(st) == before
