@@ -1207,14 +1207,15 @@ static bool rows_grouped_pays(int x_bits, int w_bits, int is_signed, int M, int 
     if (!is_signed || !rows_grouped_runs(M, N, K, x_bits, w_bits, group_size, act) || K < 1024 || !rows_grouped_covers(M, N))
         return false;
     const long tiles = (N + 15) / 16, work = tiles * ((M + 15) / 16);
-    // Measured up to 512 rows.  Above 128 only where the plan makes one round (700 x 1024 x 4096, two: 21.1 against 12.4), and on short
+    // Measured up to 2048 rows, above 512 with up to two tiles per workgroup (1024 x 256 x 4096 7.9 against 12.6, 2048 x 128 x 1024 4.7
+    // against 7.2).  Above 128 only where the plan makes one round (700 x 1024 x 4096, two: 21.1 against 12.4), and on short
     // K above 32 rows only with up to two tiles per workgroup: the tiles' time falls with K, the fold and the final sum do not
     // (W4A8 512 x 1024 x 1024 6.5 against 7.1, but three tiles, 192 x 3072 x 1024, 9.1 against 7.6, 43 x 12288 x 1024 8.1
     // against 7.7; K = 1536 8.2 against 9.1; up to 32 rows 32 x 12288 x 1024 6.8 against 7.4).
-    if (M > 512)
+    if (M > 2048)
         return false;
     const RowsPlan plan = rows_grouped_plan(w_bits, M, N, K, act, true);
-    if ((M > 128 && plan.rounds > 1) || (M > 32 && K < (M > 128 ? 2048 : 1536) && plan.rounds * plan.tiles > 2))
+    if ((M > 512 && plan.tiles > 2) || (M > 128 && plan.rounds > 1) || (M > 32 && K < (M > 128 ? 2048 : 1536) && plan.rounds * plan.tiles > 2))
         return false;
     if (w_bits == 8)
         return work <= 2048 && tiles <= 512;

@@ -124,7 +124,8 @@ def test_the_plan_for_17_rows_counts_rounds_per_xcd(tmp_path):
 
 def test_the_kernel_for_17_rows_is_bounded_in_rows(tmp_path):
     shape = lambda m, n, k, p=4: dict(q=8, p=p, signed=1, M=m, N=n, K=k, group=128, zeros=1)  # noqa: E731
-    on = [shape(43, 4096, 4096), shape(128, 4096, 4096), shape(512, 1024, 4096), shape(32, 12288, 1024), shape(512, 1024, 1024)]
+    on = [shape(43, 4096, 4096), shape(128, 4096, 4096), shape(512, 1024, 4096), shape(32, 12288, 1024), shape(512, 1024, 1024), shape(1024, 256, 4096),
+          shape(2048, 128, 1024)]
     off = [shape(700, 1024, 4096), shape(1400, 512, 4096), shape(5000, 128, 4096), shape(192, 3072, 1024), shape(43, 12288, 1024), shape(513, 1024, 4096)]
     for c, r in zip(on + off, launches(tmp_path, on + off)):
         assert rows_kernel(r) == (c in on) and runs_what_it_says(r), (c, r)
