@@ -64,6 +64,55 @@ __global__ __launch_bounds__(256) void pack_i32_kernel(const int4 *__restrict__ 
     }
 }
 
+// The same for large inputs of narrow codes (a loader's weight matrices): a wave takes 2048 consecutive elements as eight
+// loads of 1 KiB, every lane 16 bytes next to its neighbour's, all in flight together.  A lane then holds four bits per load
+// and plane: a nibble; an 8 x 8 nibble transpose over each eight lanes makes whole words of them, which leave as 256
+// consecutive bytes per plane.
+// Bound by the read of the codes (16 times what a 2-bit operand writes): pack_i32_kernel's two loads of 16 bytes 32 bytes
+// apart fetched every line with two instructions, and kept the lines in the caches for a reader that never comes (12288 x 4096
+// into 2 bits, cold: 39.1 us there, 38.3 with this access pattern, 36.2 with it and non-temporal loads, as a kernel that
+// only reads; 22016 x 4096 72.0 -> 64.8, 4096 x 4096 13.6 -> 11.9).
+typedef int pack_quad __attribute__((ext_vector_type(4)));
+
+template <int BITS>
+__global__ __launch_bounds__(256) void pack_i32_lines_kernel(const pack_quad *__restrict__ in, uint32_t *__restrict__ planes,
+                                                             uint32_t n_quads)
+{
+    const int lane = threadIdx.x & 63;
+    const uint32_t plane_words = n_quads / 8, stride = gridDim.x * 4u * 512u;
+    for (uint32_t base = ((blockIdx.x * 256u + threadIdx.x) >> 6) * 512u; base < n_quads; base += stride) { // (wave-uniform)
+        pack_quad v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) // past the end: the last quad once more, into words that are not stored
+            v[j] = __builtin_nontemporal_load(in + min(base + 64u * j + lane, n_quads - 1u));
+        uint32_t codes[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            codes[j] = pack_low_bytes(v[j][3], v[j][2], v[j][1], v[j][0]); // the first element in the top byte
+#pragma unroll
+        for (int b = 0; b < BITS; ++b) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) { // load j's nibble, the first element on top, goes to nibble j from the top
+                uint32_t x = (codes[j] >> b) & 0x01010101u;
+                x = (x | (x >> 7)) & 0x00030003u;
+                x |= x >> 14;
+                w |= (x & 0xFu) << (28 - 4 * j);
+            }
+            // lane l of eight ends with nibble l of lanes 0 .. 7, lane 0's on top: its word is load l's, these eight lanes'
+            const uint32_t far = (uint32_t)__shfl_xor((int)w, 4);
+            w = (lane & 4) ? ((far << 16) | (w & 0x0000FFFFu)) : ((w & 0xFFFF0000u) | (far >> 16));
+            const uint32_t mid = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x4E, 0xF, 0xF, true); // lane ^ 2
+            w = (lane & 2) ? (((mid << 8) & 0xFF00FF00u) | (w & 0x00FF00FFu)) : ((w & 0xFF00FF00u) | ((mid >> 8) & 0x00FF00FFu));
+            const uint32_t near = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0xB1, 0xF, 0xF, true); // lane ^ 1
+            w = (lane & 1) ? (((near << 4) & 0xF0F0F0F0u) | (w & 0x0F0F0F0Fu)) : ((w & 0xF0F0F0F0u) | ((near >> 4) & 0x0F0F0F0Fu));
+            const uint32_t word = base / 8u + 8u * (lane & 7) + (lane >> 3);
+            if (word < plane_words)
+                planes[(size_t)b * plane_words + word] = w;
+        }
+    }
+}
+
 __global__ __launch_bounds__(256) void pack_f16_kernel(const uint4 *__restrict__ in,
                                                        const float *__restrict__ scale,
                                                        uint32_t *__restrict__ planes,
@@ -239,10 +288,12 @@ __global__ __launch_bounds__(256) void relayout_planes_kernel(const uint32_t *__
         if (row < rows && kt < kt_tiles) {
             uint32_t pw[4][BITS]; // [word-set][plane]
             const uint32_t *p = planes + (size_t)row * KW + 4 * kt;
+            uint4 v = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
             for (int b = 0; b < BITS; ++b) {
-                uint4 v = *reinterpret_cast<const uint4 *>(p + min(b, in_bits - 1) * plane_stride);
-                if (b >= in_bits && !(sign_extend & 1))
+                if (b < in_bits) // (the same in every lane; the top plane stays in v for those above it)
+                    v = *reinterpret_cast<const uint4 *>(p + b * plane_stride);
+                else if (!(sign_extend & 1))
                     v = make_uint4(0u, 0u, 0u, 0u);
                 pw[0][b] = v.x; pw[1][b] = v.y; pw[2][b] = v.z; pw[3][b] = v.w;
             }
@@ -1100,21 +1151,26 @@ hipError_t launch_quant_pack_rows(const void *x, uint32_t *planes, float *scale,
 
 // w_zero_term[n] = sum_g w_scale[n][g] * (sum of the weight codes of row n in group g
 //                                         - group_size * w_zero[n][g]);
-// one wave per weight row, lanes over the row's groups.
+// 2^lanes_log2 lanes per weight row (64, or the fewest that still take all groups of a row at once), lanes over the row's groups.
 // WIDE: groups of a multiple of 128, planes on 16-byte boundaries: a group's words in 16-byte loads, those of all planes in
-// flight together (22016 x 4096, 2 bits, groups of 128: 14.4 -> 12.8 us).
+// flight together with the scale and the zero point, and rows of 32 groups or fewer side by side in a wave: one trip to
+// memory per row is all the kernel does, so what counts is how many are under way (22016 x 4096, 2 bits, groups of 128:
+// 14.4 us word by word, 12.8 with a row per wave).
 template <bool WIDE>
 __global__ __launch_bounds__(256) void weight_zero_term_kernel(const uint32_t *__restrict__ planes, int N, int KW, int bits,
                                                                int is_signed, const float *__restrict__ w_scale,
                                                                const float *__restrict__ w_zero, int group_size,
-                                                               float *__restrict__ out)
+                                                               float *__restrict__ out, int lanes_log2)
 {
-    const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & ((1 << lanes_log2) - 1);
+    const int n = (int)(blockIdx.x * (256u >> lanes_log2) + (threadIdx.x >> lanes_log2));
     if (n >= N)
-        return; // whole waves leave; no barrier below
+        return; // whole rows' lanes leave; no barrier below
     const int wpg = group_size / 32, groups = KW / wpg;
     float t = 0.f;
-    for (int gi = lane; gi < groups; gi += 64) {
+    for (int gi = lane; gi < groups; gi += 1 << lanes_log2) {
+        const size_t idx = (size_t)n * groups + gi;
+        const float scale = w_scale[idx], zero = w_zero ? w_zero[idx] : 0.f;
         int sum = 0;
         if constexpr (WIDE) {
             for (int w = 0; w < wpg; w += 4) {
@@ -1138,11 +1194,9 @@ __global__ __launch_bounds__(256) void weight_zero_term_kernel(const uint32_t *_
                 sum += (is_signed && b == bits - 1) ? -(c << b) : (c << b);
             }
         }
-        const size_t idx = (size_t)n * groups + gi;
-        t += w_scale[idx] * ((float)sum - (float)group_size * (w_zero ? w_zero[idx] : 0.f));
+        t += scale * ((float)sum - (float)group_size * zero);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+    for (int o = 1 << lanes_log2 >> 1; o > 0; o >>= 1)
         t += __shfl_xor(t, o);
     if (lane == 0)
         out[n] = t;
@@ -1152,8 +1206,10 @@ hipError_t launch_weight_zero_term(const uint32_t *planes, int n, int k, int bit
                                    const float *w_zero, int group_size, float *out, hipStream_t stream)
 {
     const bool wide = bits <= 8 && group_size % 128 == 0 && (k / 32) % 4 == 0 && (reinterpret_cast<size_t>(planes) & 15) == 0;
-    hipLaunchKernelGGL(wide ? weight_zero_term_kernel<true> : weight_zero_term_kernel<false>, dim3((n + 3) / 4), dim3(256), 0, stream, planes, n,
-                       k / 32, bits, is_signed, w_scale, w_zero, group_size, out);
+    const int groups = k / group_size, lanes_log2 = groups <= 16 ? 4 : groups <= 32 ? 5 : 6;
+    const unsigned blocks = (unsigned)(((size_t)n + (256 >> lanes_log2) - 1) >> (8 - lanes_log2));
+    hipLaunchKernelGGL(wide ? weight_zero_term_kernel<true> : weight_zero_term_kernel<false>, dim3(blocks), dim3(256), 0, stream, planes, n,
+                       k / 32, bits, is_signed, w_scale, w_zero, group_size, out, lanes_log2);
     return hipGetLastError();
 }
 
@@ -1171,6 +1227,21 @@ hipError_t launch_pack_i32(const int32_t *in, uint32_t *planes, int rows, int k,
                            hipStream_t stream)
 {
     const size_t n_units = (size_t)rows * k / 8;
+    // Whole lines per load from 8 M elements on, where the kernel is bound by its read (grids of 4096 workgroups of at least
+    // one trip per wave); below, the waves of pack_i32_kernel have a quarter of the work each (128 x 5120: 3.5 us on either).
+    // Up to 4 bits: beyond, its arithmetic per plane would come close to the time of the loads.
+    if (bits >= 1 && bits <= 4 && n_units >= ((size_t)1 << 20) && n_units < ((size_t)1 << 30) && (reinterpret_cast<size_t>(in) & 15) == 0) {
+        const uint32_t quads = (uint32_t)(n_units * 2);
+        const dim3 grid(grid_for(n_units / 4));
+        const pack_quad *src = reinterpret_cast<const pack_quad *>(in);
+        switch (bits) {
+        case 1: hipLaunchKernelGGL(pack_i32_lines_kernel<1>, grid, dim3(256), 0, stream, src, planes, quads); break;
+        case 2: hipLaunchKernelGGL(pack_i32_lines_kernel<2>, grid, dim3(256), 0, stream, src, planes, quads); break;
+        case 3: hipLaunchKernelGGL(pack_i32_lines_kernel<3>, grid, dim3(256), 0, stream, src, planes, quads); break;
+        default: hipLaunchKernelGGL(pack_i32_lines_kernel<4>, grid, dim3(256), 0, stream, src, planes, quads); break;
+        }
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(pack_i32_kernel, dim3(grid_for(n_units)), dim3(256), 0, stream,
                        reinterpret_cast<const int4 *>(in), planes, n_units, bits);
     return hipGetLastError();
