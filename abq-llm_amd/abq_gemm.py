@@ -30,7 +30,7 @@ EXPORTED = [
     "abq_status_string", "abq_last_hip_error", "abq_version",
     "abq_pack_i32", "abq_pack_u4", "abq_pack_f16", "abq_pack_f16_tiled",
     "abq_parse_kernel_name", "abq_format_kernel_name",
-    "abq_native_config_count", "abq_native_config_get",
+    "abq_native_config_count", "abq_native_config_get", "abq_native_config_list",
     "abq_gemm_init", "abq_gemm_set_scales", "abq_gemm_exec", "abq_gemm_launch",
     "abq_planes_bytes", "abq_relayout_planes", "abq_gemm_set_operand_layout", "abq_gemm_workspace_bytes",
     "abq_gemm_set_workspace", "abq_fp6_bytes", "abq_fp6_eligible", "abq_prepared_decode_pays", "abq_gemm_set_dynamic_f16_activations", "abq_relayout_planes_fp6",
@@ -115,6 +115,8 @@ def lib():
         L.abq_native_config_count.argtypes = [ci, ci, ci]
         L.abq_native_config_count.restype = ci
         L.abq_native_config_get.argtypes = [ci, ci, ci, ci, ctypes.POINTER(TileConfig)]
+        L.abq_native_config_list.argtypes = [ci, ci, ci, ctypes.POINTER(TileConfig), ci]
+        L.abq_native_config_list.restype = ci
         L.abq_gemm_init.argtypes = [ctypes.POINTER(TileConfig), ci, ci, ci, vp, vp, ci, ci, ci, vp, vp, ci, ci,
                                     ctypes.POINTER(GemmState)]
         L.abq_gemm_set_scales.argtypes = [ctypes.POINTER(GemmState), vp, vp, ci]
@@ -176,7 +178,10 @@ def _check(status, what):
 def _stream_ptr(stream):
     if stream is None:
         import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        if not torch.cuda.is_initialized():
+            torch.cuda.init()
+        # (the pointer itself: building torch's Stream object around it takes as long as launching a kernel)
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
     if isinstance(stream, int):
         return ctypes.c_void_p(stream)
     return ctypes.c_void_p(stream.cuda_stream)
@@ -196,12 +201,8 @@ def format_kernel_name(cfg, is_wmma=False):
 
 def native_configs(x_bits, w_bits, signed):
     n = lib().abq_native_config_count(x_bits, w_bits, int(signed))
-    out = []
-    for i in range(n):
-        c = TileConfig()
-        _check(lib().abq_native_config_get(x_bits, w_bits, int(signed), i, ctypes.byref(c)), "abq_native_config_get")
-        out.append(c)
-    return out
+    out = (TileConfig * n)()
+    return list(out[:lib().abq_native_config_list(x_bits, w_bits, int(signed), out, n)])
 
 
 def planes_empty(bits, rows, k, device="cuda"):
@@ -306,6 +307,25 @@ def relayout_planes_padded(planes, signed, stream=None):
     return out
 
 
+def _host_flag():
+    """A zeroed int in pinned host memory, which a kernel can set where it stands: no fill before the kernel and no copy
+    behind it, each a launch of its own with the host waiting for it (a loader reads one such flag per weight matrix)."""
+    import torch
+    flag = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    ctypes.c_int32.from_address(flag.data_ptr()).value = 0
+    return flag
+
+
+def _flag_after(flag, stream):
+    """The flag once everything enqueued on the stream so far is done"""
+    import torch
+    if stream is None:
+        torch.cuda.current_stream().synchronize()
+    else:
+        torch.cuda.ExternalStream(_stream_ptr(stream).value or 0).synchronize()
+    return ctypes.c_int32.from_address(flag.data_ptr()).value
+
+
 def relayout_planes_folded(planes, w_zero, group_size, signed, stream=None):
     """Weight planes [bits, rows, k/32] and their zero points [rows, k/group_size] (whole numbers) -> K-tiled records of
     the signed differences code - zero point, [k/128, rows, folded bits, 4]; a GEMM on them needs no weight zero points.
@@ -316,10 +336,10 @@ def relayout_planes_folded(planes, w_zero, group_size, signed, stream=None):
     assert planes.is_cuda and planes.is_contiguous() and kw % 4 == 0 and rb
     assert w_zero.dtype == torch.float32 and w_zero.is_contiguous() and tuple(w_zero.shape) == (rows, kw * 32 // group_size)
     out = torch.empty((kw // 4, rows, rb, 4), dtype=torch.int32, device=planes.device)
-    misfit = torch.zeros(1, dtype=torch.int32, device=planes.device)
+    misfit = _host_flag()
     _check(lib().abq_relayout_planes_folded(planes.data_ptr(), w_zero.data_ptr(), group_size, out.data_ptr(), rows, kw * 32, bits,
                                             int(bool(signed)), misfit.data_ptr(), _stream_ptr(stream)), "abq_relayout_planes_folded")
-    if int(misfit.item()):
+    if _flag_after(misfit, stream):
         raise ValueError("zero points that are no whole numbers, or differences that do not fit the records")
     return out
 
@@ -331,10 +351,10 @@ def relayout_planes_fp6_folded(planes, w_zero, group_size, signed, stream=None):
     assert planes.is_cuda and planes.is_contiguous() and kw % 4 == 0
     assert w_zero.dtype == torch.float32 and w_zero.is_contiguous() and tuple(w_zero.shape) == (rows, kw * 32 // group_size)
     out = torch.empty((kw // 4, rows, 24), dtype=torch.int32, device=planes.device)
-    misfit = torch.zeros(1, dtype=torch.int32, device=planes.device)
+    misfit = _host_flag()
     _check(lib().abq_relayout_planes_fp6_folded(planes.data_ptr(), w_zero.data_ptr(), group_size, out.data_ptr(), rows, kw * 32, bits,
                                                 int(bool(signed)), misfit.data_ptr(), _stream_ptr(stream)), "abq_relayout_planes_fp6_folded")
-    if int(misfit.item()):
+    if _flag_after(misfit, stream):
         raise ValueError("zero points that are no whole numbers, or differences without an FP6 code")
     return out
 

@@ -698,6 +698,14 @@ abq_status abq_native_config_get(int x_bits, int w_bits, int is_signed, int inde
     return index < n ? ABQ_OK : ABQ_ERR_INVALID_ARG;
 }
 
+int abq_native_config_list(int x_bits, int w_bits, int is_signed, abq_tile_config *cfgs, int capacity)
+{
+    const int n = native_config(x_bits, w_bits, is_signed, -1, nullptr);
+    for (int i = 0; cfgs && i < n && i < capacity; ++i)
+        native_config(x_bits, w_bits, is_signed, i, &cfgs[i]);
+    return n;
+}
+
 // ---- GEMM --------------------------------------------------------------------------------
 
 static void apply_tuned(abq_gemm_state *st);

@@ -140,6 +140,8 @@ abq_status abq_format_kernel_name(const abq_tile_config *cfg, int is_wmma, char 
 int abq_native_config_count(int x_bits, int w_bits, int is_signed);
 abq_status abq_native_config_get(int x_bits, int w_bits, int is_signed, int index,
                                  abq_tile_config *cfg);
+/* The first `capacity` of them at once; returns how many there are. */
+int abq_native_config_list(int x_bits, int w_bits, int is_signed, abq_tile_config *cfgs, int capacity);
 
 /* ---------------------------------------------------------------------------------------
  * GEMM
