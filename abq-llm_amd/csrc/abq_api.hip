@@ -1607,13 +1607,15 @@ static abq_status static_scratch_address(void **out)
     return ABQ_OK;
 }
 
+static size_t least_workspace_bytes(const abq_gemm_state *st);
+
 abq_status abq_gemm_exec_static(const abq_gemm_state *st, void *stream)
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
     // only the strategies on prepared layouts convert anything
     const bool converts = st->strategy == ABQ_STRATEGY_TILED || st->strategy == ABQ_STRATEGY_FP6 || st->strategy == ABQ_STRATEGY_DECODE_TILED;
-    const size_t need = converts ? abq_gemm_workspace_bytes(st) : 0;
+    const size_t need = converts ? least_workspace_bytes(st) : 0;
     if (need > (size_t)ABQ_STATIC_WORKSPACE_BYTES) {
         fprintf(stderr, "[ABQ][Error] abq_gemm_exec_static: this GEMM converts %zu bytes of operands, the static workspace holds %zu\n",
                 need, (size_t)ABQ_STATIC_WORKSPACE_BYTES);
@@ -1644,10 +1646,10 @@ static RowSumPlan row_sum_plan(const abq_gemm_state *st, size_t converted)
 {
     const abq_tile_config &c = st->cfg;
     RowSumPlan p{ true, 0, 0, 0 };
-    // which operands are fed as value - 128: every unsigned 8-bit one on the prefill kernel; on the decode kernel of
-    // prepared operands those whose codes are not declared narrower
+    // which operands are fed as value - 128: the unsigned 8-bit ones whose codes are not declared narrower, and both where
+    // the weights' records hold code - 128
     int flip_x = c.x_bits == 8, flip_w = c.w_bits == 8;
-    if (st->strategy == ABQ_STRATEGY_DECODE_TILED)
+    if (st->strategy == ABQ_STRATEGY_DECODE_TILED || !biased_w(st))
         decode_tiled_flips(st, &flip_x, &flip_w);
     const bool take_x = flip_w && !st->x_row_sums, take_w = flip_x && !st->w_row_sums;
     if ((take_x && st->x_layout != ABQ_LAYOUT_PLANES) || (take_w && st->w_layout != ABQ_LAYOUT_PLANES)) {
@@ -1828,10 +1830,42 @@ abq_status abq_relayout_planes_folded(const uint32_t *planes, const float *w_zer
                                                     is_signed ? 1 : 0, misfit_dev, (hipStream_t)stream));
 }
 
+// Unsigned activations of several fields that arrive as planes, against K-tiled weights of one narrower field, on the
+// library's own choice of tile: exec converts the activations anyway, and as records of the next single-field width (their
+// codes stay below 128: no value - 128, no row sums) they run on the LDS-staged kernel, where the odd widths' own kernel is
+// staged through registers (W2A6, 128 rows, kernel alone: 5120 x 13824 50.9 against 22.5 us, 13824 x 5120 27.6 against 19.3).
+// The state keeps its own pair (signed pairs become the padded one: abq_gemm_set_operand_layout); what runs is decided per call
+// from the workspace, which holds the wider records or does not.
+static bool unsigned_pads_activations(const abq_gemm_state *st)
+{
+    const abq_tile_config &c = st->cfg;
+    return !c.is_signed && st->strategy == ABQ_STRATEGY_TILED && st->auto_chosen && st->M > 16 && !st->group_size && !st->act &&
+           st->x_layout == ABQ_LAYOUT_PLANES && st->w_layout == ABQ_LAYOUT_TILED && !one_field(c.x_bits) && one_field(c.w_bits) &&
+           c.w_bits < 8 && st->reserved[2] == 0 && st->reserved[3] == 0;
+}
+
+static bool run_unsigned_padded(const abq_gemm_state *st, abq_gemm_state *padded)
+{
+    if (!unsigned_pads_activations(st) || !st->workspace ||
+        st->workspace_bytes < planes_bytes(st->M, st->K, abq_padded_bits(st->cfg.x_bits)))
+        return false;
+    *padded = *st;
+    padded->reserved[2] = st->cfg.x_bits;
+    padded->reserved[3] = st->cfg.w_bits;
+    padded->cfg.x_bits = abq_padded_bits(st->cfg.x_bits);
+    if (switch_to_tiled(padded) != ABQ_OK)
+        return false;
+    apply_tuned(padded);
+    return true;
+}
+
 abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    abq_gemm_state padded;
+    if (run_unsigned_padded(st, &padded))
+        st = &padded;
     const bool x_dynamic = st->x_layout == ABQ_LAYOUT_F16 && st->reserved[1] != 0; // the kernel takes the token scales itself
     if (st->out_kind == ABQ_OUT_F16_SCALED && ((!st->x_scale && !x_dynamic) || !st->w_scale))
         return ABQ_ERR_INVALID_ARG;
@@ -1936,7 +1970,7 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
             const bool narrow = st->strategy == ABQ_STRATEGY_TILED && !biased && x_plane_bits(st) < c.x_bits && w_plane_bits(st) < c.w_bits;
             const bool wanted = biased ? true
                                 : st->strategy == ABQ_STRATEGY_DECODE_TILED ? a.flip_w != 0
-                                : !narrow && (t->entries[st->variant].flags & kNeedsRowSums) && c.w_bits == 8;
+                                : !narrow && (t->entries[st->variant].flags & kNeedsRowSums) && a.flip_w;
             const RowSumPlan plan = row_sum_plan(st, xb + wb);
             if (wanted && plan.ok) {
                 e = launch_relayout_planes_padded(st->X, reinterpret_cast<uint32_t *>(ws), st->M, st->K, xrec, x_plane_bits(st), biased ? 2 : 0,
@@ -2029,7 +2063,7 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
             // The sums the caller set are taken; those of an operand still in planes are taken here, into the
             // workspace behind the converted copies, if it has the room.  Otherwise the kernel of the same tile
             // that gathers the sums itself runs.
-            const bool need_x = c.w_bits == 8, need_w = c.x_bits == 8;
+            const bool need_x = a.flip_w != 0, need_w = a.flip_x != 0;
             const RowSumPlan plan = row_sum_plan(st, xb + wb);
             if (plan.ok) {
                 if (need_x && !st->x_row_sums && !x_sums_taken) {
@@ -2139,10 +2173,9 @@ abq_status abq_relayout_planes_fp6_folded(const uint32_t *planes, const float *w
                                                  misfit_dev));
 }
 
-size_t abq_gemm_workspace_bytes(const abq_gemm_state *st)
+// What exec needs at least: the operands still in planes as records of their own width.
+static size_t least_workspace_bytes(const abq_gemm_state *st)
 {
-    if (!st || !st->init_success)
-        return 0;
     if (st->strategy == ABQ_STRATEGY_FP6)
         return (st->x_layout == ABQ_LAYOUT_FP6 ? 0 : fp6_bytes(st->M, st->K)) +
                (st->w_layout == ABQ_LAYOUT_FP6 ? 0 : fp6_bytes(st->N, st->K));
@@ -2152,6 +2185,14 @@ size_t abq_gemm_workspace_bytes(const abq_gemm_state *st)
     const size_t wb = st->w_layout == ABQ_LAYOUT_TILED ? 0 : planes_bytes(st->N, st->K, st->cfg.w_bits);
     // (pairs with an unsigned 8-bit operand on the staged kernel: the row sums of the operands still in planes)
     return xb + wb + (wants_row_sums(st) ? row_sum_plan(st, xb + wb).bytes : 0);
+}
+
+size_t abq_gemm_workspace_bytes(const abq_gemm_state *st)
+{
+    if (!st || !st->init_success)
+        return 0;
+    const size_t least = least_workspace_bytes(st);
+    return unsigned_pads_activations(st) ? std::max(least, planes_bytes(st->M, st->K, abq_padded_bits(st->cfg.x_bits))) : least;
 }
 
 static abq_status set_operand_layout_by_rules(abq_gemm_state *st, int x_layout, int w_layout);

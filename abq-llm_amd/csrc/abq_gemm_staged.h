@@ -14,7 +14,8 @@
 //             operands need nothing).  Signed operands are placed at the top of the byte and the
 //             result shifted right by 16 - q - p, unsigned ones of at most 4 bits are fed as they
 //             are.  An unsigned 8-bit operand is fed as value - 128 (bit 7 flipped after the LDS read,
-//             one xor per dword of the operand) and the result corrected in the epilogue with 128 x the
+//             one xor per dword of the operand; records of codes below 128 as they are, flip_x / flip_w of
+//             GemmArgs) and the result corrected in the epilogue with 128 x the
 //             other operand's row sums, which the kernel does not take itself (gathering them beside
 //             the MFMAs cost more than the staging saved): they come in through GemmArgs, computed once
 //             per weight matrix and once per activation block by abq_row_sums.  The widths made of
@@ -77,14 +78,14 @@ template <int BITS, bool FP6> struct StagedOperand {
 // int8 MFMA operand of K step c (0..3) out of the pieces of one fragment (kReads 16-byte reads: this
 // lane half's 64 elements as field words; element order as abq_bits.h: field word j of a word-set
 // carries in byte c', at bits [f s, f s + f), the element at expanded dword (8 / f) j + s, byte c').
-template <int BITS, bool SIGNED> __device__ __forceinline__ v4i staged_int8_operand(const v4i *piece, int c)
+// flip: 0x80808080 where unsigned 8-bit codes are fed as value - 128, 0 where the records hold codes below 128.
+template <int BITS, bool SIGNED> __device__ __forceinline__ v4i staged_int8_operand(const v4i *piece, int c, int flip)
 {
     if constexpr (BITS == 8) {
         if constexpr (SIGNED)
             return piece[c];
-        else // value - 128
-            return v4i{ piece[c][0] ^ (int)0x80808080u, piece[c][1] ^ (int)0x80808080u, piece[c][2] ^ (int)0x80808080u,
-                        piece[c][3] ^ (int)0x80808080u };
+        else
+            return v4i{ piece[c][0] ^ flip, piece[c][1] ^ flip, piece[c][2] ^ flip, piece[c][3] ^ flip };
     } else if constexpr (BITS == 4) {
         // step c <- words 2c, 2c + 1 of the lane's eight; each word holds two expanded dwords
         const uint32_t w0 = (uint32_t)piece[c / 2][2 * (c % 2)], w1 = (uint32_t)piece[c / 2][2 * (c % 2) + 1];
@@ -155,7 +156,7 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     constexpr int NPW = NPR + (GROUPED ? 1 : 0);               // GROUPED: and one load of 64 scales (256 bytes)
     static_assert(!GROUPED || BN / 64 <= WM * WN || BN < 64, "group scales: a wave per block of 64 scales");
     constexpr int kSteps = FP6 ? 2 : 4;                        // MFMA K steps per tile of 128
-    constexpr bool FLIP_X = !FP6 && !SIGNED && QB == 8, FLIP_W = !FP6 && !SIGNED && PB == 8; // fed as value - 128
+    constexpr bool FLIP_X = !FP6 && !SIGNED && QB == 8, FLIP_W = !FP6 && !SIGNED && PB == 8; // fed as value - 128 where the host says so
     static_assert(!GROUPED || !(FLIP_X || FLIP_W), "no group scales on unsigned 8-bit operands");
     static_assert(S >= 3 && S <= 4, "three or four LDS stages");
     static_assert(NPW * S < 64, "the load counter has six bits");
@@ -183,6 +184,8 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     const int M = __builtin_amdgcn_readfirstlane(a.M), N = __builtin_amdgcn_readfirstlane(a.N);
     const int ktot = __builtin_amdgcn_readfirstlane(a.K) / 128;         // K tiles
     const int ktiles = (ktot + WK - 1) / WK;                            // trips of the K loop: a K tile per group
+
+    const int flip_x = FLIP_X && a.flip_x ? (int)0x80808080u : 0, flip_w = FLIP_W && a.flip_w ? (int)0x80808080u : 0;
 
     int mb, nb;
     tile_of_workgroup(blockIdx.x, m_blocks, n_blocks_per_xcd, &mb, &nb);
@@ -264,8 +267,8 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
                                    : __builtin_shufflevector(pb[1], pb[2], 2, 3, 4, 5, 6, 7, -1, -1);
             c = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, fresh ? zero : c, 2, 2, 0, 0, 0, 0);
         } else {
-            c = __builtin_amdgcn_mfma_i32_32x32x32_i8(staged_int8_operand<QB, SIGNED>(pa, ks),
-                                                      staged_int8_operand<PB, SIGNED>(pb, ks), fresh ? zero : c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_i32_32x32x32_i8(staged_int8_operand<QB, SIGNED>(pa, ks, flip_x),
+                                                      staged_int8_operand<PB, SIGNED>(pb, ks, flip_w), fresh ? zero : c, 0, 0, 0);
         }
     };
     // The tile the next requests are for: its operands' records and its scales, all wave-uniform (scalar
@@ -506,8 +509,8 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     // unsigned pair written with the 128 already taken off (abq_relayout_planes_biased), and nothing was flipped here.
     constexpr bool MAY_BE_BIASED = !FP6 && SIGNED && QB == 8 && PB == 8 && !GROUPED;
     if constexpr (FLIP_X || FLIP_W || MAY_BE_BIASED) {
-        const bool fix_x = FLIP_X || (MAY_BE_BIASED && a.w_row_sums != nullptr); // X was fed as value - 128
-        const bool fix_w = FLIP_W || (MAY_BE_BIASED && a.x_row_sums != nullptr);
+        const bool fix_x = (FLIP_X && a.flip_x) || (MAY_BE_BIASED && a.w_row_sums != nullptr); // X was fed as value - 128
+        const bool fix_w = (FLIP_W && a.flip_w) || (MAY_BE_BIASED && a.x_row_sums != nullptr);
         if (fix_x || fix_w) {
             int col_fix[TN];
 #pragma unroll
