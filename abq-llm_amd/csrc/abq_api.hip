@@ -319,11 +319,11 @@ static abq_status resolve(const abq_tile_config *cfg, int x_bits, int w_bits, in
             return ABQ_ERR_UNSUPPORTED;
         const KernelEntry &e = es[v];
         const int bm = 32 * e.tm * e.wm, bn = 32 * e.tn * e.wn;
-        const int mblocks = (M + bm - 1) / bm, npx = ((N + bn - 1) / bn + 7) / 8;
+        const int mblocks = (M + bm - 1) / bm, nblocks = (N + bn - 1) / bn;
         st->strategy = strategy;
         st->variant = v;
         entry_to_config(e, strategy, x_bits, w_bits, is_signed, 0, &st->cfg);
-        st->grid_dim = abq_dim3{ (unsigned)(8 * npx * mblocks), 1, 1 };
+        st->grid_dim = abq_dim3{ tile_grid(mblocks, nblocks), 1, 1 };
         st->block_dim = abq_dim3{ (unsigned)(64 * e.wm * e.wn * e.wk), 1, 1 };
         st->shared_mem_size = e.lds;
         return ABQ_OK;
@@ -393,11 +393,11 @@ static abq_status resolve(const abq_tile_config *cfg, int x_bits, int w_bits, in
             return ABQ_ERR_TOO_LARGE;
         const KernelEntry &e = tt_->entries[v];
         const int bm = 32 * e.tm * e.wm, bn = 32 * e.tn * e.wn;
-        const int mblocks = (M + bm - 1) / bm, npx = ((N + bn - 1) / bn + 7) / 8;
+        const int mblocks = (M + bm - 1) / bm, nblocks = (N + bn - 1) / bn;
         st->strategy = strategy;
         st->variant = v;
         entry_to_config(e, strategy, x_bits, w_bits, is_signed, 0, &st->cfg);
-        st->grid_dim = abq_dim3{ (unsigned)(8 * npx * mblocks), 1, 1 };
+        st->grid_dim = abq_dim3{ tile_grid(mblocks, nblocks), 1, 1 };
         st->block_dim = abq_dim3{ (unsigned)(64 * e.wm * e.wn * e.wk), 1, 1 };
         st->shared_mem_size = e.lds ? e.lds : 2 * (size_t)(bm + bn) * (e.kb + 16) + (bm + bn) * 4;
         return ABQ_OK;
@@ -993,7 +993,7 @@ static abq_status switch_to_fp6(abq_gemm_state *st)
         entry_to_config(e, ABQ_STRATEGY_FP6, xb_, wb_, sg_, 0, &st->cfg);
         st->strategy = ABQ_STRATEGY_FP6;
         st->variant = gpick;
-        st->grid_dim = abq_dim3{ (unsigned)(8 * (((st->N + bn - 1) / bn + 7) / 8) * ((st->M + bm - 1) / bm)), 1, 1 };
+        st->grid_dim = abq_dim3{ tile_grid((st->M + bm - 1) / bm, (st->N + bn - 1) / bn), 1, 1 };
         st->block_dim = abq_dim3{ (unsigned)(64 * e.wm * e.wn * e.wk), 1, 1 };
         st->shared_mem_size = e.lds;
         return ABQ_OK;
@@ -1402,7 +1402,7 @@ static abq_status pick_grouped_tiled(abq_gemm_state *state)
     {
         const KernelEntry &e = tg->entries[pick];
         const int bm = block_m(e), bn = block_n(e);
-        state->grid_dim = abq_dim3{ (unsigned)(8 * (((state->N + bn - 1) / bn + 7) / 8) * ((state->M + bm - 1) / bm)), 1, 1 };
+        state->grid_dim = abq_dim3{ tile_grid((state->M + bm - 1) / bm, (state->N + bn - 1) / bn), 1, 1 };
         state->block_dim = abq_dim3{ (unsigned)(64 * e.wm * e.wn * e.wk), 1, 1 };
         state->shared_mem_size = e.lds ? e.lds : 2 * (size_t)(bm + bn) * (e.kb + 16) + (bm + bn) * 4;
     }

@@ -142,7 +142,7 @@ template <int TM, int TN, int WM, int WN, int STAGE_BYTES> struct StagedOutputLd
 // them under a scale of zero).
 template <int QB, int PB, bool SIGNED, bool FP6, int TM, int TN, int WM, int WN, int S, bool GROUPED = false, int WK = 1>
 __global__ __launch_bounds__(64 * WM * WN * WK, (WM * WN * WK > 4 || TM * TN > 4) ? 1 : 2)
-void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_blocks, int n_blocks_per_xcd)
+void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_blocks, int n_blocks)
 {
     using TA = StagedOperand<QB, FP6>;
     using TB = StagedOperand<PB, FP6>;
@@ -188,10 +188,9 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     const int flip_x = FLIP_X && a.flip_x ? (int)0x80808080u : 0, flip_w = FLIP_W && a.flip_w ? (int)0x80808080u : 0;
 
     int mb, nb;
-    tile_of_workgroup(blockIdx.x, m_blocks, n_blocks_per_xcd, &mb, &nb);
-    const int m0 = mb * BM, n0 = nb * BN;
-    if (n0 >= N)
+    if (!tile_of_workgroup(blockIdx.x, m_blocks, n_blocks, &mb, &nb))
         return; // uniform over the workgroup, before any barrier
+    const int m0 = mb * BM, n0 = nb * BN;
 
     // Wave load q of a tile fills LDS units [64 q, 64 q + 64) of the stage, activations first; the unit
     // at LDS place P of an operand block is unit lds_offset(P) / 16 of that operand's tile.  Loads past
@@ -644,8 +643,7 @@ static hipError_t launch_mfma_staged(const GemmArgs &a, hipStream_t stream)
     const int m_blocks = (a.M + BM - 1) / BM, n_blocks = (a.N + BN - 1) / BN;
     using Stages = StagedStages<QB, PB, FP6, TM, TN, WM, WN, GROUPED, WK>;
     constexpr int S = Stages::value;
-    const int npx = (n_blocks + 7) / 8;
-    const dim3 grid(8 * npx * m_blocks);
+    const dim3 grid(tile_grid(m_blocks, n_blocks));
     static const hipError_t attr = hipFuncSetAttribute(
         reinterpret_cast<const void *>(&gemm_mfma_staged<QB, PB, SIGNED, FP6, TM, TN, WM, WN, S, GROUPED, WK>),
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -654,7 +652,7 @@ static hipError_t launch_mfma_staged(const GemmArgs &a, hipStream_t stream)
     // int32 results are stored from the registers; every other kind goes through LDS
     const size_t lds = a.out_kind == 0 ? Stages::kLds : (size_t)StagedOutputLds<TM, TN, WM, WN, (int)Stages::kLds>::value;
     hipLaunchKernelGGL((gemm_mfma_staged<QB, PB, SIGNED, FP6, TM, TN, WM, WN, S, GROUPED, WK>), grid, dim3(64 * WM * WN * WK), lds,
-                       stream, a, reinterpret_cast<const v4u *>(a.X), reinterpret_cast<const v4u *>(a.W), m_blocks, npx);
+                       stream, a, reinterpret_cast<const v4u *>(a.X), reinterpret_cast<const v4u *>(a.W), m_blocks, n_blocks);
     return hipGetLastError();
 }
 

@@ -204,7 +204,7 @@ template <int BITS, int ROWS, int NT, int KB, Int8Mode MODE, bool SUM> struct Op
 // cut the L2 -> L1 traffic per MFMA).
 template <int Q, int P, bool SIGNED, int TM, int TN, bool GROUPED, int KB, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, (WM * WN > 4 ? 1 : (TM * TN <= 4 || KB == 64 ? 2 : 1)))
-void gemm_mfma_tiled(const GemmArgs a, const uint32_t *xt, const uint32_t *wt, int m_blocks, int n_blocks_per_xcd)
+void gemm_mfma_tiled(const GemmArgs a, const uint32_t *xt, const uint32_t *wt, int m_blocks, int n_blocks)
 {
     constexpr int NT = 64 * WM * WN; // threads
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
@@ -232,12 +232,10 @@ void gemm_mfma_tiled(const GemmArgs a, const uint32_t *xt, const uint32_t *wt, i
     const int M = __builtin_amdgcn_readfirstlane(a.M), N = __builtin_amdgcn_readfirstlane(a.N);
     const int ktiles = __builtin_amdgcn_readfirstlane(a.K) / KB; // stages
 
-    // workgroup -> tile: XCD x = id % 8 owns n blocks [x * npx, (x+1) * npx), M fastest
     int mb, nb;
-    tile_of_workgroup(blockIdx.x, m_blocks, n_blocks_per_xcd, &mb, &nb);
-    const int m0 = mb * BM, n0 = nb * BN;
-    if (n0 >= N)
+    if (!tile_of_workgroup(blockIdx.x, m_blocks, n_blocks, &mb, &nb))
         return; // uniform over the workgroup, before any barrier
+    const int m0 = mb * BM, n0 = nb * BN;
 
     // this thread's share of the two operands of a stage (rows past the edge are clamped for loading
     // and dropped at the store)
@@ -453,15 +451,14 @@ static hipError_t launch_mfma_tiled(const GemmArgs &a, hipStream_t stream)
     if (GROUPED && (Int8ModeOf<Q, SIGNED>::value == kFlip || Int8ModeOf<P, SIGNED>::value == kFlip))
         return hipErrorInvalidValue; // group scales with 8-bit unsigned operands: not built
     const int m_blocks = (a.M + BM - 1) / BM, n_blocks = (a.N + BN - 1) / BN;
-    const int npx = (n_blocks + 7) / 8;
     const size_t lds = 2 * (size_t)(BM + BN) * (KB + 16) + (BM + BN) * sizeof(int);
     static const hipError_t attr = hipFuncSetAttribute(
         reinterpret_cast<const void *>(&gemm_mfma_tiled<Q, P, SIGNED, TM, TN, GROUPED, KB, WM, WN>),
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (attr != hipSuccess)
         return attr;
-    const dim3 grid(8 * npx * m_blocks);
-    hipLaunchKernelGGL((gemm_mfma_tiled<Q, P, SIGNED, TM, TN, GROUPED, KB, WM, WN>), grid, dim3(64 * WM * WN), lds, stream, a, a.X, a.W, m_blocks, npx);
+    const dim3 grid(tile_grid(m_blocks, n_blocks));
+    hipLaunchKernelGGL((gemm_mfma_tiled<Q, P, SIGNED, TM, TN, GROUPED, KB, WM, WN>), grid, dim3(64 * WM * WN), lds, stream, a, a.X, a.W, m_blocks, n_blocks);
     return hipGetLastError();
 }
 

@@ -118,15 +118,53 @@ inline int decode_grouped_tiled_waves(int K, int w_bits, int group_size)
 // activation and weight block they load is shared in that XCD's L2, whatever M is (with M fastest over
 // all m blocks, 16384 rows ran 25-35 % slower; groups of 2, 4 and 8 measured within 2 %, 4 ahead by up
 // to 4 % at 2048 rows).
-__device__ __forceinline__ void tile_of_workgroup(int id, int m_blocks, int n_blocks_per_xcd, int *mb, int *nb)
+// Where whole columns of tiles would give some XCDs a good deal more than their share (tiles_spread), an XCD owns n_blocks / 8 of
+// them, and the tiles of the n_blocks % 8 that are left are dealt out evenly: behind every eight m blocks of its own an XCD takes an
+// eighth of theirs, in runs of consecutive m blocks, whose activations it has just read.
+// Returns false for the workgroups of a grid (tile_grid) that are left without a tile.
+constexpr int kSpreadM = 8;
+// From six rounds of an XCD's 32 compute units on, where the XCD with the most columns has an eighth more than its share: 9 columns
+// are 2 for four of the XCDs and none for three (decoder-layer linears, W2A8 groups of 128: hidden 1152 8192 rows 615 -> 581 us, W4A4
+// 535 -> 505; hidden 2176 1476 -> 1392; 12000 rows of 1536 1173 -> 1134).  Below that the tiles dealt out cost what they save: 2048
+// rows of 1408 253 -> 259; W4A4 with one scale, 4096 rows of 1152, 145 -> 150.
+__host__ __device__ __forceinline__ bool tiles_spread(int m_blocks, int n_blocks)
+{
+    const int most = (n_blocks + 7) / 8;
+    return (long)m_blocks * most > 200 && 8l * 8 * most > 9l * n_blocks;
+}
+
+__device__ __forceinline__ bool tile_of_workgroup(int id, int m_blocks, int n_blocks, int *mb, int *nb)
 {
     constexpr int GM = 4;
     const int xcd = id & 7, slot = id >> 3;
-    const int per_group = GM * n_blocks_per_xcd;
-    const int grp = slot / per_group, in = slot - grp * per_group;
-    const int gm = min(GM, m_blocks - grp * GM); // the last group may be short
-    *mb = grp * GM + in % gm;
-    *nb = xcd * n_blocks_per_xcd + in / gm;
+    const bool spread = tiles_spread(m_blocks, n_blocks);
+    const int npx = spread ? n_blocks >> 3 : (n_blocks + 7) >> 3, left = spread ? n_blocks & 7 : 0;
+    // the m blocks an XCD goes through before it takes its part of what is left: all of them where nothing is
+    const int most = spread ? kSpreadM : m_blocks, sup = slot / (most * npx + left), in = slot - sup * (most * npx + left);
+    const int sm = min(most, m_blocks - sup * most);
+    if (in < sm * npx) {
+        const int per_group = GM * npx;
+        const int grp = in / per_group, pos = in - grp * per_group;
+        const int gm = min(GM, sm - grp * GM); // the last group may be short
+        *mb = sup * most + grp * GM + pos % gm;
+        *nb = xcd * npx + pos / gm;
+        return *nb < n_blocks;
+    }
+    const int rest = left * sm, u = xcd * ((rest + 7) >> 3) + in - sm * npx;
+    if (u >= rest)
+        return false;
+    *mb = sup * most + u % sm;
+    *nb = 8 * npx + u / sm;
+    return true;
+}
+
+// Workgroups of a launch over m_blocks x n_blocks tiles numbered like that.
+inline unsigned tile_grid(int m_blocks, int n_blocks)
+{
+    if (!tiles_spread(m_blocks, n_blocks))
+        return 8u * (((unsigned)n_blocks + 7) / 8) * (unsigned)m_blocks;
+    const unsigned npx = (unsigned)n_blocks / 8, left = (unsigned)n_blocks % 8, last = (unsigned)m_blocks % kSpreadM;
+    return 8u * ((unsigned)(m_blocks / kSpreadM) * (kSpreadM * npx + left) + last * npx + (last * left + 7u) / 8u);
 }
 
 // ---- byte shuffles inside a quad of lanes (the packing kernels and the decode kernel that quantises its own

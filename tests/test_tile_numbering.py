@@ -1,0 +1,51 @@
+"""Every output tile belongs to exactly one workgroup of the grid, an even share of them to each XCD (workgroup id modulo 8):
+the numbering shared by the prefill kernels, compiled for the host."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#define __device__
+#define __host__
+#define __forceinline__ inline
+#include <algorithm>
+using std::min;
+namespace abq {
+%s
+}
+extern "C" int tile(int id, int m_blocks, int n_blocks, int *mb, int *nb) { return abq::tile_of_workgroup(id, m_blocks, n_blocks, mb, nb); }
+extern "C" unsigned grid(int m_blocks, int n_blocks) { return abq::tile_grid(m_blocks, n_blocks); }
+"""
+
+
+@pytest.fixture(scope="module")
+def numbering(tmp_path_factory):
+    text = open(os.path.join(ROOT, "abq-llm_amd", "csrc", "abq_kernels.h")).read()
+    first = text.index("constexpr int kSpreadM")
+    last = text.index("}\n", text.index("inline unsigned tile_grid")) + 2
+    d = tmp_path_factory.mktemp("numbering")
+    src, lib = d / "numbering.cpp", d / "numbering.so"
+    src.write_text(SOURCE % text[first:last])
+    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", "-o", str(lib), str(src)])
+    return ctypes.CDLL(str(lib))
+
+
+@pytest.mark.parametrize("m_blocks", [1, 2, 3, 4, 5, 7, 8, 13, 128])
+@pytest.mark.parametrize("n_blocks", [1, 2, 7, 8, 9, 15, 16, 33, 86, 172])
+def test_every_tile_once_and_evenly(numbering, m_blocks, n_blocks):
+    seen, per_xcd = set(), [0] * 8
+    for i in range(numbering.grid(m_blocks, n_blocks)):
+        mb, nb = ctypes.c_int(), ctypes.c_int()
+        if numbering.tile(i, m_blocks, n_blocks, ctypes.byref(mb), ctypes.byref(nb)):
+            assert 0 <= mb.value < m_blocks and 0 <= nb.value < n_blocks
+            assert (mb.value, nb.value) not in seen
+            seen.add((mb.value, nb.value))
+            per_xcd[i % 8] += 1
+    assert len(seen) == m_blocks * n_blocks
+    if m_blocks * ((n_blocks + 7) // 8) > 200:  # from six rounds of an XCD's compute units on: within an eighth of an even share,
+        # but for what the runs of eight m blocks cannot divide
+        assert max(per_xcd) <= 1.125 * len(seen) / 8 + (m_blocks % 8 > 0)
