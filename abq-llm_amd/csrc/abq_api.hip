@@ -21,7 +21,8 @@ hipError_t launch_pack_f16_tiled(const void *, const float *, uint32_t *, int, i
 hipError_t launch_pack_f16_fp6(const void *, const float *, uint32_t *, int, int, int, int, hipStream_t);
 hipError_t launch_pack_u4(const uint32_t *, uint32_t *, int, int, int, hipStream_t);
 hipError_t launch_relayout_planes(const uint32_t *, uint32_t *, int, int, int, hipStream_t);
-hipError_t launch_relayout_planes_padded(const uint32_t *, uint32_t *, int, int, int, int, int, hipStream_t, int *row_sums = nullptr);
+hipError_t launch_relayout_planes_padded(const uint32_t *, uint32_t *, int, int, int, int, int, hipStream_t, int *row_sums = nullptr,
+                                         int *clear = nullptr, uint32_t n_clear = 0);
 hipError_t launch_relayout_planes_folded(const uint32_t *, const float *, int, uint32_t *, int, int, int, int, int, int *, hipStream_t);
 hipError_t launch_relayout_planes_fp6(const uint32_t *, uint32_t *, int, int, int, int, hipStream_t, const float *zero = nullptr,
                                       int group_size = 0, int *flag = nullptr);
@@ -1830,6 +1831,25 @@ abq_status abq_relayout_planes_folded(const uint32_t *planes, const float *w_zer
                                                     is_signed ? 1 : 0, misfit_dev, (hipStream_t)stream));
 }
 
+// Parts of K for an int32 GEMM on 128x64 tiles (gemm_mfma_staged, KP), 1 where that does not pay.  Measured with the conversion
+// of the activations in the call and weights from memory, us on the tile that ran before / in parts:
+//   W8A8  128 x 5120 x 13824 32.6 / 26.1, 128 x 4096 x 11008 27.6 / 20.7, 128 x 2048 x 8192 16.7 / 13.3 (unsigned 22.1 / 14.5),
+//         100 x 4096 x 6144 16.6 / 14.4, 256 x 2560 x 11008 28.7 / 23.0, 512 x 1024 x 8192 19.3 / 19.2; 1024 x 512 x 8192 21.6 / 23.8
+//   W4A8  128 x 5120 x 13824 27.5 / 23.0, 128 x 2048 x 16384 23.8 / 18.0;  W4A4 22.6 / 21.4;  W2A2 128 x 4096 x 11008 17.3 / 15.9
+// Two parts (86 to 128 tiles) move as many bytes per compute unit as the 64x64 tile did: 512 x 2048 x 8192 W8A8 21.9 / 24.0, W2A2
+// 17.0 / 19.5.  Shorter parts lose to the second pass over the result what they gain: W8A8 below 16 K tiles (128 x 5120 x 5120
+// 16.7 / 16.8 in three), the others below 28 (W4A8 100 x 4096 x 6144 13.9 / 14.1 in two).  W2A8 is as fast on its 64x64 tile with four
+// K groups (128 x 5120 x 13824 23.0 / 23.4).
+static int k_parts_of_shape(int x_bits, int w_bits, int M, int N, int K)
+{
+    const bool w8a8 = x_bits == 8 && w_bits == 8;
+    const long m_blocks = (M + 127) / 128, tiles = m_blocks * ((N + 63) / 64);
+    if (m_blocks > 4 || tiles > 85 || M * 4l < m_blocks * 128 * 3 || (x_bits == 8 && w_bits == 2))
+        return 1;
+    const long fit = 256 / tiles, long_enough = K / 128 / (w8a8 ? 16 : 28), parts = fit < long_enough ? fit : long_enough;
+    return parts < 3 ? 1 : parts > 8 ? 8 : (int)parts;
+}
+
 // Unsigned activations of several fields that arrive as planes, against K-tiled weights of one narrower field, on the
 // library's own choice of tile: exec converts the activations anyway, and as records of the next single-field width (their
 // codes stay below 128: no value - 128, no row sums) they run on the LDS-staged kernel, where the odd widths' own kernel is
@@ -1859,6 +1879,32 @@ static bool run_unsigned_padded(const abq_gemm_state *st, abq_gemm_state *padded
     return true;
 }
 
+// int32 results of a GEMM whose activations exec converts, on a grid of 128x64 tiles that leaves half of the compute units free,
+// and long K: several workgroups per tile, each with a part of K, add into the result, which the conversion's launch clears
+// (gemm_mfma_staged, KP).  Returns the parts, 1 for a call that runs as its state says; *split is the state on that tile.
+static int run_k_parts(const abq_gemm_state *st, abq_gemm_state *split)
+{
+    const abq_tile_config &c = st->cfg;
+    if (st->strategy != ABQ_STRATEGY_TILED || !st->auto_chosen || st->out_kind != ABQ_OUT_I32 || st->group_size || st->act ||
+        st->x_layout != ABQ_LAYOUT_PLANES || st->w_layout != ABQ_LAYOUT_TILED)
+        return 1;
+    const int parts = k_parts_of_shape(c.x_bits, c.w_bits, st->M, st->N, st->K);
+    if (parts < 2)
+        return 1;
+    const KernelTable *t = find_table(registry().tiled, c.x_bits, c.w_bits, c.is_signed);
+    // (two groups of waves in a workgroup for the narrow pairs, whose K tiles are short: W4A4 128 x 5120 x 13824 17.1 against 18.4 us)
+    const int wk = c.x_bits + c.w_bits <= 8 ? 2 : 1;
+    for (int i = 0; t && i < t->count; ++i) {
+        const KernelEntry &e = t->entries[i];
+        if (e.lds != 0 && e.tm == 2 && e.tn == 1 && e.wm == 2 && e.wn == 2 && e.wk == wk && e.kb == 128) {
+            *split = *st;
+            split->variant = i;
+            return parts;
+        }
+    }
+    return 1;
+}
+
 abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
 {
     if (!st || !st->init_success)
@@ -1866,6 +1912,10 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
     abq_gemm_state padded;
     if (run_unsigned_padded(st, &padded))
         st = &padded;
+    abq_gemm_state split;
+    const int k_parts = run_k_parts(st, &split);
+    if (k_parts > 1)
+        st = &split;
     const bool x_dynamic = st->x_layout == ABQ_LAYOUT_F16 && st->reserved[1] != 0; // the kernel takes the token scales itself
     if (st->out_kind == ABQ_OUT_F16_SCALED && ((!st->x_scale && !x_dynamic) || !st->w_scale))
         return ABQ_ERR_INVALID_ARG;
@@ -1893,6 +1943,9 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
     a.x_row_sums = nullptr; // (handed to a kernel only by the branches below that need them)
     a.w_row_sums = nullptr;
     decode_tiled_flips(st, &a.flip_x, &a.flip_w);
+    a.k_parts = k_parts;
+    int *clear = k_parts > 1 ? static_cast<int *>(st->D) : nullptr; // the result several workgroups will add into
+    const uint32_t n_clear = k_parts > 1 ? (uint32_t)((size_t)st->M * st->N) : 0;
     const Registry &reg = registry();
     const abq_tile_config &c = st->cfg;
     hipError_t e;
@@ -1974,7 +2027,7 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
             const RowSumPlan plan = row_sum_plan(st, xb + wb);
             if (wanted && plan.ok) {
                 e = launch_relayout_planes_padded(st->X, reinterpret_cast<uint32_t *>(ws), st->M, st->K, xrec, x_plane_bits(st), biased ? 2 : 0,
-                                                  (hipStream_t)stream, reinterpret_cast<int *>(ws + plan.x_off));
+                                                  (hipStream_t)stream, reinterpret_cast<int *>(ws + plan.x_off), clear, n_clear);
                 if (e != hipSuccess)
                     return hip_status(e);
                 a.X = reinterpret_cast<const uint32_t *>(ws);
@@ -1984,7 +2037,7 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
         if (xb && !x_sums_taken) {
             // (planes of fewer bits than the records: the codes are extended to the record's width)
             e = launch_relayout_planes_padded(st->X, reinterpret_cast<uint32_t *>(ws), st->M, st->K, xrec, x_plane_bits(st),
-                                              biased ? 2 : (xrec != x_plane_bits(st) && c.is_signed ? 1 : 0), (hipStream_t)stream);
+                                              biased ? 2 : (xrec != x_plane_bits(st) && c.is_signed ? 1 : 0), (hipStream_t)stream, nullptr, clear, n_clear);
             if (e != hipSuccess)
                 return hip_status(e);
             a.X = reinterpret_cast<const uint32_t *>(ws);

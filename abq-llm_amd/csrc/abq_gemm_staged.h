@@ -140,9 +140,14 @@ template <int TM, int TN, int WM, int WN, int STAGE_BYTES> struct StagedOutputLd
 // times.  With a number of K tiles that is no multiple of WK the last trip finds some groups without a tile: they
 // request their last tile once more, like every wave past the end, and leave its MFMAs out (with group scales: run
 // them under a scale of zero).
-template <int QB, int PB, bool SIGNED, bool FP6, int TM, int TN, int WM, int WN, int S, bool GROUPED = false, int WK = 1>
-__global__ __launch_bounds__(64 * WM * WN * WK, (WM * WN * WK > 4 || TM * TN > 4) ? 1 : 2)
-void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_blocks, int n_blocks)
+//
+// KP: a.k_parts workgroups share an output tile: part i goes through the i-th part of the K tiles and adds its int32 results
+// into D, which an earlier launch has cleared (the sums are exact in any order).  For grids that leave most compute
+// units free, where a workgroup's time is that of bringing its tiles in: a compute unit has some 50 KB of loads in flight at
+// most, 57 GB/s on weights from memory whatever the number of stages (W8A8 128 x 5120 x 13824: 160 tiles of 64 x 64, 108 K tiles of
+// 16 KB 31.8 us, the same without MFMAs and LDS reads; 80 tiles of 128 x 64 in three parts, 36 of 24 KB, 22.2).
+template <int QB, int PB, bool SIGNED, bool FP6, int TM, int TN, int WM, int WN, int S, bool GROUPED, int WK, bool KP>
+__device__ __forceinline__ void staged_gemm(const GemmArgs &a, const v4u *xt, const v4u *wt, int m_blocks, int columns)
 {
     using TA = StagedOperand<QB, FP6>;
     using TB = StagedOperand<PB, FP6>;
@@ -182,13 +187,17 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     const int wm = wid / WN, wn = wid % WN;
     const int r = lane & 31, g = lane >> 5;
     const int M = __builtin_amdgcn_readfirstlane(a.M), N = __builtin_amdgcn_readfirstlane(a.N);
-    const int ktot = __builtin_amdgcn_readfirstlane(a.K) / 128;         // K tiles
+    const int kall = __builtin_amdgcn_readfirstlane(a.K) / 128;         // K tiles
+    const int k_parts = KP ? __builtin_amdgcn_readfirstlane(a.k_parts) : 1;
+    const int grid_tiles = KP ? (int)gridDim.x / k_parts : 0, part = KP ? (int)blockIdx.x / grid_tiles : 0;
+    const int k_first = KP ? kall * part / k_parts : 0;                 // ... of this workgroup: ktot from k_first on
+    const int ktot = KP ? kall * (part + 1) / k_parts - k_first : kall;
     const int ktiles = (ktot + WK - 1) / WK;                            // trips of the K loop: a K tile per group
 
     const int flip_x = FLIP_X && a.flip_x ? (int)0x80808080u : 0, flip_w = FLIP_W && a.flip_w ? (int)0x80808080u : 0;
 
     int mb, nb;
-    if (!tile_of_workgroup(blockIdx.x, m_blocks, n_blocks, &mb, &nb))
+    if (!tile_of_workgroup(KP ? (int)blockIdx.x - part * grid_tiles : (int)blockIdx.x, m_blocks, columns, &mb, &nb) || nb * BN >= N)
         return; // uniform over the workgroup, before any barrier
     const int m0 = mb * BM, n0 = nb * BN;
 
@@ -196,18 +205,20 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     // at LDS place P of an operand block is unit lds_offset(P) / 16 of that operand's tile.  Loads past
     // the last one repeat an earlier load of the wave (same data, same place), so that every wave
     // issues NPW loads per tile.  Rows past the edge are clamped for loading and dropped at the store.
+    // (which operand load i of a wave is for does not depend on the wave when the waves divide both operands' loads)
+    constexpr bool kDealt = NIA % NW == 0 && NI % NW == 0;
     uint32_t goff[NPW]; // bytes from the start of the operand's records of one K tile
 #pragma unroll
     for (int i = 0; i < NPR; ++i) {
         int q = wid + NW * i;
-        if (q >= NI)
+        if (NI % NW != 0 && q >= NI)
             q -= NW;
-        if (q < NIA) { // wave-uniform
-            const int v = TA::lds_offset(64 * q + lane) >> 4;
-            goff[i] = 16u * ((uint32_t)min(m0 + v / TA::kUnits, M - 1) * TA::kUnits + v % TA::kUnits);
+        if (kDealt ? NW * i < NIA : q < NIA) { // wave-uniform
+            const uint32_t v = (uint32_t)TA::lds_offset(64 * q + lane) >> 4;
+            goff[i] = 16u * ((uint32_t)min(m0 + (int)(v / TA::kUnits), M - 1) * TA::kUnits + v % TA::kUnits);
         } else {
-            const int v = TB::lds_offset(64 * (q - NIA) + lane) >> 4;
-            goff[i] = 16u * ((uint32_t)min(n0 + v / TB::kUnits, N - 1) * TB::kUnits + v % TB::kUnits);
+            const uint32_t v = (uint32_t)TB::lds_offset(64 * (q - NIA) + lane) >> 4;
+            goff[i] = 16u * ((uint32_t)min(n0 + (int)(v / TB::kUnits), N - 1) * TB::kUnits + v % TB::kUnits);
         }
     }
     // GROUPED: the wave's last load of a tile brings the scales of 64 weight rows (waves take the 64-row
@@ -274,7 +285,7 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     // registers), the lanes adding their 32-bit offsets.  Tiles past the end are copies of the last, into stages
     // nobody reads.
     const int first = min(wk, ktot - 1); // (a group beyond the last K tile never has one of its own)
-    const v4u *xq = xt + first * stride_a, *wq = wt + first * stride_b;
+    const v4u *xq = xt + (k_first + first) * stride_a, *wq = wt + (k_first + first) * stride_b;
     const float *sq = a.w_scale + first;
     const unsigned lds_wave = lds0 + wk * BUF_BYTES + wid * 1024;
     int kq = 0;
@@ -286,8 +297,7 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
         int q = wid + NW * i;
         if (NI % NW != 0 && q >= NI)
             q -= NW;
-        // (which operand request i is for does not depend on the wave when the waves divide both operands' loads)
-        const bool activations = (NIA % NW == 0 && NI % NW == 0) ? NW * i < NIA : q < NIA;
+        const bool activations = kDealt ? NW * i < NIA : q < NIA;
         lds_dma16(activations ? (const void *)xq : (const void *)wq, goff[i], lds_wave + stage + (q - wid) * 1024);
     };
     auto next_tile = [&]() {
@@ -508,15 +518,16 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     // unsigned pair written with the 128 already taken off (abq_relayout_planes_biased), and nothing was flipped here.
     constexpr bool MAY_BE_BIASED = !FP6 && SIGNED && QB == 8 && PB == 8 && !GROUPED;
     if constexpr (FLIP_X || FLIP_W || MAY_BE_BIASED) {
-        const bool fix_x = (FLIP_X && a.flip_x) || (MAY_BE_BIASED && a.w_row_sums != nullptr); // X was fed as value - 128
-        const bool fix_w = (FLIP_W && a.flip_w) || (MAY_BE_BIASED && a.x_row_sums != nullptr);
+        // (several parts of K: the sums are those of whole rows, the first part adds them)
+        const bool fix_x = part == 0 && ((FLIP_X && a.flip_x) || (MAY_BE_BIASED && a.w_row_sums != nullptr)); // X was fed as value - 128
+        const bool fix_w = part == 0 && ((FLIP_W && a.flip_w) || (MAY_BE_BIASED && a.x_row_sums != nullptr));
         if (fix_x || fix_w) {
             int col_fix[TN];
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 unsigned v = fix_x ? 128u * (unsigned)a.w_row_sums[min(n0 + wn * 32 * TN + j * 32 + r, N - 1)] : 0u;
                 if (fix_x && fix_w)
-                    v -= 16384u * (unsigned)(ktot * 128);
+                    v -= 16384u * (unsigned)(kall * 128);
                 col_fix[j] = (int)v;
             }
             // a lane's rows come in runs of four (e % 4): all of their sums are requested before any is used, one
@@ -554,6 +565,22 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
         else
             return SIGNED ? acc[i][j][e] >> (16 - QB - PB) : acc[i][j][e]; // signed fields sit at the top of their bytes
     };
+    if constexpr (KP) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int n = n0 + wn * 32 * TN + j * 32 + r;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int m = m0 + wm * 32 * TM + i * 32 + 8 * (e / 4) + 4 * g + (e % 4);
+                    if (m < M && n < N)
+                        __hip_atomic_fetch_add(reinterpret_cast<int *>(a.D) + ((size_t)m * N + n), result(i, j, e), __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+        return;
+    }
     if (a.out_kind == 2) {
         // per-token x per-channel scales, fp16 out (same arithmetic as store_result): the lane's TN
         // channel scales are loaded once, a row's token scale once per row
@@ -623,6 +650,21 @@ void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_bloc
     }
 }
 
+template <int QB, int PB, bool SIGNED, bool FP6, int TM, int TN, int WM, int WN, int S, bool GROUPED = false, int WK = 1>
+__global__ __launch_bounds__(64 * WM * WN * WK, (WM * WN * WK > 4 || TM * TN > 4) ? 1 : 2)
+void gemm_mfma_staged(const GemmArgs a, const v4u *xt, const v4u *wt, int m_blocks, int columns)
+{
+    staged_gemm<QB, PB, SIGNED, FP6, TM, TN, WM, WN, S, GROUPED, WK, false>(a, xt, wt, m_blocks, columns);
+}
+
+// The same with K in a.k_parts parts (KP above): integer fields, int32 results, no group scales.
+template <int QB, int PB, bool SIGNED, int TM, int TN, int WM, int WN, int S, int WK>
+__global__ __launch_bounds__(64 * WM * WN * WK, (WM * WN * WK > 4 || TM * TN > 4) ? 1 : 2)
+void gemm_mfma_staged_parts(const GemmArgs a, const v4u *xt, const v4u *wt, int m_blocks, int columns)
+{
+    staged_gemm<QB, PB, SIGNED, false, TM, TN, WM, WN, S, false, WK, true>(a, xt, wt, m_blocks, columns);
+}
+
 // LDS stages of a tile: as many (up to four) as leave room for the workgroups that share a compute
 // unit: two for the four-wave tiles when three stages of theirs fit twice, else one.
 template <int QB, int PB, bool FP6, int TM, int TN, int WM, int WN, bool GROUPED = false, int WK = 1> struct StagedStages {
@@ -644,6 +686,22 @@ static hipError_t launch_mfma_staged(const GemmArgs &a, hipStream_t stream)
     using Stages = StagedStages<QB, PB, FP6, TM, TN, WM, WN, GROUPED, WK>;
     constexpr int S = Stages::value;
     const dim3 grid(tile_grid(m_blocks, n_blocks));
+    const int columns = tile_columns(m_blocks, n_blocks);
+    if constexpr (!FP6 && !GROUPED && TM == 2 && TN == 1 && WM == 2 && WN == 2) { // (the tile the host splits K on)
+        if (a.k_parts > 1) {
+            if (a.out_kind != 0)
+                return hipErrorInvalidValue;
+            static const hipError_t kp_attr = hipFuncSetAttribute(
+                reinterpret_cast<const void *>(&gemm_mfma_staged_parts<QB, PB, SIGNED, TM, TN, WM, WN, S, WK>),
+                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (kp_attr != hipSuccess)
+                return kp_attr;
+            hipLaunchKernelGGL((gemm_mfma_staged_parts<QB, PB, SIGNED, TM, TN, WM, WN, S, WK>), dim3(grid.x * a.k_parts),
+                               dim3(64 * WM * WN * WK), Stages::kLds, stream, a, reinterpret_cast<const v4u *>(a.X),
+                               reinterpret_cast<const v4u *>(a.W), m_blocks, columns);
+            return hipGetLastError();
+        }
+    }
     static const hipError_t attr = hipFuncSetAttribute(
         reinterpret_cast<const void *>(&gemm_mfma_staged<QB, PB, SIGNED, FP6, TM, TN, WM, WN, S, GROUPED, WK>),
         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
@@ -652,7 +710,7 @@ static hipError_t launch_mfma_staged(const GemmArgs &a, hipStream_t stream)
     // int32 results are stored from the registers; every other kind goes through LDS
     const size_t lds = a.out_kind == 0 ? Stages::kLds : (size_t)StagedOutputLds<TM, TN, WM, WN, (int)Stages::kLds>::value;
     hipLaunchKernelGGL((gemm_mfma_staged<QB, PB, SIGNED, FP6, TM, TN, WM, WN, S, GROUPED, WK>), grid, dim3(64 * WM * WN * WK), lds,
-                       stream, a, reinterpret_cast<const v4u *>(a.X), reinterpret_cast<const v4u *>(a.W), m_blocks, n_blocks);
+                       stream, a, reinterpret_cast<const v4u *>(a.X), reinterpret_cast<const v4u *>(a.W), m_blocks, columns);
     return hipGetLastError();
 }
 

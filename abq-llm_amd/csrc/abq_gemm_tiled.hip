@@ -204,7 +204,7 @@ template <int BITS, int ROWS, int NT, int KB, Int8Mode MODE, bool SUM> struct Op
 // cut the L2 -> L1 traffic per MFMA).
 template <int Q, int P, bool SIGNED, int TM, int TN, bool GROUPED, int KB, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, (WM * WN > 4 ? 1 : (TM * TN <= 4 || KB == 64 ? 2 : 1)))
-void gemm_mfma_tiled(const GemmArgs a, const uint32_t *xt, const uint32_t *wt, int m_blocks, int n_blocks)
+void gemm_mfma_tiled(const GemmArgs a, const uint32_t *xt, const uint32_t *wt, int m_blocks, int columns)
 {
     constexpr int NT = 64 * WM * WN; // threads
     constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
@@ -233,7 +233,7 @@ void gemm_mfma_tiled(const GemmArgs a, const uint32_t *xt, const uint32_t *wt, i
     const int ktiles = __builtin_amdgcn_readfirstlane(a.K) / KB; // stages
 
     int mb, nb;
-    if (!tile_of_workgroup(blockIdx.x, m_blocks, n_blocks, &mb, &nb))
+    if (!tile_of_workgroup(blockIdx.x, m_blocks, columns, &mb, &nb) || nb * BN >= N)
         return; // uniform over the workgroup, before any barrier
     const int m0 = mb * BM, n0 = nb * BN;
 
@@ -458,7 +458,7 @@ static hipError_t launch_mfma_tiled(const GemmArgs &a, hipStream_t stream)
     if (attr != hipSuccess)
         return attr;
     const dim3 grid(tile_grid(m_blocks, n_blocks));
-    hipLaunchKernelGGL((gemm_mfma_tiled<Q, P, SIGNED, TM, TN, GROUPED, KB, WM, WN>), grid, dim3(64 * WM * WN), lds, stream, a, a.X, a.W, m_blocks, n_blocks);
+    hipLaunchKernelGGL((gemm_mfma_tiled<Q, P, SIGNED, TM, TN, GROUPED, KB, WM, WN>), grid, dim3(64 * WM * WN), lds, stream, a, a.X, a.W, m_blocks, tile_columns(m_blocks, n_blocks));
     return hipGetLastError();
 }
 

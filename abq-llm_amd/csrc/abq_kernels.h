@@ -37,6 +37,9 @@ struct GemmArgs {
     // the kernels on prepared operands, unsigned pairs: whether the 8-bit records of X (W) hold codes up to 255
     // (fed as value - 128, with the row sums above) or padded narrower codes, which are fed as they are
     int flip_x, flip_w;
+    // int32 results of the LDS-staged kernel: workgroups that share an output tile, each with its part of K, and add into D,
+    // which holds zeros then; 1: one workgroup per tile, which stores
+    int k_parts;
 };
 
 typedef hipError_t (*GemmLauncher)(const GemmArgs &, hipStream_t);
@@ -121,39 +124,60 @@ inline int decode_grouped_tiled_waves(int K, int w_bits, int group_size)
 // Where whole columns of tiles would give some XCDs a good deal more than their share (tiles_spread), an XCD owns n_blocks / 8 of
 // them, and the tiles of the n_blocks % 8 that are left are dealt out evenly: behind every eight m blocks of its own an XCD takes an
 // eighth of theirs, in runs of consecutive m blocks, whose activations it has just read.
-// Returns false for the workgroups of a grid (tile_grid) that are left without a tile.
 constexpr int kSpreadM = 8;
-// From six rounds of an XCD's 32 compute units on, where the XCD with the most columns has an eighth more than its share: 9 columns
+// Where the XCD with the most columns has at least a round of its 32 compute units, and an eighth, more than its share: 9 columns
 // are 2 for four of the XCDs and none for three (decoder-layer linears, W2A8 groups of 128: hidden 1152 8192 rows 615 -> 581 us, W4A4
 // 535 -> 505; hidden 2176 1476 -> 1392; 12000 rows of 1536 1173 -> 1134).  Below that the tiles dealt out cost what they save: 2048
-// rows of 1408 253 -> 259; W4A4 with one scale, 4096 rows of 1152, 145 -> 150.
-__host__ __device__ __forceinline__ bool tiles_spread(int m_blocks, int n_blocks)
+// rows of 1408 253 -> 259; W4A4 with one scale, 4096 rows of 1152, 145 -> 150; 86 columns of 16 tiles of the FP6 kernel 68.0 -> 70.5.
+inline bool tiles_spread(int m_blocks, int n_blocks)
 {
-    const int most = (n_blocks + 7) / 8;
-    return (long)m_blocks * most > 200 && 8l * 8 * most > 9l * n_blocks;
+    const long most = (n_blocks + 7) / 8;
+    return (8 * most - n_blocks) * m_blocks >= 256 && 8 * 8 * most > 9l * n_blocks;
 }
 
-__device__ __forceinline__ bool tile_of_workgroup(int id, int m_blocks, int n_blocks, int *mb, int *nb)
+// What the kernels are told of the columns of tiles: columns of an XCD, or minus all columns where they are spread.
+inline int tile_columns(int m_blocks, int n_blocks) { return tiles_spread(m_blocks, n_blocks) ? -n_blocks : (n_blocks + 7) / 8; }
+
+// n / d for n below 2^31 and d in 1 .. 4, without a branch
+__device__ __forceinline__ int div_small(int n, int d)
+{
+    const uint32_t m = d == 2 ? 0x80000000u : d == 3 ? 0x55555556u : 0x40000000u; // 2^32 / d, rounded up
+    const int q = (int)(((uint64_t)(uint32_t)n * m) >> 32);
+    return d == 1 ? n : q;
+}
+
+// Returns false for workgroups of a grid (tile_grid) that are left without a tile; a column past the last one (N) has none either.
+// (A division by a number the compiler does not know is some 40 instructions in front of a workgroup's first load; grids of up to four
+// m blocks have none.)
+__device__ __forceinline__ bool tile_of_workgroup(int id, int m_blocks, int columns, int *mb, int *nb)
 {
     constexpr int GM = 4;
     const int xcd = id & 7, slot = id >> 3;
-    const bool spread = tiles_spread(m_blocks, n_blocks);
-    const int npx = spread ? n_blocks >> 3 : (n_blocks + 7) >> 3, left = spread ? n_blocks & 7 : 0;
-    // the m blocks an XCD goes through before it takes its part of what is left: all of them where nothing is
-    const int most = spread ? kSpreadM : m_blocks, sup = slot / (most * npx + left), in = slot - sup * (most * npx + left);
-    const int sm = min(most, m_blocks - sup * most);
+    if (__builtin_expect(columns >= 0, 1)) {
+        const int per_group = GM * columns;
+        const int grp = __builtin_expect(m_blocks > GM, 0) ? slot / per_group : 0, in = slot - grp * per_group;
+        const int gm = min(GM, m_blocks - grp * GM); // the last group may be short
+        const int col = div_small(in, gm);
+        *mb = grp * GM + in - col * gm;
+        *nb = xcd * columns + col;
+        return true;
+    }
+    const int npx = -columns >> 3, left = -columns & 7;
+    const int per_super = kSpreadM * npx + left; // an XCD's tiles of eight m blocks
+    const int sup = slot / per_super, in = slot - sup * per_super;
+    const int sm = min(kSpreadM, m_blocks - sup * kSpreadM); // the last ones may be fewer
     if (in < sm * npx) {
         const int per_group = GM * npx;
-        const int grp = in / per_group, pos = in - grp * per_group;
-        const int gm = min(GM, sm - grp * GM); // the last group may be short
-        *mb = sup * most + grp * GM + pos % gm;
-        *nb = xcd * npx + pos / gm;
-        return *nb < n_blocks;
+        const int grp = in >= per_group ? 1 : 0, pos = in - grp * per_group;
+        const int gm = min(GM, sm - grp * GM), col = div_small(pos, gm);
+        *mb = sup * kSpreadM + grp * GM + pos - col * gm;
+        *nb = xcd * npx + col;
+        return true;
     }
     const int rest = left * sm, u = xcd * ((rest + 7) >> 3) + in - sm * npx;
     if (u >= rest)
         return false;
-    *mb = sup * most + u % sm;
+    *mb = sup * kSpreadM + u % sm;
     *nb = 8 * npx + u / sm;
     return true;
 }

@@ -278,6 +278,28 @@ __device__ __forceinline__ void row_sums_of_four_rows(const uint32_t *__restrict
         sums[row] = (int)total;
 }
 
+// What the workgroups behind those that convert do: rows in fours for the sums (if any), then kClearInts ints each to clear.
+constexpr uint32_t kClearInts = 8192;
+
+__device__ __forceinline__ void relayout_side_job(const uint32_t *planes, int *row_sums, int rows, int KW, int bits, int *clear,
+                                                  uint32_t n_clear, int job)
+{
+    const int sum_jobs = row_sums ? (rows + 3) / 4 : 0;
+    if (job < sum_jobs) {
+        row_sums_of_four_rows(planes, row_sums, rows, KW, bits, job);
+        return;
+    }
+    const size_t first = (size_t)(job - sum_jobs) * kClearInts; // (a job past the last one clears nothing)
+    const bool wide = (reinterpret_cast<size_t>(clear) & 15) == 0;
+    for (size_t i = first + 4 * threadIdx.x; i < first + kClearInts && i < n_clear; i += 4 * 256) {
+        if (wide && i + 4 <= n_clear)
+            *reinterpret_cast<uint4 *>(clear + i) = make_uint4(0u, 0u, 0u, 0u);
+        else
+            for (size_t c = i; c < i + 4 && c < n_clear; ++c)
+                clear[c] = 0;
+    }
+}
+
 // One workgroup converts 32 rows x 8 K tiles.  A thread owns one record (one row, one K tile): it
 // reads 16 bytes per plane (eight threads cover 128 contiguous bytes of a plane row), converts its
 // four word-sets in registers, and parks the record in LDS; the records of one K tile are then
@@ -293,17 +315,18 @@ template <int BITS>
 __global__ __launch_bounds__(256) void relayout_planes_kernel(const uint32_t *__restrict__ planes,
                                                               uint32_t *__restrict__ tiled, int rows, int KW, int in_bits,
                                                               int sign_extend, const float *__restrict__ zero = nullptr,
-                                                              int group_size = 0, int *flag = nullptr, int *__restrict__ row_sums = nullptr)
+                                                              int group_size = 0, int *flag = nullptr, int *__restrict__ row_sums = nullptr,
+                                                              int *__restrict__ clear = nullptr, uint32_t n_clear = 0)
 {
     constexpr int REC = BITS * 4;          // words per record
     constexpr int SLAB = 32 * REC + 4;     // words per K tile in LDS (+16 bytes against bank conflicts)
     __shared__ __align__(16) uint32_t buf[8 * SLAB];
     const int tid = threadIdx.x;
     const int kt_tiles = KW / 4;
-    // row_sums: the grid has further layers of workgroups behind those that convert, which take the rows' sums of codes
-    // from the same planes (one launch instead of two for an operand that needs both)
-    if (row_sums && (int)blockIdx.y >= (kt_tiles + 7) / 8) {
-        row_sums_of_four_rows(planes, row_sums, rows, KW, in_bits, ((int)blockIdx.y - (kt_tiles + 7) / 8) * (int)gridDim.x + (int)blockIdx.x);
+    // row_sums, clear: the grid has further layers of workgroups behind those that convert, which take the rows' sums of codes
+    // from the same planes and clear the result the GEMM will add into (one launch instead of two or three)
+    if ((int)blockIdx.y >= (kt_tiles + 7) / 8) {
+        relayout_side_job(planes, row_sums, rows, KW, in_bits, clear, n_clear, ((int)blockIdx.y - (kt_tiles + 7) / 8) * (int)gridDim.x + (int)blockIdx.x);
         return;
     }
     const int row0 = blockIdx.x * 32, kt0 = blockIdx.y * 8;
@@ -367,15 +390,16 @@ __global__ __launch_bounds__(256) void relayout_planes_kernel(const uint32_t *__
 template <int BITS>
 __global__ __launch_bounds__(256) void relayout_planes_ws_kernel(const uint32_t *__restrict__ planes,
                                                                  uint32_t *__restrict__ tiled, int rows, int KW, int in_bits,
-                                                                 int sign_extend, int *__restrict__ row_sums = nullptr)
+                                                                 int sign_extend, int *__restrict__ row_sums = nullptr,
+                                                                 int *__restrict__ clear = nullptr, uint32_t n_clear = 0)
 {
     constexpr int REC = BITS * 4;          // words per record
     constexpr int SLAB = 8 * REC + 4;      // words per K tile in LDS (+16 bytes against bank conflicts)
     __shared__ __align__(16) uint32_t buf[8 * SLAB];
     const int tid = threadIdx.x;
     const int kt_tiles = KW / 4;
-    if (row_sums && (int)blockIdx.y >= (kt_tiles + 7) / 8) { // (see relayout_planes_kernel)
-        row_sums_of_four_rows(planes, row_sums, rows, KW, in_bits, ((int)blockIdx.y - (kt_tiles + 7) / 8) * (int)gridDim.x + (int)blockIdx.x);
+    if ((int)blockIdx.y >= (kt_tiles + 7) / 8) { // (see relayout_planes_kernel)
+        relayout_side_job(planes, row_sums, rows, KW, in_bits, clear, n_clear, ((int)blockIdx.y - (kt_tiles + 7) / 8) * (int)gridDim.x + (int)blockIdx.x);
         return;
     }
     const int row0 = blockIdx.x * 8, kt0 = blockIdx.y * 8;
@@ -411,20 +435,21 @@ __global__ __launch_bounds__(256) void relayout_planes_ws_kernel(const uint32_t 
 }
 
 // bits: width of the records written; in_bits <= bits: planes the operand has (sign_extend: what the rest repeats)
-// row_sums != nullptr: the rows' sums of codes (as abq_row_sums takes them from the in_bits planes) in the same launch.
+// row_sums != nullptr: the rows' sums of codes (as abq_row_sums takes them from the in_bits planes) in the same launch;
+// clear != nullptr: and n_clear zeros there.
 hipError_t launch_relayout_planes_padded(const uint32_t *planes, uint32_t *tiled, int rows, int k, int bits, int in_bits,
-                                         int sign_extend, hipStream_t stream, int *row_sums)
+                                         int sign_extend, hipStream_t stream, int *row_sums, int *clear, uint32_t n_clear)
 {
     const int KW = k / 32;
     dim3 grid((rows + 31) / 32, (KW / 4 + 7) / 8);
-    const int sum_jobs = row_sums ? (rows + 3) / 4 : 0; // workgroups of four waves, a row each
+    const int sum_jobs = (row_sums ? (rows + 3) / 4 : 0) + (clear ? (int)((n_clear + kClearInts - 1) / kClearInts) : 0); // workgroups
     if ((long)grid.x * grid.y < 256) { // less than a workgroup per compute unit: the finer kernel
         dim3 fine((rows + 7) / 8, (KW / 4 + 7) / 8);
         fine.y += (sum_jobs + fine.x - 1) / fine.x;
         switch (bits) {
 #define ABQ_RELAYOUT_CASE(B)                                                                                     \
     case B:                                                                                                      \
-        hipLaunchKernelGGL(relayout_planes_ws_kernel<B>, fine, dim3(256), 0, stream, planes, tiled, rows, KW, in_bits, sign_extend, row_sums); \
+        hipLaunchKernelGGL(relayout_planes_ws_kernel<B>, fine, dim3(256), 0, stream, planes, tiled, rows, KW, in_bits, sign_extend, row_sums, clear, n_clear); \
         break;
             ABQ_RELAYOUT_CASE(1) ABQ_RELAYOUT_CASE(2) ABQ_RELAYOUT_CASE(3) ABQ_RELAYOUT_CASE(4)
             ABQ_RELAYOUT_CASE(5) ABQ_RELAYOUT_CASE(6) ABQ_RELAYOUT_CASE(7) ABQ_RELAYOUT_CASE(8)
@@ -439,7 +464,7 @@ hipError_t launch_relayout_planes_padded(const uint32_t *planes, uint32_t *tiled
 #define ABQ_RELAYOUT_CASE(B)                                                                                     \
     case B:                                                                                                      \
         hipLaunchKernelGGL(relayout_planes_kernel<B>, grid, dim3(256), 0, stream, planes, tiled, rows, KW, in_bits, sign_extend, \
-                           (const float *)nullptr, 0, (int *)nullptr, row_sums);                                 \
+                           (const float *)nullptr, 0, (int *)nullptr, row_sums, clear, n_clear);                 \
         break;
         ABQ_RELAYOUT_CASE(1) ABQ_RELAYOUT_CASE(2) ABQ_RELAYOUT_CASE(3) ABQ_RELAYOUT_CASE(4)
         ABQ_RELAYOUT_CASE(5) ABQ_RELAYOUT_CASE(6) ABQ_RELAYOUT_CASE(7) ABQ_RELAYOUT_CASE(8)
@@ -472,7 +497,7 @@ hipError_t launch_relayout_planes_folded(const uint32_t *planes, const float *ze
 
 hipError_t launch_relayout_planes(const uint32_t *planes, uint32_t *tiled, int rows, int k, int bits, hipStream_t stream)
 {
-    return launch_relayout_planes_padded(planes, tiled, rows, k, bits, bits, 0, stream, nullptr);
+    return launch_relayout_planes_padded(planes, tiled, rows, k, bits, bits, 0, stream, nullptr, nullptr, 0);
 }
 
 // ---- FP6 records ---------------------------------------------------------------------------

@@ -1,0 +1,78 @@
+"""int32 GEMMs whose K is split over several workgroups per output tile (activations as planes, long K, few tiles): on either side
+of the rule's lines, ragged rows and columns, K tiles that do not divide by the parts, results that held something before."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(96, 1000, 6144), (95, 1000, 6144), (128, 72, 16512), (128, 5440, 7168), (128, 5504, 7168), (200, 200, 13824), (97, 2600, 10880),
+          (512, 640, 8320), (513, 640, 8320)]
+
+
+def operands(abq, q, p, signed, M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    codes = []
+    for rows, bits in ((M, q), (N, p)):
+        lo, hi = (-(1 << (bits - 1)), (1 << (bits - 1)) - 1) if signed else (0, (1 << bits) - 1)
+        c = torch.randint(lo, hi + 1, (rows, K), generator=g, device="cuda", dtype=torch.int32)
+        c[0], c[-1] = lo, hi
+        codes.append(c)
+    return codes
+
+
+def product(x, w):
+    return (x.double() @ w.double().T).long()  # exact: sums below 2^31
+
+
+@pytest.mark.parametrize("q,p,signed", [(8, 8, True), (8, 8, False), (8, 4, True), (8, 4, False), (4, 4, True), (4, 2, False), (2, 2, True)])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_parts_add_up(abq, q, p, signed, M, N, K):
+    x, w = operands(abq, q, p, signed, M, N, K)
+    xd, wd = abq.pack_i32(x, q), abq.pack_i32(w, p)
+    want = product(x, w)
+    kw = {} if signed or 8 not in (q, p) else {"w_row_sums": abq.row_sums(wd)}
+    ws = torch.empty(M * K + 4 * M + 1024, dtype=torch.uint8, device="cuda")
+    weights = [(abq.relayout_planes(wd), kw)]
+    if (q, p, signed) == (8, 8, False):
+        weights.append((abq.relayout_planes_biased(wd), dict(kw, biased=(False, True))))
+    for wt, k in weights:
+        for off in (0, 1):  # a result off 16-byte boundaries as well
+            out = torch.full((M * N + 1,), 7, dtype=torch.int32, device="cuda")[off:off + M * N].view(M, N)
+            g = abq.Gemm(xd, wt, signed, out=out, w_tiled=True, workspace=ws, **k)
+            for _ in range(2):  # (the second run finds the first one's result)
+                assert torch.equal(g.run().long(), want), (g.config_name, off)
+
+
+def test_parts_under_capture(abq):
+    M, N, K = 128, 1024, 8192
+    x, w = operands(abq, 8, 8, True, M, N, K)
+    xd, wt = abq.pack_i32(x, 8), abq.relayout_planes(abq.pack_i32(w, 8))
+    g = abq.Gemm(xd, wt, True, w_tiled=True, workspace=torch.empty(M * K, dtype=torch.uint8, device="cuda"))
+    g.run()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        g.run()
+    for i in range(4):
+        x = x.roll(1, 0)
+        xd.copy_(abq.pack_i32(x, 8))
+        g.out.fill_(i)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(g.out.long(), product(x, w)), i
+        assert torch.equal(g.run().long(), product(x, w))
+
+
+@pytest.mark.parametrize("kind", ["scaled", "tensor"])
+def test_other_epilogues_keep_one_workgroup_per_tile(abq, kind):
+    M, N, K = 128, 512, 8192
+    x, w = operands(abq, 4, 4, True, M, N, K)
+    xd, wt = abq.pack_i32(x, 4), abq.relayout_planes(abq.pack_i32(w, 4))
+    xs, wsc = torch.full((M,), 2.0 ** -8, device="cuda"), torch.full((N,), 0.5, device="cuda")
+    kw = dict(out_kind=abq.OUT_F16_SCALED, x_scale=xs, w_scale=wsc) if kind == "scaled" else dict(
+        out_kind=abq.OUT_F16_TENSOR_F32SCALE, c_scale=torch.full((1,), 2.0 ** -9, device="cuda"))
+    got = abq.Gemm(xd, wt, True, w_tiled=True, workspace=torch.empty(M * K, dtype=torch.uint8, device="cuda"), **kw).run()
+    sums = product(x, w)
+    want = (sums.double() * 2.0 ** -9).half() if kind == "scaled" else sums.float().half() * 2.0 ** -9
+    assert torch.equal(got, want)
