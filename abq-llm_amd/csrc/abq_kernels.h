@@ -225,6 +225,12 @@ __device__ __forceinline__ void quad_transpose_selectors(int quad_lane, uint32_t
 __device__ __forceinline__ float silu(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 
 // ---- output stage shared by all kernels ------------------------------------------------
+// half(acc) * scale, both steps rounding to fp16: out_kind 1 and 3 with the scale at hand
+__device__ __forceinline__ void store_scaled(const GemmArgs &a, int m, int n, int acc, _Float16 scale)
+{
+    reinterpret_cast<_Float16 *>(a.D)[(size_t)m * a.N + n] = (_Float16)(float)acc * scale;
+}
+
 // out_kind values mirror abq_out_kind in include/abq_gemm.h.
 __device__ __forceinline__ void store_result(const GemmArgs &a, int m, int n, int acc)
 {
