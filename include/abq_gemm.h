@@ -507,7 +507,10 @@ abq_status abq_gemm_set_padded_activations(abq_gemm_state *state, int padded);
 /* Workspace needed by abq_gemm_exec if the state ran as ABQ_STRATEGY_TILED, ABQ_STRATEGY_DECODE_TILED
  * (ABQ_STRATEGY_FP6) with its current operand layouts: the converted copies of the operands still in
  * the reference layout.  Operands declared K-tiled (FP6 records) count 0, and so do fp16 activations
- * handed to the decode kernel (ABQ_LAYOUT_F16: quantised inside the kernel, nothing is converted). */
+ * handed to the decode kernel (ABQ_LAYOUT_F16: quantised inside the kernel, nothing is converted).
+ * Unsigned activations of several fields that stay in planes against K-tiled weights of 2 or 4 bits (W2A6), above 16
+ * rows: the bytes of 8-bit records, on which the LDS-staged kernel runs; with a smaller workspace that holds records of
+ * their own width abq_gemm_exec runs the pair's own kernel, slower. */
 size_t abq_gemm_workspace_bytes(const abq_gemm_state *state);
 
 /* Hands a caller-owned device buffer to the state.  If the tile was the library's choice, M > 64
