@@ -101,7 +101,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
     const int rows = min(M, 16);
     const int m0 = blockIdx.y * 16;
     const int Mb = min(16, M - m0);
-    const int once = gridDim.y == 1; // no other workgroup reads this one's weight records
+    const int once = gridDim.y == 1; // no other workgroup reads this one's weight records (XM: always so, its rows are at most sixteen)
     const bool zp = a.w_zero != nullptr;
 
     // LDS: [wave][tile][row][16] partial results | per wave: scales, zero points, group sums of its blocks in flight
@@ -126,7 +126,8 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
         woff[t] = n * (P * 16u) + (uint32_t)g * (4u * P);
         soff[t] = (uint32_t)min((tile0 + t) * 16 + (lane >> 2), N - 1) * (uint32_t)NG;
     }
-    const size_t wstep = (size_t)N * (P * 16u), xstep = (size_t)M * (Q * 16u);
+    using Step = typename std::conditional<XM != 0, uint32_t, size_t>::type; // (records lie within 4 GiB; packed activations: no registers to spare for it)
+    const Step wstep = (Step)N * (P * 16u), xstep = (Step)M * (Q * 16u);
     // activations: chunk `lane` (and 64 + lane) of the rows' records, past the last row's end the last chunk once more
     const uint32_t xoff = (uint32_t)m0 * (Q * 16u) + (uint32_t)min(lane, Mb * Q - 1) * 16u;
     const uint32_t xoff2 = (uint32_t)m0 * (Q * 16u) + (uint32_t)min(64 + lane, Mb * Q - 1) * 16u;
@@ -216,7 +217,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
         // ---- a step's weights and the next one's activations (steps past the end of K repeat the last one) ---------------
         auto k_tile = [&](int i) { return min(S * block_of(i / S) + i % S, KT - 1); };
         auto request_acts = [&](int i) {
-            const char *xp = Xt + (size_t)k_tile(i) * xstep;
+            const char *xp = Xt + (Step)k_tile(i) * xstep;
             if constexpr (XS) {
                 xs[i % XR][0] = dt_load16(xp, xoff);
                 if constexpr (XL > 1)
@@ -226,10 +227,10 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
         auto request = [&](int i) {
             if (i + 1 < NS)
                 request_acts(i + 1);
-            const char *wp = Wt + (size_t)k_tile(i) * wstep;
+            const char *wp = Wt + (Step)k_tile(i) * wstep;
 #pragma unroll
             for (int t = 0; t < T; ++t)
-                wb[i % WB][t].issue(wp, woff[t], once);
+                wb[i % WB][t].template issue<XM != 0>(wp, woff[t], once);
         };
         request_acts(0);
 #pragma unroll
