@@ -93,7 +93,9 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_tiled(const GemmArgs a, i
     // loads it does not know of), and what the result needs put a memory latency behind the last barrier: with the
     // activations requested up here as well, W2A8 x 1 row with a static scale 5.2 -> 4.2 us a GEMM over 4096 x 4096,
     // 11008 x 4096 and 4096 x 11008, W8A8 9.9 -> 9.2.
-    const bool tensor_scale = a.out_kind == 3;
+    // (The scale of the result only with fp16 activations: the instances for packed ones feed the int32 results, where the test
+    // and its branches cost 0.02 us of 4.04 a launch, and gained nothing on W4A4 with a scale.)
+    const bool tensor_scale = XF16 && a.out_kind == 3;
     int *own = red + wid * T * 256;
     const unsigned own_addr = (unsigned)(size_t)own;
     if constexpr (XF16)
@@ -298,8 +300,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_tiled(const GemmArgs a, i
             if (4 * g + e < Mb)
                 red[((wid * T + t) * 16 + 4 * g + e) * 16 + r] = acc[t][0][e] + acc[t][1][e];
     __syncthreads();
-    if (tid < T * 256) {
-        const int t = tid >> 8, rem = tid & 255;
+    for (int o = tid; o < T * 256; o += NT) {
+        const int t = o >> 8, rem = o & 255;
         const int n = (tile0 + t) * 16 + (rem & 15);
         if ((rem >> 4) < Mb && n < N) {
             int part[NW];
@@ -391,11 +393,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_fields(const GemmArgs a, 
     const unsigned xs_addr = (unsigned)(size_t)xs;
     const int xchunks = KT * Mb * QP;
 
-    // the scale of the whole result and the weights' row sums: as in gemm_decode_tiled
-    const bool tensor_scale = a.out_kind == 3;
+    // the weights' row sums: as in gemm_decode_tiled
     int *own = red + wid * 256;
-    if (tensor_scale)
-        lds_dma4(a.C, 0u, (unsigned)(size_t)own);
     if constexpr (FLIP_X)
         lds_dma4(a.w_row_sums, (uint32_t)min(tile0 * 16 + lane, N - 1) * 4u, (unsigned)(size_t)own + 256u);
 
@@ -490,7 +489,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_fields(const GemmArgs a, 
             wb[d] = dt_load16_weights(Wt, weight_offset(t), once);
         }
         if (round == 0) {
-            dt_wait_loads<D>(); // the loads of the scale and the activations are older than these
+            dt_wait_loads<D>(); // the loads of the sums and the activations are older than these
             __syncthreads();
         }
 #pragma unroll
@@ -522,14 +521,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_fields(const GemmArgs a, 
 
     // ---- the waves' partial tiles meet in LDS ----------------------------------------------------------
     static_assert(256 <= NT, "one element per thread");
-    const int out_scale = tensor_scale ? own[0] : 0, w_sum = FLIP_X ? own[64 + (tid & 15)] : 0;
+    const int w_sum = FLIP_X ? own[64 + (tid & 15)] : 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
         if (4 * g + e < Mb)
             red[(wid * 16 + 4 * g + e) * 16 + r] = acc[0][e] + acc[1][e];
     __syncthreads();
-    if (tid < 256) {
-        const int o = tid, n = tile0 * 16 + (o & 15);
+    for (int o = tid; o < 256; o += NT) {
+        const int n = tile0 * 16 + (o & 15);
         if ((o >> 4) < Mb && n < N) {
             int part[NW];
 #pragma unroll
@@ -543,10 +542,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_fields(const GemmArgs a, 
                 v >>= 16 - QP - P;
             if constexpr (FLIP_X)
                 v = (int)((unsigned)v + 128u * (unsigned)w_sum);
-            if (tensor_scale)
-                store_scaled(a, m0 + (o >> 4), n, v, (_Float16)__builtin_bit_cast(float, out_scale));
-            else
-                store_result(a, m0 + (o >> 4), n, v);
+            store_result(a, m0 + (o >> 4), n, v);
         }
     }
 }
