@@ -1879,6 +1879,13 @@ static bool run_unsigned_padded(const abq_gemm_state *st, abq_gemm_state *padded
     return true;
 }
 
+// Whether exec runs the signed pair's entry of the tile: biased records, or unsigned codes that leave the top bit of both
+// operands' records clear.  No sums are needed to choose it.
+static bool signed_entry_runs(const abq_gemm_state *st)
+{
+    return biased_w(st) || (!st->cfg.is_signed && x_plane_bits(st) < st->cfg.x_bits && w_plane_bits(st) < st->cfg.w_bits);
+}
+
 // int32 results of a GEMM whose activations exec converts, on a grid of 128x64 tiles that leaves half of the compute units free,
 // and long K: several workgroups per tile, each with a part of K, add into the result, which the conversion's launch clears
 // (gemm_mfma_staged, KP).  Returns the parts, 1 for a call that runs as its state says; *split is the state on that tile.
@@ -1897,6 +1904,10 @@ static int run_k_parts(const abq_gemm_state *st, abq_gemm_state *split)
     for (int i = 0; t && i < t->count; ++i) {
         const KernelEntry &e = t->entries[i];
         if (e.lds != 0 && e.tm == 2 && e.tn == 1 && e.wm == 2 && e.wn == 2 && e.wk == wk && e.kb == 128) {
+            // (unsigned 8-bit operands without the row sums: the kernel that gathers them itself runs, which has no parts, and
+            // as few tiles as this would leave it on half the compute units)
+            if ((e.flags & kNeedsRowSums) && !signed_entry_runs(st) && !row_sums_at_hand(st))
+                return 1;
             *split = *st;
             split->variant = i;
             return parts;

@@ -137,3 +137,15 @@ def test_no_decode_records_above_128_rows(abq):
             for m in (129, 200, 700, 1400, 5000):
                 assert not abq.prepared_decode_pays(8, p, True, m, n, k, 128)
     assert abq.prepared_decode_pays(8, 4, True, 128, 4096, 4096, 128)
+
+
+@pytest.mark.parametrize("q,p", [(8, 8), (8, 4)])
+def test_k_is_split_over_workgroups_only_where_the_row_sums_are_there(tmp_path, q, p):
+    """Unsigned 8-bit operands without the weights' row sums run the kernel that gathers them, which does not split K: on the tile the
+    library's rules give it."""
+    c = dict(q=q, p=p, signed=0, M=128, N=5120, K=13824, layouts=(0, 1), workspace=1 << 30)
+    without, with_sums = launches(tmp_path, [c, dict(c, row_sums=(0, 0xB00000))])
+    made = without["launches"][-1]
+    assert made["kernel"] == "gemm_mfma_tiled<%d, %d, false, 1, 1, false, 128, 2, 2>" % (q, p), without
+    assert without["tile"] == tile64(q, p, 0, 1) and made["grid"] == without["grid"]
+    assert with_sums["launches"][-1]["kernel"].startswith("gemm_mfma_staged_parts<%d, %d, false, " % (q, p)), with_sums
