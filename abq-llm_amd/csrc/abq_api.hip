@@ -105,6 +105,12 @@ static void set_rows_kernel(abq_gemm_state *st, bool on)
     st->shared_mem_size = plan.lds;
 }
 
+// reserved[4] bits 8 to 11: workgroups that share an output tile of this state, each with a part of K (gemm_mfma_staged_parts);
+// 0: one.  Tile, grid and workgroup are then those of that kernel.  A state moved to another kernel loses them (resolve).
+constexpr int kPartsShift = 8, kPartsMask = 15 << kPartsShift;
+static int k_parts(const abq_gemm_state *st) { return st->reserved[4] & kPartsMask ? (st->reserved[4] & kPartsMask) >> kPartsShift : 1; }
+constexpr int kPartsStage = 8; // NSTAGE of the kernel's tuple
+
 static const Registry &registry()
 {
     static const Registry r;
@@ -217,6 +223,42 @@ static int best_lpr_log2(int K)
     return best;
 }
 
+// The tile that is split over several workgroups along K: 128x64, with two groups of waves for the narrow pairs, whose K tiles are
+// short (W4A4 128 x 5120 x 13824 17.1 against 18.4 us).  Index in the pair's table, or -1.
+static int parts_entry(const KernelTable *t)
+{
+    const int wk = t && t->x_bits + t->w_bits <= 8 ? 2 : 1;
+    for (int i = 0; t && i < t->count; ++i) {
+        const KernelEntry &e = t->entries[i];
+        if (e.lds != 0 && e.tm == 2 && e.tn == 1 && e.wm == 2 && e.wn == 2 && e.wk == wk && e.kb == 128)
+            return i;
+    }
+    return -1;
+}
+
+// Workgroups per output tile there: as many as fill the chip with parts that are long enough (shorter ones lose to the second pass
+// over the result what they gain: k_parts_pay has the figures), at most eight.  Below two the tile is not split.
+static int k_parts_that_fit(int x_bits, int w_bits, int M, int N, int K)
+{
+    const long tiles = (long)((M + 127) / 128) * ((N + 63) / 64);
+    const long fit = 256 / tiles, long_enough = K / 128 / (x_bits == 8 && w_bits == 8 ? 16 : 28), parts = fit < long_enough ? fit : long_enough;
+    return parts < 2 ? 1 : parts > 8 ? 8 : (int)parts;
+}
+
+// Puts a state on that tile.
+static void set_k_parts(abq_gemm_state *st, const KernelTable *t, int variant, int parts)
+{
+    const KernelEntry &e = t->entries[variant];
+    st->strategy = ABQ_STRATEGY_TILED;
+    st->variant = variant;
+    entry_to_config(e, ABQ_STRATEGY_TILED, t->x_bits, t->w_bits, t->is_signed, 0, &st->cfg);
+    st->cfg.nstage = kPartsStage;
+    st->reserved[4] = (st->reserved[4] & ~kPartsMask) | parts << kPartsShift;
+    st->grid_dim = abq_dim3{ tile_grid((st->M + 127) / 128, (st->N + 63) / 64) * (unsigned)parts, 1, 1 };
+    st->block_dim = abq_dim3{ (unsigned)(64 * e.wm * e.wn * e.wk), 1, 1 };
+    st->shared_mem_size = e.lds;
+}
+
 static int find_mfma_variant(const KernelTable &t, int mi, int tm, int tn, int wm, int wn, int wk)
 {
     for (int i = 0; i < t.count; ++i) {
@@ -292,7 +334,25 @@ static abq_status resolve(const abq_tile_config *cfg, int x_bits, int w_bits, in
 {
     const Registry &reg = registry();
     int strategy = cfg ? strategy_of_mma(*cfg) : ABQ_STRATEGY_AUTO;
-    st->reserved[4] &= ~kRowsKernel;
+    st->reserved[4] &= ~(kRowsKernel | kPartsMask);
+    if (strategy == ABQ_STRATEGY_MFMA32 && cfg->nstage == kPartsStage) {
+        // the tile that is split along K, asked for by name: it runs once the activations' layout and a workspace are declared
+        const KernelTable *t = find_table(reg.tiled, x_bits, w_bits, is_signed);
+        const int v = parts_entry(t), parts = k_parts_that_fit(x_bits, w_bits, M, N, K);
+        if (v < 0 || parts < 2)
+            return ABQ_ERR_UNSUPPORTED;
+        abq_gemm_state on = *st;
+        on.M = M;
+        on.N = N;
+        on.K = K;
+        set_k_parts(&on, t, v, parts);
+        if (memcmp(cfg, &on.cfg, sizeof on.cfg) != 0)
+            return ABQ_ERR_UNSUPPORTED;
+        if (K >= (1 << 17))
+            return ABQ_ERR_TOO_LARGE;
+        *st = on;
+        return ABQ_OK;
+    }
     if (strategy == ABQ_STRATEGY_MFMA16 && cfg->nstage == kRowsStage) {
         // the kernel for 17 rows and more asked for by name: it carries group scales only, so the state runs once they are set
         const abq_tile_config want = rows_config(x_bits, w_bits);
@@ -741,6 +801,8 @@ abq_status abq_gemm_init(const abq_tile_config *cfg, int x_bits, int w_bits, int
     abq_status s = resolve(cfg, x_bits, w_bits, is_signed, M, N, K, state);
     if (s != ABQ_OK)
         return s;
+    if (k_parts(state) > 1 && out_kind != ABQ_OUT_I32) // (its workgroups add int32 sums)
+        return ABQ_ERR_UNSUPPORTED;
     state->M = M;
     state->N = N;
     state->K = K;
@@ -1441,11 +1503,73 @@ static void apply_tuned(abq_gemm_state *st)
         *st = tmp;
 }
 
+// Parts of K for an int32 GEMM on 128x64 tiles (gemm_mfma_staged, KP), 1 where that does not pay.  Measured with the conversion
+// of the activations in the call and weights from memory, us on the tile that ran before / in parts:
+//   W8A8  128 x 5120 x 13824 32.6 / 26.1, 128 x 4096 x 11008 27.6 / 20.7, 128 x 2048 x 8192 16.7 / 13.3 (unsigned 22.1 / 14.5),
+//         100 x 4096 x 6144 16.6 / 14.4, 256 x 2560 x 11008 28.7 / 23.0, 512 x 1024 x 8192 19.3 / 19.2; 1024 x 512 x 8192 21.6 / 23.8
+//   W4A8  128 x 5120 x 13824 27.5 / 23.0, 128 x 2048 x 16384 23.8 / 18.0;  W4A4 22.6 / 21.4;  W2A2 128 x 4096 x 11008 17.3 / 15.9
+// Two parts (86 to 128 tiles) move as many bytes per compute unit as the 64x64 tile did: 512 x 2048 x 8192 W8A8 21.9 / 24.0, W2A2
+// 17.0 / 19.5.  Shorter parts lose to the second pass over the result what they gain: W8A8 below 16 K tiles (128 x 5120 x 5120
+// 16.7 / 16.8 in three), the others below 28 (W4A8 100 x 4096 x 6144 13.9 / 14.1 in two).  W2A8 is as fast on its 64x64 tile with four
+// K groups (128 x 5120 x 13824 23.0 / 23.4).
+static int k_parts_that_pay(int x_bits, int w_bits, int M, int N, int K)
+{
+    const int m_blocks = (M + 127) / 128, parts = k_parts_that_fit(x_bits, w_bits, M, N, K);
+    return parts < 3 || m_blocks > 4 || M * 4l < m_blocks * 128 * 3 || (x_bits == 8 && w_bits == 2) ? 1 : parts;
+}
+
+// Whether the kernel that runs for a TILED state on entry e wants the row sums: biased records, and unsigned 8-bit operands unless their
+// codes leave the top bit of both operands' records clear (the signed pair's kernel then runs).
+static bool runs_on_row_sums(const abq_gemm_state *st, const KernelEntry &e)
+{
+    const bool narrow = !st->cfg.is_signed && x_plane_bits(st) < st->cfg.x_bits && w_plane_bits(st) < st->cfg.w_bits;
+    return biased_w(st) || ((e.flags & kNeedsRowSums) && !narrow);
+}
+
+// int32 results of a GEMM whose activations exec converts: several workgroups per tile, each with a part of K, may add into the
+// result, which the conversion's launch clears (gemm_mfma_staged, KP).  Unsigned 8-bit operands without their row sums run the kernel
+// that gathers them itself, which has no parts.
+static bool may_split_k(const abq_gemm_state *st)
+{
+    if (st->strategy != ABQ_STRATEGY_TILED || !st->auto_chosen || st->out_kind != ABQ_OUT_I32 || st->group_size || st->act ||
+        st->x_layout != ABQ_LAYOUT_PLANES || st->w_layout != ABQ_LAYOUT_TILED)
+        return false;
+    const KernelTable *t = find_table(registry().tiled, st->cfg.x_bits, st->cfg.w_bits, st->cfg.is_signed);
+    const int v = parts_entry(t);
+    return v >= 0 && (!runs_on_row_sums(st, t->entries[v]) || row_sums_at_hand(st));
+}
+
+// What a state runs follows from everything that has been declared of it: each declaration takes the last of these decisions back
+// (unsettle), does its own part, and has it made again (settle).
+static void unsettle(abq_gemm_state *st)
+{
+    if (st->auto_chosen && k_parts(st) > 1)
+        (void)switch_to_tiled(st); // (the tile of the rules, which the state was on)
+}
+
+static void settle(abq_gemm_state *st)
+{
+    if (!may_split_k(st))
+        return;
+    const abq_tile_config &c = st->cfg;
+    const KernelTable *t = find_table(registry().tiled, c.x_bits, c.w_bits, c.is_signed);
+    const int parts = k_parts_that_pay(c.x_bits, c.w_bits, st->M, st->N, st->K);
+    if (parts > 1)
+        set_k_parts(st, t, parts_entry(t), parts);
+}
+
+struct Declaration {
+    abq_gemm_state *st;
+    explicit Declaration(abq_gemm_state *state) : st(state) { unsettle(st); }
+    ~Declaration() { settle(st); }
+};
+
 abq_status abq_gemm_set_scales(abq_gemm_state *state, const float *x_scale, const float *w_scale,
                                int group_size)
 {
     if (!state || !state->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(state);
     if (!x_scale || !w_scale)
         return ABQ_ERR_INVALID_ARG;
     if (group_size != 0) {
@@ -1499,6 +1623,7 @@ abq_status abq_gemm_set_zero_points(abq_gemm_state *state, const float *x_zero, 
 {
     if (!state || !state->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(state);
     if (state->group_size == 0) // only the group-scale kernel carries the correction terms
         return ABQ_ERR_UNSUPPORTED;
     const bool x_dynamic = state->x_layout == ABQ_LAYOUT_F16 && state->reserved[1] != 0; // sums and zero points made in the kernel
@@ -1517,6 +1642,7 @@ abq_status abq_gemm_set_activation(abq_gemm_state *state, int act)
 {
     if (!state || !state->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(state);
     if (act != ABQ_ACT_NONE && act != ABQ_ACT_SILU_GATE)
         return ABQ_ERR_INVALID_ARG;
     if (act == ABQ_ACT_SILU_GATE) {
@@ -1628,8 +1754,16 @@ abq_status abq_gemm_exec_static(const abq_gemm_state *st, void *stream)
         const abq_status rc = static_scratch_address(&ptr);
         if (rc != ABQ_OK)
             return rc;
-        local.workspace = ptr;
-        local.workspace_bytes = ABQ_STATIC_WORKSPACE_BYTES;
+        auto take = [&]() {
+            local.workspace = ptr;
+            local.workspace_bytes = ABQ_STATIC_WORKSPACE_BYTES;
+        };
+        if (local.cfg.is_signed) {
+            take();
+        } else { // (row sums may be had from the planes now)
+            const Declaration declaration(&local);
+            take();
+        }
     }
     return abq_gemm_exec(&local, stream);
 }
@@ -1739,6 +1873,7 @@ abq_status abq_gemm_set_row_sums(abq_gemm_state *st, const int32_t *x_row_sums, 
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(st);
     st->x_row_sums = x_row_sums;
     st->w_row_sums = w_row_sums;
     reconsider_decode_tiled(st);
@@ -1749,6 +1884,7 @@ abq_status abq_gemm_set_value_bits(abq_gemm_state *st, int x_value_bits, int w_v
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(st);
     if (x_value_bits < 1 || x_value_bits > st->cfg.x_bits || w_value_bits < 1 || w_value_bits > st->cfg.w_bits)
         return ABQ_ERR_INVALID_ARG;
     st->reserved[2] = x_value_bits;
@@ -1761,6 +1897,7 @@ abq_status abq_gemm_set_padded_activations(abq_gemm_state *st, int padded)
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(st);
     if (padded && one_field(st->cfg.x_bits))
         padded = 0; // records of one field are their own padding
     st->reserved[4] = (st->reserved[4] & ~4) | (padded ? 4 : 0);
@@ -1784,6 +1921,7 @@ abq_status abq_gemm_set_biased_records(abq_gemm_state *st, int x_biased, int w_b
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(st);
     if ((x_biased || w_biased) && (st->cfg.is_signed || st->cfg.x_bits != 8 || st->cfg.w_bits != 8 || st->group_size))
         return ABQ_ERR_UNSUPPORTED;
     if (x_biased && !w_biased)
@@ -1831,25 +1969,6 @@ abq_status abq_relayout_planes_folded(const uint32_t *planes, const float *w_zer
                                                     is_signed ? 1 : 0, misfit_dev, (hipStream_t)stream));
 }
 
-// Parts of K for an int32 GEMM on 128x64 tiles (gemm_mfma_staged, KP), 1 where that does not pay.  Measured with the conversion
-// of the activations in the call and weights from memory, us on the tile that ran before / in parts:
-//   W8A8  128 x 5120 x 13824 32.6 / 26.1, 128 x 4096 x 11008 27.6 / 20.7, 128 x 2048 x 8192 16.7 / 13.3 (unsigned 22.1 / 14.5),
-//         100 x 4096 x 6144 16.6 / 14.4, 256 x 2560 x 11008 28.7 / 23.0, 512 x 1024 x 8192 19.3 / 19.2; 1024 x 512 x 8192 21.6 / 23.8
-//   W4A8  128 x 5120 x 13824 27.5 / 23.0, 128 x 2048 x 16384 23.8 / 18.0;  W4A4 22.6 / 21.4;  W2A2 128 x 4096 x 11008 17.3 / 15.9
-// Two parts (86 to 128 tiles) move as many bytes per compute unit as the 64x64 tile did: 512 x 2048 x 8192 W8A8 21.9 / 24.0, W2A2
-// 17.0 / 19.5.  Shorter parts lose to the second pass over the result what they gain: W8A8 below 16 K tiles (128 x 5120 x 5120
-// 16.7 / 16.8 in three), the others below 28 (W4A8 100 x 4096 x 6144 13.9 / 14.1 in two).  W2A8 is as fast on its 64x64 tile with four
-// K groups (128 x 5120 x 13824 23.0 / 23.4).
-static int k_parts_of_shape(int x_bits, int w_bits, int M, int N, int K)
-{
-    const bool w8a8 = x_bits == 8 && w_bits == 8;
-    const long m_blocks = (M + 127) / 128, tiles = m_blocks * ((N + 63) / 64);
-    if (m_blocks > 4 || tiles > 85 || M * 4l < m_blocks * 128 * 3 || (x_bits == 8 && w_bits == 2))
-        return 1;
-    const long fit = 256 / tiles, long_enough = K / 128 / (w8a8 ? 16 : 28), parts = fit < long_enough ? fit : long_enough;
-    return parts < 3 ? 1 : parts > 8 ? 8 : (int)parts;
-}
-
 // Unsigned activations of several fields that arrive as planes, against K-tiled weights of one narrower field, on the
 // library's own choice of tile: exec converts the activations anyway, and as records of the next single-field width (their
 // codes stay below 128: no value - 128, no row sums) they run on the LDS-staged kernel, where the odd widths' own kernel is
@@ -1879,43 +1998,6 @@ static bool run_unsigned_padded(const abq_gemm_state *st, abq_gemm_state *padded
     return true;
 }
 
-// Whether exec runs the signed pair's entry of the tile: biased records, or unsigned codes that leave the top bit of both
-// operands' records clear.  No sums are needed to choose it.
-static bool signed_entry_runs(const abq_gemm_state *st)
-{
-    return biased_w(st) || (!st->cfg.is_signed && x_plane_bits(st) < st->cfg.x_bits && w_plane_bits(st) < st->cfg.w_bits);
-}
-
-// int32 results of a GEMM whose activations exec converts, on a grid of 128x64 tiles that leaves half of the compute units free,
-// and long K: several workgroups per tile, each with a part of K, add into the result, which the conversion's launch clears
-// (gemm_mfma_staged, KP).  Returns the parts, 1 for a call that runs as its state says; *split is the state on that tile.
-static int run_k_parts(const abq_gemm_state *st, abq_gemm_state *split)
-{
-    const abq_tile_config &c = st->cfg;
-    if (st->strategy != ABQ_STRATEGY_TILED || !st->auto_chosen || st->out_kind != ABQ_OUT_I32 || st->group_size || st->act ||
-        st->x_layout != ABQ_LAYOUT_PLANES || st->w_layout != ABQ_LAYOUT_TILED)
-        return 1;
-    const int parts = k_parts_of_shape(c.x_bits, c.w_bits, st->M, st->N, st->K);
-    if (parts < 2)
-        return 1;
-    const KernelTable *t = find_table(registry().tiled, c.x_bits, c.w_bits, c.is_signed);
-    // (two groups of waves in a workgroup for the narrow pairs, whose K tiles are short: W4A4 128 x 5120 x 13824 17.1 against 18.4 us)
-    const int wk = c.x_bits + c.w_bits <= 8 ? 2 : 1;
-    for (int i = 0; t && i < t->count; ++i) {
-        const KernelEntry &e = t->entries[i];
-        if (e.lds != 0 && e.tm == 2 && e.tn == 1 && e.wm == 2 && e.wn == 2 && e.wk == wk && e.kb == 128) {
-            // (unsigned 8-bit operands without the row sums: the kernel that gathers them itself runs, which has no parts, and
-            // as few tiles as this would leave it on half the compute units)
-            if ((e.flags & kNeedsRowSums) && !signed_entry_runs(st) && !row_sums_at_hand(st))
-                return 1;
-            *split = *st;
-            split->variant = i;
-            return parts;
-        }
-    }
-    return 1;
-}
-
 abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
 {
     if (!st || !st->init_success)
@@ -1923,10 +2005,6 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
     abq_gemm_state padded;
     if (run_unsigned_padded(st, &padded))
         st = &padded;
-    abq_gemm_state split;
-    const int k_parts = run_k_parts(st, &split);
-    if (k_parts > 1)
-        st = &split;
     const bool x_dynamic = st->x_layout == ABQ_LAYOUT_F16 && st->reserved[1] != 0; // the kernel takes the token scales itself
     if (st->out_kind == ABQ_OUT_F16_SCALED && ((!st->x_scale && !x_dynamic) || !st->w_scale))
         return ABQ_ERR_INVALID_ARG;
@@ -1954,9 +2032,7 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
     a.x_row_sums = nullptr; // (handed to a kernel only by the branches below that need them)
     a.w_row_sums = nullptr;
     decode_tiled_flips(st, &a.flip_x, &a.flip_w);
-    a.k_parts = k_parts;
-    int *clear = k_parts > 1 ? static_cast<int *>(st->D) : nullptr; // the result several workgroups will add into
-    const uint32_t n_clear = k_parts > 1 ? (uint32_t)((size_t)st->M * st->N) : 0;
+    a.k_parts = 1;
     const Registry &reg = registry();
     const abq_tile_config &c = st->cfg;
     hipError_t e;
@@ -2027,6 +2103,15 @@ abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
         const bool rows = st->group_size && rows_kernel(st);
         if (!t || (!rows && (st->variant < 0 || st->variant >= t->count)))
             return ABQ_ERR_NOT_INITIALIZED;
+        // Several workgroups per output tile add into the result, which the conversion's launch clears.  (A tile asked for by name may
+        // lack the sums: the kernel that gathers them itself stores.)
+        int *clear = nullptr;
+        uint32_t n_clear = 0;
+        if (k_parts(st) > 1 && xb && (!runs_on_row_sums(st, t->entries[st->variant]) || row_sum_plan(st, xb + wb).ok)) {
+            a.k_parts = k_parts(st);
+            clear = static_cast<int *>(st->D);
+            n_clear = (uint32_t)((size_t)st->M * st->N);
+        }
         // Activations that arrive as planes and whose row sums a branch below will take from those planes: the
         // conversion's launch takes the sums as well (further workgroups of the same grid), where that branch puts them.
         bool x_sums_taken = false;
@@ -2275,6 +2360,7 @@ abq_status abq_gemm_set_operand_layout(abq_gemm_state *st, int x_layout, int w_l
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(st);
     abq_gemm_state next = *st; // the caller's state changes only if the declaration is taken
     abq_status rc = set_operand_layout_by_rules(&next, x_layout, w_layout);
     // Activations of several fields that arrive as planes, against K-tiled weights of one field: exec converts the
@@ -2314,6 +2400,8 @@ static abq_status set_operand_layout_by_rules(abq_gemm_state *st, int x_layout, 
     const bool any_tiled = x_layout == ABQ_LAYOUT_TILED || w_layout == ABQ_LAYOUT_TILED;
     if (any_fp6 && any_tiled)
         return ABQ_ERR_UNSUPPORTED;
+    if (k_parts(st) > 1 && x_layout != ABQ_LAYOUT_PLANES)
+        return ABQ_ERR_UNSUPPORTED; // (asked for by name: the launch that converts the activations clears the result)
     if (any_fp6 && st->strategy != ABQ_STRATEGY_FP6) {
         if (!st->auto_chosen)
             return ABQ_ERR_UNSUPPORTED;
@@ -2413,6 +2501,7 @@ abq_status abq_gemm_set_workspace(abq_gemm_state *st, void *workspace, size_t by
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    const Declaration declaration(st);
     if (!workspace && bytes)
         return ABQ_ERR_INVALID_ARG;
     st->workspace = workspace;

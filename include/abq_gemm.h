@@ -89,7 +89,11 @@ abq_status abq_pack_f16(const void *in_f16, const float *scale_dev, uint32_t *pl
  *   32 x 32 x 32  the same feeding v_mfma_i32_32x32x32_i8 (NSTAGE = 4: LDS-staged kernels on K-tiled
  *                 operands, WK = 128 (or 64) = K elements per LDS stage and group of waves; BK = 2 WK:
  *                 two groups of waves share the tile and split K between them, for small grids; BK = 4 WK:
- *                 four groups, the 64 x 64 tile of pairs of 2-, 4- and 8-bit fields other than W8A8)
+ *                 four groups, the 64 x 64 tile of pairs of 2-, 4- and 8-bit fields other than W8A8; NSTAGE = 8,
+ *                 128x64 with BK = WK, or 2 WK for pairs of at most 8 bits together: K in parts, several workgroups
+ *                 per output tile, which add int32 results into D.  Runs on activations in planes, whose conversion
+ *                 clears D, from 2 parts on of 28 K tiles of 128 (W8A8: 16) that fit the chip's 256 compute units
+ *                 side by side; not part of the native tile space)
  * Any other triple (the reference's 8x8x128, 16x8x128, 16x8x256 tensor-core shapes) asks the
  * library to choose strategy and tile itself from (bits, M, N, K).
  * ------------------------------------------------------------------------------------- */
@@ -189,7 +193,9 @@ typedef struct abq_gemm_state {
                               abq_gemm_set_dynamic_f16_activations; [2], [3] see abq_gemm_set_value_bits; [4] bits 0, 1 see
                               abq_gemm_set_biased_records, bit 2 abq_gemm_set_padded_activations, bit 4: the NSTAGE 7 kernel
                               runs (cfg is then that of the tile it stands in for, or its own if asked for;
-                              grid_dim, block_dim and shared_mem_size are its own) */
+                              grid_dim, block_dim and shared_mem_size are its own); bits 8 to 11: parts of K (NSTAGE 8),
+                              0 for one.  D is then cleared first and added into: while a call is under way nothing else may
+                              write or read it, another call on the same state included */
     /* K-tiled operands (ABQ_STRATEGY_TILED) */
     int x_layout, w_layout;  /* abq_layout of X and W as handed to init                    */
     int auto_chosen;         /* 1 if the tile was the library's choice                     */

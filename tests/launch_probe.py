@@ -11,7 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 def launches(tmp_path, calls):
     """calls: dicts of q, p, signed, M, N, K and optionally tile (a kernel name), layouts, group, zeros, act, row_sums, value_bits,
-    workspace, tuning (lines of a tuning table).  Returns a list of dicts: status, tile, strategy, grid, block, lds, launches."""
+    workspace, tuning (lines of a tuning table), order (of the declarations), then (further ones: [what, value]).  Returns a list of dicts: status, tile, strategy, grid, block, lds, launches."""
     so = str(tmp_path / "librecorder.so")
     if not os.path.exists(so):
         subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", os.path.join(HERE, "cpp", "launch_recorder.cpp"), "-o", so])
@@ -41,17 +41,21 @@ def main():
         tile = abq.parse_kernel_name(c["tile"])[0] if c.get("tile") else None
         group = c.get("group", 0)
         rc = [L.abq_gemm_init(ctypes.byref(tile) if tile else None, c["q"], c["p"], c["signed"], 0x100000, 0x200000, c["M"], c["N"], c["K"],
-                              0x300000, None, 0, abq.OUT_F16_SCALED if group else abq.OUT_I32, s)]
+                              0x300000, 0x380000, 0, abq.OUT_F16_SCALED if group else c.get("out_kind", abq.OUT_I32), s)]
         steps = {"value_bits": lambda: L.abq_gemm_set_value_bits(s, *c["value_bits"]) if "value_bits" in c else 0,
                  "layouts": lambda: L.abq_gemm_set_operand_layout(s, *c.get("layouts", (abq.LAYOUT_TILED, abq.LAYOUT_TILED))),
                  "row_sums": lambda: L.abq_gemm_set_row_sums(s, *c["row_sums"]) if "row_sums" in c else 0,
-                 "scales": lambda: L.abq_gemm_set_scales(s, 0x400000, 0x500000, group) if group else 0,
+                 "scales": lambda: L.abq_gemm_set_scales(s, 0x400000, 0x500000, group) if group or c.get("out_kind") == abq.OUT_F16_SCALED else 0,
                  "zeros": lambda: L.abq_gemm_set_zero_points(s, 0x600000, 0x700000, 0x800000, 0x900000) if c.get("zeros") else 0,
                  "act": lambda: L.abq_gemm_set_activation(s, c["act"]) if c.get("act") else 0,
                  "workspace": lambda: L.abq_gemm_set_workspace(s, 0xA00000, c["workspace"]) if c.get("workspace") else 0}
         for step in c.get("order", list(steps)):
             if rc[-1] == 0:
                 rc.append(steps[step]())
+        for what, value in c.get("then", []):
+            c = dict(c, **{what: value})
+            if rc[-1] == 0:
+                rc.append(steps[what]())
         rec.recorder_clear()
         if rc[-1] == 0:
             rc.append(L.abq_gemm_exec(s, None))

@@ -149,3 +149,63 @@ def test_k_is_split_over_workgroups_only_where_the_row_sums_are_there(tmp_path, 
     assert made["kernel"] == "gemm_mfma_tiled<%d, %d, false, 1, 1, false, 128, 2, 2>" % (q, p), without
     assert without["tile"] == tile64(q, p, 0, 1) and made["grid"] == without["grid"]
     assert with_sums["launches"][-1]["kernel"].startswith("gemm_mfma_staged_parts<%d, %d, false, " % (q, p)), with_sums
+
+
+def parts_tile(q, p, signed):
+    return "AqBMMA_%dx%dx%s_128x64x%d_64x32x128_32x32x32_8" % (q, p, "true" if signed else "false", 256 if q + p <= 8 else 128)
+
+
+def split(r):
+    """workgroups per output tile of the call's GEMM, None if one that the state does not describe ran"""
+    convert, made = r["launches"]
+    if r["status"] or (made["grid"], made["block"], made["lds"]) != (r["grid"], r["block"], r["lds"]) or not convert["kernel"].startswith("relayout_planes"):
+        return None
+    parts = made["kernel"].startswith("gemm_mfma_staged_parts<")
+    return made["grid"][0] // (8 * -(-r["N"] // 512) * -(-r["M"] // 128)) if parts else 1
+
+
+# (rows, columns, K) -> parts per pair, on either side of the rule's lines: three quarters of the blocks of rows, four of them, 85 tiles, K tiles
+# per part, eight parts
+SPLITS = [((192, 200, 13824), {(8, 8): 6, (8, 4): 3, (4, 4): 3, (4, 2): 3, (2, 2): 3, (8, 2): 1}), ((191, 200, 13824), {(8, 8): 1, (8, 4): 1, (4, 4): 1, (2, 2): 1}),
+          ((512, 640, 8320), {(8, 8): 4, (8, 4): 1}), ((513, 640, 8320), {(8, 8): 1}), ((128, 5440, 7168), {(8, 8): 3, (8, 4): 1}), ((128, 5504, 7168), {(8, 8): 1}),
+          ((200, 200, 10752), {(8, 8): 5, (8, 4): 3, (4, 4): 3, (2, 2): 3}), ((200, 200, 10624), {(8, 8): 5, (8, 4): 1, (4, 4): 1, (2, 2): 1}),
+          ((256, 64, 16512), {(8, 8): 8, (8, 4): 4, (4, 4): 4}), ((97, 2600, 10880), {(8, 8): 5, (8, 4): 3})]
+
+
+@pytest.mark.parametrize("signed", [1, 0])
+def test_states_on_parts_of_k_describe_the_kernel_that_runs(tmp_path, signed):
+    cases = [(parts, dict(q=q, p=p, signed=signed, M=m, N=n, K=k, layouts=(0, 1), workspace=1 << 30, **({} if signed or 8 not in (q, p) else {"row_sums": (0, 0xB00000)})))
+             for (m, n, k), pairs in SPLITS for (q, p), parts in pairs.items()]
+    orders = [["layouts", "row_sums", "workspace"], ["row_sums", "workspace", "layouts"], ["workspace", "layouts", "row_sums"]]
+    cases = [(parts, dict(c, order=o)) for parts, c in cases for o in orders]
+    for (parts, c), r in zip(cases, launches(tmp_path, [c for _, c in cases])):
+        assert split(dict(r, **c)) == parts, (c, r)
+        assert (r["tile"] == parts_tile(c["q"], c["p"], signed)) == (parts > 1), (c, r)
+
+
+def test_parts_of_k_are_left_again(tmp_path):
+    """A state on that tile moves back when a later declaration takes away what it needs."""
+    c = dict(q=8, p=8, signed=0, M=128, N=5120, K=13824, layouts=(0, 1), workspace=1 << 30, row_sums=(0, 0xB00000))
+    sums_gone, both_tiled = launches(tmp_path, [dict(c, then=[["row_sums", [0, 0]]]), dict(c, signed=1, then=[["layouts", [1, 1]]])])
+    assert sums_gone["tile"] == tile64(8, 8, 0, 1) and sums_gone["launches"][-1]["kernel"].startswith("gemm_mfma_tiled<8, 8, false, 1, 1, ")
+    assert runs_what_it_says(both_tiled) and both_tiled["tile"] == tile64(8, 8, 1, 1)
+
+
+def test_parts_of_k_run_by_name(tmp_path):
+    ask = lambda q, p, signed, **c: dict(dict(q=q, p=p, signed=signed, M=128, N=5120, K=13824, tile=parts_tile(q, p, signed), layouts=(0, 1),  # noqa: E731
+                                              workspace=1 << 30), **c)
+    sums = {"row_sums": (0, 0xB00000)}
+    cases = [(3, ask(8, 8, 1)), (3, ask(8, 2, 1)), (3, ask(4, 2, 0)), (3, ask(8, 4, 0, **sums)), (2, ask(8, 8, 1, M=256, N=4096, K=4096)), (8, ask(4, 4, 1, M=3, N=64, K=28672))]
+    for (parts, c), r in zip(cases, launches(tmp_path, [c for _, c in cases])):
+        assert split(dict(r, **c)) == parts and r["tile"] == c["tile"], (c, r)
+    plain, narrow, short, wide, odd, records, scaled, fp16 = launches(tmp_path, [
+        ask(8, 8, 0), ask(8, 8, 1, tile=parts_tile(8, 8, 1).replace("128x64x128", "128x64x256")), ask(8, 8, 1, K=3968), ask(8, 8, 1, M=2048), ask(6, 6, 1),
+        ask(8, 8, 1, layouts=(1, 1)), ask(8, 8, 1, group=128), ask(8, 8, 1, out_kind=3)])
+    assert plain["status"] == 0 and plain["launches"][-1]["kernel"] == "gemm_mfma_tiled<8, 8, false, 2, 1, false, 128, 2, 2>"  # (no sums: the same tile, one part)
+    assert [r["status"] for r in (narrow, short, wide, odd, records, scaled, fp16)] == [3] * 7
+
+
+@pytest.mark.parametrize("out_kind", [1, 2, 3])
+def test_halves_are_never_added_in_parts(tmp_path, out_kind):
+    (r,) = launches(tmp_path, [dict(q=8, p=8, signed=1, M=128, N=5120, K=13824, layouts=(0, 1), workspace=1 << 30, out_kind=out_kind)])
+    assert r["tile"] == tile64(8, 8, 1, 1) and r["launches"][-1]["kernel"].startswith("gemm_mfma_staged<") and r["grid"] == [160, 1, 1]
