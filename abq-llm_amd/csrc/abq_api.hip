@@ -109,7 +109,6 @@ static void set_rows_kernel(abq_gemm_state *st, bool on)
 // 0: one.  Tile, grid and workgroup are then those of that kernel.  A state moved to another kernel loses them (resolve).
 constexpr int kPartsShift = 8, kPartsMask = 15 << kPartsShift;
 static int k_parts(const abq_gemm_state *st) { return st->reserved[4] & kPartsMask ? (st->reserved[4] & kPartsMask) >> kPartsShift : 1; }
-constexpr int kPartsStage = 8; // NSTAGE of the kernel's tuple
 
 static const Registry &registry()
 {
@@ -1473,31 +1472,42 @@ static abq_status pick_grouped_tiled(abq_gemm_state *state)
     return ABQ_OK;
 }
 
-// Looks the state's GEMM up in the table of measured best tiles (abq_tuning.hip) and, if it holds a tile that runs
-// on the operand layouts the state has now, moves the state to that tile.  Only states whose tile is the library's
-// choice; group-scale states are looked up where their tile is picked (pick_grouped_tiled).
-static void apply_tuned(abq_gemm_state *st)
+static bool may_split_k(const abq_gemm_state *st);
+
+// Looks the state's GEMM up in the table of measured best tiles (abq_tuning.hip): the tile it holds, if it runs on the operand layouts
+// the state has now.  Only states whose tile is the library's choice; group-scale states are looked up where their tile is picked
+// (pick_grouped_tiled).
+static bool tuned_tile(const abq_gemm_state *st, TunedTile *t)
 {
     if (!st->auto_chosen || st->act || st->group_size || st->x_layout == ABQ_LAYOUT_F16)
-        return;
+        return false;
     const abq_tile_config &c = st->cfg;
     const bool any_fp6 = st->x_layout == ABQ_LAYOUT_FP6 || st->w_layout == ABQ_LAYOUT_FP6;
     const bool any_tiled = st->x_layout == ABQ_LAYOUT_TILED || st->w_layout == ABQ_LAYOUT_TILED;
-    const int mask = 1 << (any_fp6 ? ABQ_LAYOUT_FP6 : any_tiled ? ABQ_LAYOUT_TILED : ABQ_LAYOUT_PLANES);
-    TunedTile t;
-    if (!tuning_find(c.x_bits, c.w_bits, c.is_signed, st->M, st->N, st->K, 0, mask, &t))
-        return;
-    if (t.cfg.nstage == kRowsStage)
-        return; // (carries group scales only)
+    int mask = 1 << (any_fp6 ? ABQ_LAYOUT_FP6 : any_tiled ? ABQ_LAYOUT_TILED : ABQ_LAYOUT_PLANES);
+    if (may_split_k(st) && k_parts_that_fit(c.x_bits, c.w_bits, st->M, st->N, st->K) > 1)
+        mask |= kPartsBit;
+    if (!tuning_find(c.x_bits, c.w_bits, c.is_signed, st->M, st->N, st->K, 0, mask, t))
+        return false;
+    if (t->cfg.nstage == kRowsStage)
+        return false; // (carries group scales only)
     // the decode kernel on prepared operands converts activations that arrive as planes into the workspace, like the
     // prefill kernels; it cannot be chosen before there is one
-    if (t.cfg.nstage == 6 && st->x_layout != ABQ_LAYOUT_TILED &&
+    if (t->cfg.nstage == 6 && st->x_layout != ABQ_LAYOUT_TILED &&
         (!st->workspace || st->workspace_bytes < planes_bytes(st->M, st->K, c.x_bits)))
+        return false;
+    if (t->cfg.nstage == 6 && !decode_tiled_flips_ok(st))
+        return false;
+    return true;
+}
+
+// Moves a state to that tile.
+static void apply_tuned(abq_gemm_state *st)
+{
+    TunedTile t;
+    if (!tuned_tile(st, &t) || memcmp(&t.cfg, &st->cfg, sizeof(abq_tile_config)) == 0)
         return;
-    if (t.cfg.nstage == 6 && !decode_tiled_flips_ok(st))
-        return;
-    if (memcmp(&t.cfg, &st->cfg, sizeof(abq_tile_config)) == 0)
-        return;
+    const abq_tile_config &c = st->cfg;
     abq_gemm_state tmp = *st;
     if (resolve(&t.cfg, c.x_bits, c.w_bits, c.is_signed, st->M, st->N, st->K, &tmp) == ABQ_OK)
         *st = tmp;
@@ -1510,8 +1520,9 @@ static void apply_tuned(abq_gemm_state *st)
 //   W4A8  128 x 5120 x 13824 27.5 / 23.0, 128 x 2048 x 16384 23.8 / 18.0;  W4A4 22.6 / 21.4;  W2A2 128 x 4096 x 11008 17.3 / 15.9
 // Two parts (86 to 128 tiles) move as many bytes per compute unit as the 64x64 tile did: 512 x 2048 x 8192 W8A8 21.9 / 24.0, W2A2
 // 17.0 / 19.5.  Shorter parts lose to the second pass over the result what they gain: W8A8 below 16 K tiles (128 x 5120 x 5120
-// 16.7 / 16.8 in three), the others below 28 (W4A8 100 x 4096 x 6144 13.9 / 14.1 in two).  W2A8 is as fast on its 64x64 tile with four
-// K groups (128 x 5120 x 13824 23.0 / 23.4).
+// 16.7 / 16.8 in three), the others below 28 (W4A8 100 x 4096 x 6144 13.9 / 14.1 in two).  W2A8 was as fast on its 64x64 tile with four
+// K groups (unsigned 128 x 5120 x 13824 23.0 / 23.4; the autotune harness, whose weights come from memory throughout, has 27.0 / 23.6
+// there and 25.2 / 21.9 signed, and the table of measured tiles names the parts for that shape).
 static int k_parts_that_pay(int x_bits, int w_bits, int M, int N, int K)
 {
     const int m_blocks = (M + 127) / 128, parts = k_parts_that_fit(x_bits, w_bits, M, N, K);
@@ -1531,8 +1542,8 @@ static bool runs_on_row_sums(const abq_gemm_state *st, const KernelEntry &e)
 // that gathers them itself, which has no parts.
 static bool may_split_k(const abq_gemm_state *st)
 {
-    if (st->strategy != ABQ_STRATEGY_TILED || !st->auto_chosen || st->out_kind != ABQ_OUT_I32 || st->group_size || st->act ||
-        st->x_layout != ABQ_LAYOUT_PLANES || st->w_layout != ABQ_LAYOUT_TILED)
+    if (!st->auto_chosen || st->out_kind != ABQ_OUT_I32 || st->group_size || st->act || st->x_layout != ABQ_LAYOUT_PLANES ||
+        st->w_layout != ABQ_LAYOUT_TILED)
         return false;
     const KernelTable *t = find_table(registry().tiled, st->cfg.x_bits, st->cfg.w_bits, st->cfg.is_signed);
     const int v = parts_entry(t);
@@ -1551,9 +1562,16 @@ static void settle(abq_gemm_state *st)
 {
     if (!may_split_k(st))
         return;
+    // (a measured tile comes before the rule)
+    TunedTile tuned;
+    if (tuned_tile(st, &tuned)) {
+        if (tuned.cfg.nstage == kPartsStage)
+            apply_tuned(st);
+        return;
+    }
     const abq_tile_config &c = st->cfg;
     const KernelTable *t = find_table(registry().tiled, c.x_bits, c.w_bits, c.is_signed);
-    const int parts = k_parts_that_pay(c.x_bits, c.w_bits, st->M, st->N, st->K);
+    const int parts = st->strategy == ABQ_STRATEGY_TILED ? k_parts_that_pay(c.x_bits, c.w_bits, st->M, st->N, st->K) : 1;
     if (parts > 1)
         set_k_parts(st, t, parts_entry(t), parts);
 }

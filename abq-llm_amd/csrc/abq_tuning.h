@@ -10,10 +10,14 @@ struct TunedTile {
     float tops;
 };
 
-// abq_layout both operands of a tile are read in: ABQ_LAYOUT_FP6 (MMA 32x32x64), ABQ_LAYOUT_TILED (NSTAGE 4, 6 and 7),
-// else ABQ_LAYOUT_PLANES.  (A kernel on prepared layouts also takes operands still in planes and converts them into the
+// abq_layout both operands of a tile are read in: ABQ_LAYOUT_FP6 (MMA 32x32x64), ABQ_LAYOUT_TILED (NSTAGE 4, 6, 7 and
+// 8), else ABQ_LAYOUT_PLANES.  (A kernel on prepared layouts also takes operands still in planes and converts them into the
 // caller's workspace; what counts for a lookup is the layout the weights are held in.)
 int tile_operand_layout(const abq_tile_config &c);
+
+// The tile whose K is split over several workgroups (NSTAGE 8) runs on K-tiled weights like others, but for int32 results of
+// activations in planes only: its entries have a bit of their own in a lookup's mask.
+constexpr int kPartsStage = 8, kPartsBit = 1 << 8;
 
 // The fastest entry for this GEMM among those whose layout has its bit (1 << abq_layout) set in layout_mask; entries
 // loaded at run time come before the compiled-in ones.

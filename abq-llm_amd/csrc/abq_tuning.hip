@@ -11,7 +11,7 @@
 // One line per entry, '#' starts a comment:
 //     <kernel name> <M> <N> <K> <group size> <TOPS>
 // The kernel name carries bit widths, signedness and the tile tuple (abq_parse_kernel_name); the tuple says which
-// operand layout the tile runs on (NSTAGE 5: FP6 records; NSTAGE 4, 6 and 7: K-tiled; else planes).  An entry serves
+// operand layout the tile runs on (NSTAGE 5: FP6 records; NSTAGE 4, 6, 7 and 8: K-tiled; else planes).  An entry serves
 // the M of its bucket (1, 2, 3-4, 5-8, 9-16, 17-32, 33-64, ...) on exactly its N, K and group size.  A file may hold
 // several entries per shape, e.g. the best tile of each layout: a lookup takes the fastest among those the caller
 // can run.
@@ -91,7 +91,7 @@ const TunedTile *best_of(const std::vector<TunedTile> &table, int x_bits, int w_
         if (t.cfg.x_bits != x_bits || t.cfg.w_bits != w_bits || (t.cfg.is_signed != 0) != (is_signed != 0) || t.N != N || t.K != K ||
             t.group_size != group || m_bucket(t.M) != bucket)
             continue;
-        if (!(layout_mask & (1 << tile_operand_layout(t.cfg))))
+        if (!(layout_mask & (t.cfg.nstage == kPartsStage ? kPartsBit : 1 << tile_operand_layout(t.cfg))))
             continue;
         // among the entries of a table the fastest; at equal figures the later line
         if (!best || t.tops >= best->tops)
@@ -106,7 +106,7 @@ int tile_operand_layout(const abq_tile_config &c)
 {
     if (c.mma_m == 32 && c.mma_n == 32 && c.mma_k == 64)
         return ABQ_LAYOUT_FP6;
-    if ((c.mma_m == 32 && c.mma_k == 32 && c.nstage == 4) || (c.mma_m == 16 && c.mma_k == 64 && (c.nstage == 6 || c.nstage == 7)))
+    if ((c.mma_m == 32 && c.mma_k == 32 && (c.nstage == 4 || c.nstage == kPartsStage)) || (c.mma_m == 16 && c.mma_k == 64 && (c.nstage == 6 || c.nstage == 7)))
         return ABQ_LAYOUT_TILED;
     return ABQ_LAYOUT_PLANES;
 }
@@ -213,7 +213,10 @@ abq_status abq_tuning_lookup(int x_bits, int w_bits, int is_signed, int M, int N
     if (!cfg)
         return ABQ_ERR_INVALID_ARG;
     TunedTile t;
-    if (!tuning_find(x_bits, w_bits, is_signed, M, N, K, group_size, layout_mask ? layout_mask : 7, &t))
+    int mask = layout_mask ? layout_mask & 7 : 7;
+    if (mask & 1 << ABQ_LAYOUT_TILED)
+        mask |= kPartsBit;
+    if (!tuning_find(x_bits, w_bits, is_signed, M, N, K, group_size, mask, &t))
         return ABQ_ERR_UNSUPPORTED;
     *cfg = t.cfg;
     if (tops)
@@ -230,7 +233,7 @@ int abq_preferred_weight_layout(int x_bits, int w_bits, int is_signed, int M, in
     if (activations_run_padded(x_bits, w_bits, is_signed, M, group_size))
         return ABQ_LAYOUT_TILED; // (whatever was measured on the pair's own kernels: the padded pair's run on these)
     TunedTile t;
-    if (tuning_find(x_bits, w_bits, is_signed, M, N, K, group_size, 7, &t))
+    if (tuning_find(x_bits, w_bits, is_signed, M, N, K, group_size, 7 | kPartsBit, &t))
         return tile_operand_layout(t.cfg);
     // no measurement: FP6 records for the pairs that qualify once the GEMM is prefill-sized (the FP6 matrix cores run
     // at twice the int8 rate and nothing is unpacked), K-tiled records otherwise (every decode and prefill kernel

@@ -586,7 +586,7 @@ int main(int argc, char **argv)
         const bool via_padded = !cfg && pad_weights && d_wpad != nullptr;
         const bool both = prepared || (cfg ? cfg->nstage == 6 : (tuned_decode && !via_padded));
         const bool fp6 = cfg ? cfg->nstage == 5 : (!prepared && !via_padded && M > 16 && preferred == ABQ_LAYOUT_FP6 && fp6_ok);
-        const bool tiled = both || via_padded || (cfg ? cfg->nstage == 4 : (M > 16 && !fp6 && preferred != ABQ_LAYOUT_PLANES));
+        const bool tiled = both || via_padded || (cfg ? cfg->nstage == 4 || cfg->nstage == 8 : (M > 16 && !fp6 && preferred != ABQ_LAYOUT_PLANES));
         if (fp6 && !fp6_ok) {
             t.status = -1;
             return;
@@ -665,21 +665,26 @@ int main(int argc, char **argv)
 
     double best_tops = 0;
     std::string best;
-    // the fastest tile of each operand layout (planes, K-tiled, FP6), for --tuning-out
-    double layout_tops[3] = { 0, 0, 0 };
-    abq_tile_config layout_best[3];
+    // the fastest tile of each operand layout (planes, K-tiled, FP6), for --tuning-out; the tile with K in parts runs for some of the
+    // calls on K-tiled weights only and has a line of its own
+    double layout_tops[4] = { 0, 0, 0, 0 };
+    abq_tile_config layout_best[4];
     std::vector<abq_tile_config> tiles;
     for (int i = 0; i < abq_native_config_count(x_bits, w_bits, is_signed); ++i) {
         abq_tile_config cfg;
         if (abq_native_config_get(x_bits, w_bits, is_signed, i, &cfg) == ABQ_OK)
             tiles.push_back(cfg);
     }
-    // ... and the 64 x 64 tile whose four groups of waves split K, which the native list leaves out, where the pair has it
+    // ... and the tiles the native list leaves out, where the pair and the shape have them: 64 x 64 with four groups of waves that split
+    // K, and 128 x 64 with K in parts over several workgroups
     if (M > 16) {
-        const abq_tile_config four = { x_bits, w_bits, is_signed, 64, 64, 512, 32, 32, 128, 32, 32, 32, 4 };
-        abq_gemm_state probe;
-        if (abq_gemm_init(&four, 0, 0, 0, d_xp, d_xp, M, N, K, d_xp, nullptr, 0, ABQ_OUT_I32, &probe) == ABQ_OK)
-            tiles.push_back(four);
+        const abq_tile_config further[] = { { x_bits, w_bits, is_signed, 64, 64, 512, 32, 32, 128, 32, 32, 32, 4 },
+                                            { x_bits, w_bits, is_signed, 128, 64, x_bits + w_bits <= 8 ? 256 : 128, 64, 32, 128, 32, 32, 32, 8 } };
+        for (const abq_tile_config &cfg : further) {
+            abq_gemm_state probe;
+            if (abq_gemm_init(&cfg, 0, 0, 0, d_xp, d_xp, M, N, K, d_xp, nullptr, 0, ABQ_OUT_I32, &probe) == ABQ_OK)
+                tiles.push_back(cfg);
+        }
     }
     const int ncfg = (int)tiles.size();
     // + the library's choice (+ its choice on prepared operands (+ the same with the weights padded as well))
@@ -724,7 +729,7 @@ int main(int argc, char **argv)
             best = buf;
         }
         if (t.status == 0 && !library_default) {
-            const int layout = c.nstage == 5 ? ABQ_LAYOUT_FP6 : (c.nstage == 4 || c.nstage == 6) ? ABQ_LAYOUT_TILED : ABQ_LAYOUT_PLANES;
+            const int layout = c.nstage == 8 ? 3 : c.nstage == 5 ? ABQ_LAYOUT_FP6 : (c.nstage == 4 || c.nstage == 6) ? ABQ_LAYOUT_TILED : ABQ_LAYOUT_PLANES;
             if (tops > layout_tops[layout]) {
                 layout_tops[layout] = tops;
                 layout_best[layout] = c;
@@ -740,7 +745,7 @@ int main(int argc, char **argv)
             std::printf("Error, cannot append to %s\n", tuning_out.c_str());
             return -1;
         }
-        for (int layout = 0; layout < 3; ++layout) {
+        for (int layout = 0; layout < 4; ++layout) {
             if (layout_tops[layout] <= 0)
                 continue;
             char name[160];

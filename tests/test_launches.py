@@ -209,3 +209,31 @@ def test_parts_of_k_run_by_name(tmp_path):
 def test_halves_are_never_added_in_parts(tmp_path, out_kind):
     (r,) = launches(tmp_path, [dict(q=8, p=8, signed=1, M=128, N=5120, K=13824, layouts=(0, 1), workspace=1 << 30, out_kind=out_kind)])
     assert r["tile"] == tile64(8, 8, 1, 1) and r["launches"][-1]["kernel"].startswith("gemm_mfma_staged<") and r["grid"] == [160, 1, 1]
+
+
+def test_a_measured_tile_comes_before_parts_of_k(tmp_path):
+    c = dict(q=8, p=8, signed=1, M=128, N=4096, K=8192, layouts=(0, 1), workspace=1 << 30)
+    entry = lambda name, tops: "%s 128 4096 8192 0 %s" % (name, tops)  # noqa: E731
+    tile, parts = "AqBMMA_8x8xtrue_128x64x256_64x32x128_32x32x32_4", parts_tile(8, 8, 1)
+    decode = "AqBMMA_8x8xtrue_16x32x512_16x32x64_16x16x64_6"
+    by_rule, by_tile, behind, ahead, elsewhere, other_m, decoding = launches(tmp_path, [dict(c, tuning=t) for t in (
+        [], [entry(tile, 500)], [entry(parts, 400), entry(tile, 500)], [entry(parts, 500), entry(tile, 400)], [entry(tile, 500).replace("4096", "4224")])] +
+        [dict(c, M=90, tuning=[entry(parts, 500)]), dict(c, tuning=[entry(decode, 500)])])
+    for r in (by_rule, ahead, elsewhere):
+        assert split(dict(r, **c)) == 4 and r["tile"] == parts, r
+    for r in (by_tile, behind):
+        assert split(dict(r, **c)) == 1 and r["tile"] == tile, r
+    assert split(dict(other_m, **dict(c, M=90))) == 4  # (an entry serves the rows of its bucket, where the rule would not split)
+    assert decoding["tile"] == decode and decoding["launches"][-1]["kernel"].startswith("gemm_decode_tiled<")
+    # an entry of the split tile says nothing of calls it does not run: activations as records, halves, row sums that are not there
+    rest = [dict(c, layouts=(1, 1)), dict(c, out_kind=3), dict(c, signed=0)]
+    entries = [entry(parts, 500), entry(parts_tile(8, 8, 0), 500)]
+    for c_, with_entry, without in zip(rest, launches(tmp_path, [dict(r, tuning=entries) for r in rest]), launches(tmp_path, rest)):
+        assert with_entry["status"] == 0 and with_entry["tile"] == without["tile"] and with_entry["launches"] == without["launches"], c_
+
+
+def test_the_compiled_in_table_holds_parts_of_k_where_they_were_measured(tmp_path):
+    calls = [dict(q=q, p=p, signed=s, M=128, N=5120, K=13824, layouts=(0, 1), workspace=1 << 30, builtin=True, **({} if s or q < 8 else {"row_sums": (0, 0xB00000)}))
+             for q, p in ((2, 2), (4, 4), (4, 2), (8, 8), (8, 4), (8, 2)) for s in (1, 0)]
+    for c, r in zip(calls, launches(tmp_path, calls)):
+        assert split(dict(r, **c)) == 3 and r["tile"] == parts_tile(c["q"], c["p"], c["signed"]), (c, r)
