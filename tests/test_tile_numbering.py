@@ -10,14 +10,10 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 SOURCE = r"""
 #define __device__
-#define __host__
 #define __forceinline__ inline
 #include <algorithm>
-#include <stdint.h>
 using std::min;
-namespace abq {
-%s
-}
+#include "abq_tile_numbering.h"
 extern "C" int tile(int id, int m_blocks, int n_blocks, int *mb, int *nb) { return abq::tile_of_workgroup(id, m_blocks, abq::tile_columns(m_blocks, n_blocks), mb, nb) && *nb < n_blocks; }
 extern "C" unsigned grid(int m_blocks, int n_blocks) { return abq::tile_grid(m_blocks, n_blocks); }
 """
@@ -25,13 +21,10 @@ extern "C" unsigned grid(int m_blocks, int n_blocks) { return abq::tile_grid(m_b
 
 @pytest.fixture(scope="module")
 def numbering(tmp_path_factory):
-    text = open(os.path.join(ROOT, "abq-llm_amd", "csrc", "abq_kernels.h")).read()
-    first = text.index("constexpr int kSpreadM")
-    last = text.index("}\n", text.index("inline unsigned tile_grid")) + 2
     d = tmp_path_factory.mktemp("numbering")
     src, lib = d / "numbering.cpp", d / "numbering.so"
-    src.write_text(SOURCE % text[first:last])
-    subprocess.check_call(["g++", "-O1", "-shared", "-fPIC", "-o", str(lib), str(src)])
+    src.write_text(SOURCE)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "abq-llm_amd", "csrc"), "-o", str(lib), str(src)])
     return ctypes.CDLL(str(lib))
 
 
