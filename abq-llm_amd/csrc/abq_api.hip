@@ -1550,16 +1550,65 @@ static bool may_split_k(const abq_gemm_state *st)
     return v >= 0 && (!runs_on_row_sums(st, t->entries[v]) || row_sums_at_hand(st));
 }
 
+// Unsigned activations of several fields that arrive as planes, against K-tiled weights of one narrower field (W2A6), on the
+// library's own choice of tile: exec converts the activations anyway, and as records of the next single-field width (their
+// codes stay below 128: no value - 128, no row sums) they run on the LDS-staged kernel, where the odd widths' own kernel is
+// staged through registers (W2A6, 128 rows, kernel alone: 5120 x 13824 50.9 against 22.5 us, 13824 x 5120 27.6 against 19.3).
+static bool unsigned_pads_activations(const abq_gemm_state *st)
+{
+    const abq_tile_config &c = st->cfg;
+    return !c.is_signed && st->strategy == ABQ_STRATEGY_TILED && st->auto_chosen && st->M > 16 && !st->group_size && !st->act &&
+           st->x_layout == ABQ_LAYOUT_PLANES && st->w_layout == ABQ_LAYOUT_TILED && !one_field(c.x_bits) && one_field(c.w_bits) &&
+           c.w_bits < 8 && st->reserved[2] == 0 && st->reserved[3] == 0;
+}
+
+// reserved[4] bit 12: settle made the state the padded pair's for that (signed pairs: abq_gemm_set_operand_layout), with the codes'
+// own widths as value bits.
+constexpr int kWidened = 1 << 12;
+static bool widened(const abq_gemm_state *st) { return (st->reserved[4] & kWidened) != 0; }
+
+// ... where the workspace holds the wider records, and no tile of the own pair was measured ahead of the padded one's (no measurement of
+// the padded pair: behind).
+static void widen_activations(abq_gemm_state *st)
+{
+    if (!unsigned_pads_activations(st) || !st->workspace || st->workspace_bytes < planes_bytes(st->M, st->K, abq_padded_bits(st->cfg.x_bits)))
+        return;
+    abq_gemm_state wide = *st;
+    wide.reserved[2] = st->cfg.x_bits;
+    wide.reserved[3] = st->cfg.w_bits;
+    wide.cfg.x_bits = abq_padded_bits(st->cfg.x_bits);
+    if (switch_to_tiled(&wide) != ABQ_OK)
+        return;
+    TunedTile own, padded;
+    if (tuned_tile(st, &own) && !(tuned_tile(&wide, &padded) && padded.tops >= own.tops))
+        return;
+    apply_tuned(&wide);
+    wide.reserved[4] |= kWidened;
+    *st = wide;
+}
+
+static void narrow_activations(abq_gemm_state *st)
+{
+    st->cfg.x_bits = st->reserved[2];
+    st->reserved[2] = st->reserved[3] = 0;
+    st->reserved[4] &= ~kWidened;
+    (void)switch_to_tiled(st);
+    apply_tuned(st);
+}
+
 // What a state runs follows from everything that has been declared of it: each declaration takes the last of these decisions back
 // (unsettle), does its own part, and has it made again (settle).
 static void unsettle(abq_gemm_state *st)
 {
-    if (st->auto_chosen && k_parts(st) > 1)
+    if (widened(st))
+        narrow_activations(st);
+    else if (st->auto_chosen && k_parts(st) > 1)
         (void)switch_to_tiled(st); // (the tile of the rules, which the state was on)
 }
 
 static void settle(abq_gemm_state *st)
 {
+    widen_activations(st);
     if (!may_split_k(st))
         return;
     // (a measured tile comes before the rule)
@@ -1758,31 +1807,27 @@ abq_status abq_gemm_exec_static(const abq_gemm_state *st, void *stream)
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
+    // (what an unsigned state runs depends on the workspace: wider activation records that it holds, row sums that may be had from the
+    // planes)
+    abq_gemm_state local = *st;
+    if (!local.cfg.is_signed)
+        unsettle(&local);
     // only the strategies on prepared layouts convert anything
-    const bool converts = st->strategy == ABQ_STRATEGY_TILED || st->strategy == ABQ_STRATEGY_FP6 || st->strategy == ABQ_STRATEGY_DECODE_TILED;
-    const size_t need = converts ? least_workspace_bytes(st) : 0;
+    const bool converts = local.strategy == ABQ_STRATEGY_TILED || local.strategy == ABQ_STRATEGY_FP6 || local.strategy == ABQ_STRATEGY_DECODE_TILED;
+    const size_t need = converts ? least_workspace_bytes(&local) : 0;
     if (need > (size_t)ABQ_STATIC_WORKSPACE_BYTES) {
         fprintf(stderr, "[ABQ][Error] abq_gemm_exec_static: this GEMM converts %zu bytes of operands, the static workspace holds %zu\n",
                 need, (size_t)ABQ_STATIC_WORKSPACE_BYTES);
         return ABQ_ERR_TOO_LARGE;
     }
-    abq_gemm_state local = *st;
     if (need) {
-        void *ptr = nullptr;
-        const abq_status rc = static_scratch_address(&ptr);
+        const abq_status rc = static_scratch_address(&local.workspace);
         if (rc != ABQ_OK)
             return rc;
-        auto take = [&]() {
-            local.workspace = ptr;
-            local.workspace_bytes = ABQ_STATIC_WORKSPACE_BYTES;
-        };
-        if (local.cfg.is_signed) {
-            take();
-        } else { // (row sums may be had from the planes now)
-            const Declaration declaration(&local);
-            take();
-        }
+        local.workspace_bytes = ABQ_STATIC_WORKSPACE_BYTES;
     }
+    if (!local.cfg.is_signed)
+        settle(&local);
     return abq_gemm_exec(&local, stream);
 }
 
@@ -1839,7 +1884,7 @@ static void repick_unsigned_tile(abq_gemm_state *st)
 // Whether the state's kernel is one that wants row sums handed in.
 static bool wants_row_sums(const abq_gemm_state *st)
 {
-    if (st->group_size || st->cfg.is_signed || (st->cfg.x_bits != 8 && st->cfg.w_bits != 8))
+    if (st->group_size || st->cfg.is_signed || widened(st) || (st->cfg.x_bits != 8 && st->cfg.w_bits != 8))
         return false;
     if (st->strategy == ABQ_STRATEGY_DECODE_TILED) {
         int fx, fw;
@@ -1987,42 +2032,10 @@ abq_status abq_relayout_planes_folded(const uint32_t *planes, const float *w_zer
                                                     is_signed ? 1 : 0, misfit_dev, (hipStream_t)stream));
 }
 
-// Unsigned activations of several fields that arrive as planes, against K-tiled weights of one narrower field, on the
-// library's own choice of tile: exec converts the activations anyway, and as records of the next single-field width (their
-// codes stay below 128: no value - 128, no row sums) they run on the LDS-staged kernel, where the odd widths' own kernel is
-// staged through registers (W2A6, 128 rows, kernel alone: 5120 x 13824 50.9 against 22.5 us, 13824 x 5120 27.6 against 19.3).
-// The state keeps its own pair (signed pairs become the padded one: abq_gemm_set_operand_layout); what runs is decided per call
-// from the workspace, which holds the wider records or does not.
-static bool unsigned_pads_activations(const abq_gemm_state *st)
-{
-    const abq_tile_config &c = st->cfg;
-    return !c.is_signed && st->strategy == ABQ_STRATEGY_TILED && st->auto_chosen && st->M > 16 && !st->group_size && !st->act &&
-           st->x_layout == ABQ_LAYOUT_PLANES && st->w_layout == ABQ_LAYOUT_TILED && !one_field(c.x_bits) && one_field(c.w_bits) &&
-           c.w_bits < 8 && st->reserved[2] == 0 && st->reserved[3] == 0;
-}
-
-static bool run_unsigned_padded(const abq_gemm_state *st, abq_gemm_state *padded)
-{
-    if (!unsigned_pads_activations(st) || !st->workspace ||
-        st->workspace_bytes < planes_bytes(st->M, st->K, abq_padded_bits(st->cfg.x_bits)))
-        return false;
-    *padded = *st;
-    padded->reserved[2] = st->cfg.x_bits;
-    padded->reserved[3] = st->cfg.w_bits;
-    padded->cfg.x_bits = abq_padded_bits(st->cfg.x_bits);
-    if (switch_to_tiled(padded) != ABQ_OK)
-        return false;
-    apply_tuned(padded);
-    return true;
-}
-
 abq_status abq_gemm_exec(const abq_gemm_state *st, void *stream)
 {
     if (!st || !st->init_success)
         return ABQ_ERR_NOT_INITIALIZED;
-    abq_gemm_state padded;
-    if (run_unsigned_padded(st, &padded))
-        st = &padded;
     const bool x_dynamic = st->x_layout == ABQ_LAYOUT_F16 && st->reserved[1] != 0; // the kernel takes the token scales itself
     if (st->out_kind == ABQ_OUT_F16_SCALED && ((!st->x_scale && !x_dynamic) || !st->w_scale))
         return ABQ_ERR_INVALID_ARG;

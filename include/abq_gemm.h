@@ -195,7 +195,8 @@ typedef struct abq_gemm_state {
                               runs (cfg is then that of the tile it stands in for, or its own if asked for;
                               grid_dim, block_dim and shared_mem_size are its own); bits 8 to 11: parts of K (NSTAGE 8),
                               0 for one.  D is then cleared first and added into: while a call is under way nothing else may
-                              write or read it, another call on the same state included */
+                              write or read it, another call on the same state included; bit 12 see
+                              abq_gemm_workspace_bytes */
     /* K-tiled operands (ABQ_STRATEGY_TILED) */
     int x_layout, w_layout;  /* abq_layout of X and W as handed to init                    */
     int auto_chosen;         /* 1 if the tile was the library's choice                     */
@@ -514,9 +515,10 @@ abq_status abq_gemm_set_padded_activations(abq_gemm_state *state, int padded);
  * (ABQ_STRATEGY_FP6) with its current operand layouts: the converted copies of the operands still in
  * the reference layout.  Operands declared K-tiled (FP6 records) count 0, and so do fp16 activations
  * handed to the decode kernel (ABQ_LAYOUT_F16: quantised inside the kernel, nothing is converted).
- * Unsigned activations of several fields that stay in planes against K-tiled weights of 2 or 4 bits (W2A6), above 16
- * rows: the bytes of 8-bit records, on which the LDS-staged kernel runs; with a smaller workspace that holds records of
- * their own width abq_gemm_exec runs the pair's own kernel, slower. */
+ * Unsigned W2A6 whose activations stay in planes against K-tiled weights, above 16 rows: the bytes of 8-bit records.  A state
+ * whose workspace holds them is the padded pair's (cfg.x_bits 8, reserved[4] bit 12) and runs the LDS-staged kernel, unless a
+ * tile of its own pair was measured ahead; with a smaller workspace that holds records of their own width it runs the
+ * pair's own kernel, slower. */
 size_t abq_gemm_workspace_bytes(const abq_gemm_state *state);
 
 /* Hands a caller-owned device buffer to the state.  If the tile was the library's choice, M > 64

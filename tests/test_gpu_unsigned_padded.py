@@ -26,8 +26,9 @@ def test_unsigned_activations_of_several_fields(abq, oracle, M, N, K):
     for size in (g.workspace_bytes, M * K - 1, M * K * 6 // 8):  # the wider records, and two workspaces that hold the pair's own only
         ws = torch.empty(size, dtype=torch.uint8, device="cuda")
         g = abq.Gemm(xd, wt, False, w_tiled=True, workspace=ws)
+        assert g.state.cfg.x_bits == (8 if size >= M * K else 6)
         assert np.array_equal(g.run().cpu().numpy(), want), (size, M, N, K)
-    assert np.array_equal(g.run_static().cpu().numpy(), want)
+        assert np.array_equal(g.run_static().cpu().numpy(), want), (size, M, N, K)
     scale = torch.full((1,), 0.125, device="cuda")  # another epilogue: half(sum) * half(scale)
     g = abq.Gemm(xd, wt, False, w_tiled=True, workspace=torch.empty(M * K, dtype=torch.uint8, device="cuda"),
                  out_kind=abq.OUT_F16_TENSOR_F32SCALE, c_scale=scale)

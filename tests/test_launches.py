@@ -237,3 +237,24 @@ def test_the_compiled_in_table_holds_parts_of_k_where_they_were_measured(tmp_pat
              for q, p in ((2, 2), (4, 4), (4, 2), (8, 8), (8, 4), (8, 2)) for s in (1, 0)]
     for c, r in zip(calls, launches(tmp_path, calls)):
         assert split(dict(r, **c)) == 3 and r["tile"] == parts_tile(c["q"], c["p"], c["signed"]), (c, r)
+
+
+def test_unsigned_w2a6_states_describe_the_padded_kernel_that_runs(tmp_path):
+    """From a workspace that holds 8-bit activation records on, whatever the order of the declarations, until it is taken away; a measured
+    tile of the pair itself comes first unless the padded pair's was measured ahead."""
+    c = dict(q=6, p=2, signed=0, M=128, N=4096, K=5120, layouts=(0, 1), workspace=128 * 5120)
+    own, padded = "AqBMMA_6x2xfalse_64x64x128_32x32x128_32x32x32_4", "AqBMMA_8x2xfalse_64x64x512_32x32x128_32x32x32_4"
+    entry = lambda name, tops: "%s 128 4096 5120 0 %s" % (name, tops)  # noqa: E731
+    wide = [c, dict(c, order=["workspace", "layouts"]), dict(c, out_kind=3), dict(c, M=17, N=64, K=512), dict(c, M=2048, workspace=1 << 30),
+            dict(c, tuning=[entry(own, 300), entry(padded, 400)]), dict(c, tuning=[entry(padded, 400)]), dict(c, workspace=1024, then=[["workspace", 1 << 30]])]
+    narrow = [dict(c, workspace=128 * 5120 - 1), dict(c, tuning=[entry(own, 300)]), dict(c, tuning=[entry(own, 500), entry(padded, 400)]),
+              dict(c, then=[["workspace", 128 * 5120 * 6 // 8]])]
+    for r in launches(tmp_path, wide):
+        convert, made = r["launches"]
+        assert r["status"] == 0 and r["tile"].startswith("AqBMMA_8x2xfalse_") and re.match(r"relayout_planes(_ws)?_kernel<8>$", convert["kernel"]), r
+        assert made["kernel"].startswith("gemm_mfma_staged<8, 2, false") and (made["grid"], made["block"]) == (r["grid"], r["block"]), r
+    for r in launches(tmp_path, narrow):
+        assert r["status"] == 0 and r["tile"].startswith("AqBMMA_6x2xfalse_") and r["launches"][-1]["kernel"].startswith("gemm_mfma_tiled<6, 2, false"), r
+    # planes against planes, and pairs that are not built, are what they were
+    both, records, unbuilt = launches(tmp_path, [dict(c, layouts=(0, 0), workspace=1 << 30), dict(c, layouts=(1, 1)), dict(c, q=5)])
+    assert both["tile"].startswith("AqBMMA_6x2xfalse_") and records["tile"].startswith("AqBMMA_6x2xfalse_") and unbuilt["status"] == 3
