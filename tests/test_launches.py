@@ -258,3 +258,28 @@ def test_unsigned_w2a6_states_describe_the_padded_kernel_that_runs(tmp_path):
     # planes against planes, and pairs that are not built, are what they were
     both, records, unbuilt = launches(tmp_path, [dict(c, layouts=(0, 0), workspace=1 << 30), dict(c, layouts=(1, 1)), dict(c, q=5)])
     assert both["tile"].startswith("AqBMMA_6x2xfalse_") and records["tile"].startswith("AqBMMA_6x2xfalse_") and unbuilt["status"] == 3
+
+
+# prefills of many rows on outputs of few columns of tiles: (call, blocks of rows, columns of tiles, kernel)
+SPREAD = [(dict(q=8, p=2, signed=1, M=9500, N=1100, K=256, group=128), 75, 9, "gemm_mfma_staged<8, 2, true, false, 2, 2, 2, 2, 3, true, 1>"),
+          (dict(q=8, p=2, signed=1, M=9500, N=600, K=384), 149, 5, "gemm_mfma_staged<8, 2, true, false, 1, 2, 2, 2, 4, false, 1>"),
+          (dict(q=4, p=4, signed=1, M=9500, N=130, K=256, group=128, layouts=(2, 2)), 75, 3, "gemm_mfma_staged<6, 6, true, true, 2, 1, 2, 2, 4, true, 1>"),
+          (dict(q=4, p=4, signed=1, M=9500, N=1290, K=128, layouts=(2, 2)), 75, 11, "gemm_mfma_staged<6, 6, true, true, 2, 2, 2, 2, 3, false, 1>"),
+          (dict(q=3, p=3, signed=1, M=9500, N=130, K=128), 149, 3, "gemm_mfma_tiled<3, 3, true, 1, 1, false, 128, 2, 2>"),
+          (dict(q=3, p=3, signed=1, M=9500, N=1100, K=256), 38, 9, "gemm_mfma_tiled<3, 3, true, 2, 2, false, 128, 4, 2>"),
+          (dict(q=6, p=6, signed=0, M=9473, N=260, K=128), 75, 3, "gemm_mfma_tiled<6, 6, false, 2, 2, false, 128, 2, 2>"),
+          (dict(q=8, p=8, signed=0, M=9600, N=1160, K=256), 75, 10, "gemm_mfma_tiled<8, 8, false, 2, 2, false, 128, 2, 2>"),
+          (dict(q=8, p=4, signed=1, M=9500, N=2200, K=256, group=64), 75, 18, "gemm_mfma_tiled<8, 4, true, 2, 2, true, 128, 2, 2>")]
+
+
+def spread_grid(m_blocks, n_blocks):
+    """Workgroups where the columns left over from whole eighths are dealt out by tiles, eight blocks of rows at a time."""
+    own, left, last = n_blocks // 8, n_blocks % 8, m_blocks % 8
+    return 8 * (m_blocks // 8 * (8 * own + left) + last * own + -(-last * left // 8))
+
+
+def test_large_prefills_on_few_columns_of_tiles_launch_the_spread_grid(tmp_path):
+    for (c, m_blocks, n_blocks, kernel), r in zip(SPREAD, launches(tmp_path, [c for c, *_ in SPREAD])):
+        (made,) = r["launches"]
+        assert r["status"] == 0 and made["kernel"] == kernel and made["grid"] == r["grid"], (c, r)
+        assert r["grid"] == [spread_grid(m_blocks, n_blocks), 1, 1] and r["grid"][0] < 8 * -(-n_blocks // 8) * m_blocks, (c, r)
