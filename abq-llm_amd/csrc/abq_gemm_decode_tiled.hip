@@ -300,8 +300,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_tiled(const GemmArgs a, i
             if (4 * g + e < Mb)
                 red[((wid * T + t) * 16 + 4 * g + e) * 16 + r] = acc[t][0][e] + acc[t][1][e];
     __syncthreads();
-    for (int o = tid; o < T * 256; o += NT) {
-        const int t = o >> 8, rem = o & 255;
+    if (tid < T * 256) {
+        const int t = tid >> 8, rem = tid & 255;
         const int n = (tile0 + t) * 16 + (rem & 15);
         if ((rem >> 4) < Mb && n < N) {
             int part[NW];
@@ -527,13 +527,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_fields(const GemmArgs a, 
         if (4 * g + e < Mb)
             red[(wid * 16 + 4 * g + e) * 16 + r] = acc[0][e] + acc[1][e];
     __syncthreads();
-    for (int o = tid; o < 256; o += NT) {
-        const int n = tile0 * 16 + (o & 15);
-        if ((o >> 4) < Mb && n < N) {
+    if (tid < 256) {
+        const int n = tile0 * 16 + (tid & 15);
+        if ((tid >> 4) < Mb && n < N) {
             int part[NW];
 #pragma unroll
             for (int w = 0; w < NW; ++w)
-                part[w] = red[w * 256 + o];
+                part[w] = red[w * 256 + tid];
             int v = 0;
 #pragma unroll
             for (int w = 0; w < NW; ++w)
@@ -542,7 +542,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_decode_fields(const GemmArgs a, 
                 v >>= 16 - QP - P;
             if constexpr (FLIP_X)
                 v = (int)((unsigned)v + 128u * (unsigned)w_sum);
-            store_result(a, m0 + (o >> 4), n, v);
+            store_result(a, m0 + (tid >> 4), n, v);
         }
     }
 }
