@@ -1280,10 +1280,12 @@ hipError_t launch_pack_i32(const int32_t *in, uint32_t *planes, int rows, int k,
                            hipStream_t stream)
 {
     const size_t n_units = (size_t)rows * k / 8;
-    // Whole lines per load from 8 M elements on, where the kernel is bound by its read (grids of 4096 workgroups of at least
-    // one trip per wave); below, the waves of pack_i32_kernel have a quarter of the work each (128 x 5120: 3.5 us on either).
-    // Up to 4 bits: beyond, its arithmetic per plane would come close to the time of the loads.
-    if (bits >= 1 && bits <= 4 && n_units >= ((size_t)1 << 20) && n_units < ((size_t)1 << 30) && (reinterpret_cast<size_t>(in) & 15) == 0) {
+    // Whole lines per non-temporal load from 16 M elements on, where the codes are weights that a loader reads once (cold, 2 bits: 4096 x
+    // 4096 14.0 -> 12.2 us, 22016 x 4096 73.1 -> 64.6).  Such loads leave nothing in the Infinity Cache: codes that lie there and are
+    // packed again cost more than on the other kernel while they fit (2 bits, the same 8192 x 4096 each time 21.5 / 21.7, 12288 x 4096
+    // 31.4 / 34.8), which is why smaller operands, activations among them, stay off it (1966 x 4480 next to the GEMMs that read
+    // the planes: 0.9 us a call more).  Up to 4 bits: beyond, its arithmetic per plane would come close to the time of the loads.
+    if (bits >= 1 && bits <= 4 && n_units >= ((size_t)1 << 21) && n_units < ((size_t)1 << 30) && (reinterpret_cast<size_t>(in) & 15) == 0) {
         const uint32_t quads = (uint32_t)(n_units * 2);
         const dim3 grid(grid_for(n_units / 4));
         const pack_quad *src = reinterpret_cast<const pack_quad *>(in);

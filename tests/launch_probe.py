@@ -11,7 +11,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 def launches(tmp_path, calls):
     """calls: dicts of q, p, signed, M, N, K and optionally tile (a kernel name), layouts, group, zeros, act, row_sums, value_bits,
-    workspace, tuning (lines of a tuning table), order (of the declarations), then (further ones: [what, value]).  Returns a list of dicts: status, tile, strategy, grid, block, lds, launches."""
+    workspace, dynamic (fp16 activations quantised in the kernel, last), tuning (lines of a tuning table), order (of the declarations), then
+    (further ones: [what, value]); or pack: [rows, k, bits], a packing of int32 codes.  Returns a list of dicts: status, tile, strategy, grid, block, lds, launches."""
     so = str(tmp_path / "librecorder.so")
     if not os.path.exists(so):
         subprocess.check_call(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", os.path.join(HERE, "cpp", "launch_recorder.cpp"), "-o", so])
@@ -29,7 +30,18 @@ def main():
     rec = ctypes.CDLL(os.environ["RECORDER"])
     rec.recorder_name.restype = ctypes.c_char_p
 
+    def recorded():
+        made = []
+        for i in range(rec.recorder_count()):
+            grid, block, lds = (ctypes.c_uint32 * 3)(), (ctypes.c_uint32 * 3)(), ctypes.c_uint64()
+            rec.recorder_sizes(i, grid, block, ctypes.byref(lds))
+            made.append({"kernel": rec.recorder_name(i).decode(), "grid": list(grid), "block": list(block), "lds": lds.value})
+        return made
+
     def one(c):
+        if "pack" in c:
+            rec.recorder_clear()
+            return {"status": L.abq_pack_i32(0x100000, 0x200000, *c["pack"], None), "launches": recorded()}
         L.abq_tuning_clear()
         for line in c.get("tuning", []):
             name, m, n, k, group, tops = line.split()
@@ -56,14 +68,12 @@ def main():
             c = dict(c, **{what: value})
             if rc[-1] == 0:
                 rc.append(steps[what]())
+        if c.get("dynamic") and rc[-1] == 0:
+            rc.append(L.abq_gemm_set_dynamic_f16_activations(s, 0x100000, 1))
         rec.recorder_clear()
         if rc[-1] == 0:
             rc.append(L.abq_gemm_exec(s, None))
-        made = []
-        for i in range(rec.recorder_count()):
-            grid, block, lds = (ctypes.c_uint32 * 3)(), (ctypes.c_uint32 * 3)(), ctypes.c_uint64()
-            rec.recorder_sizes(i, grid, block, ctypes.byref(lds))
-            made.append({"kernel": rec.recorder_name(i).decode(), "grid": list(grid), "block": list(block), "lds": lds.value})
+        made = recorded()
         d3 = lambda d: [d.x, d.y, d.z]  # noqa: E731
         return {"status": rc[-1], "tile": abq.format_kernel_name(st.cfg) if rc[0] == 0 else None, "strategy": abq.STRATEGY_NAMES[st.strategy],
                 "grid": d3(st.grid_dim), "block": d3(st.block_dim), "lds": st.shared_mem_size, "launches": made}

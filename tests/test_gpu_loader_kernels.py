@@ -1,5 +1,5 @@
 """The kernels a loader brings weight matrices through, at the sizes where their variants begin and end: packing of int32
-codes by whole lines (from 2^20 units of eight codes on, 1 to 4 bits) and the activation zero point's term."""
+codes by whole lines (from 2^21 units of eight codes on, 1 to 4 bits) and the activation zero point's term."""
 import numpy as np
 import pytest
 
@@ -7,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("bits", [1, 2, 3, 4, 5])
-@pytest.mark.parametrize("rows,k", [(2047, 4096), (2048, 4096), (65551, 128), (2731, 3200)])
+@pytest.mark.parametrize("rows,k", [(2047, 4096), (2048, 4096), (65551, 128), (2731, 3200), (4095, 4096), (4096, 4096), (131103, 128), (5461, 3200)])
 def test_packing_of_large_matrices(abq, oracle, bits, rows, k):
     import torch
     g = torch.Generator(device="cuda").manual_seed(bits * 1000 + rows)

@@ -283,3 +283,10 @@ def test_large_prefills_on_few_columns_of_tiles_launch_the_spread_grid(tmp_path)
         (made,) = r["launches"]
         assert r["status"] == 0 and made["kernel"] == kernel and made["grid"] == r["grid"], (c, r)
         assert r["grid"] == [spread_grid(m_blocks, n_blocks), 1, 1] and r["grid"][0] < 8 * -(-n_blocks // 8) * m_blocks, (c, r)
+
+
+def test_only_weight_sized_codes_are_packed_past_the_caches(tmp_path):
+    lines = {(4096, 4096, 2): True, (22016, 4096, 4): True, (4095, 4096, 2): False, (1966, 4480, 2): False, (12288, 4096, 5): False, (1, 128, 1): False}
+    for (rows, k, bits), r in zip(lines, launches(tmp_path, [dict(pack=list(c)) for c in lines])):
+        (made,) = r["launches"]
+        assert r["status"] == 0 and made["kernel"].startswith("pack_i32_lines_kernel<%d>" % bits if lines[rows, k, bits] else "pack_i32_quads_kernel"), (rows, k, bits, r)
