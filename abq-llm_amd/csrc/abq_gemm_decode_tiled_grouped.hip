@@ -75,7 +75,9 @@ constexpr int dtg_ahead(int p, int t, int steps, int x)
 // G64: groups of 64, two to a K tile: lane groups 0, 1 hold the elements of the first, 2, 3 those of the second, and the
 // matrix core sums over all four, so a step runs its two instructions twice: once on all lanes and once with the
 // activations of lane groups 2, 3 zeroed; the difference is the second group's dot product.
-template <int Q, int P, bool SIGNED, int T, int B, int S, int XM, int XL, int FE, bool G64>
+// ONCE: requests as short as they get: weight loads without the test for a second block of rows, offsets of K tiles in 32 bits
+// (dtg_once).
+template <int Q, int P, bool SIGNED, int T, int B, int S, int XM, int XL, int FE, bool G64, bool ONCE>
 __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_tiled_grouped(const GemmArgs a)
 {
     static_assert(!XM || (Q == 8 && SIGNED && !G64), "in-kernel quantisation writes signed 8-bit records, groups of 128");
@@ -126,7 +128,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
         woff[t] = n * (P * 16u) + (uint32_t)g * (4u * P);
         soff[t] = (uint32_t)min((tile0 + t) * 16 + (lane >> 2), N - 1) * (uint32_t)NG;
     }
-    using Step = typename std::conditional<XM != 0, uint32_t, size_t>::type; // (records lie within 4 GiB; packed activations: no registers to spare for it)
+    using Step = typename std::conditional<ONCE, uint32_t, size_t>::type; // (records lie within 4 GiB)
     const Step wstep = (Step)N * (P * 16u), xstep = (Step)M * (Q * 16u);
     // activations: chunk `lane` (and 64 + lane) of the rows' records, past the last row's end the last chunk once more
     const uint32_t xoff = (uint32_t)m0 * (Q * 16u) + (uint32_t)min(lane, Mb * Q - 1) * 16u;
@@ -230,7 +232,7 @@ __global__ __launch_bounds__(dtg_threads(P, T, B, XM, G64)) void gemm_decode_til
             const char *wp = Wt + (Step)k_tile(i) * wstep;
 #pragma unroll
             for (int t = 0; t < T; ++t)
-                wb[i % WB][t].template issue<XM != 0>(wp, woff[t], once);
+                wb[i % WB][t].template issue<ONCE>(wp, woff[t], once);
         };
         request_acts(0);
 #pragma unroll
@@ -580,7 +582,27 @@ static size_t dtg_lds(int nw, int t, int b, int s, int rows, bool g64)
 // instances that are built: what the registers hold
 constexpr bool dtg_built(int p, int t, int b, bool g64) { return t * b * p <= (g64 && p < 8 ? 8 : 16) && t * b <= 6 && !(g64 && b == 2 && t > 1); }
 
-template <int Q, int P, bool SIGNED, int T, int B, int S, int XM, int XL, int FE, bool G64>
+// Rows quantised here, whose grid never has a second block of rows: where the short requests (ONCE) are ahead.  They bring a wave's
+// weights forward against the activations every wave of the workgroup waits for, which pays where a wave requests one tile's or
+// where most of the time is the stream; where two to four tiles go out in front of one block's quantisation the activations of the
+// workgroup's last waves stand behind the weights of its first.  One row, us without / with: W2A8 3072 x 1792 3.80 / 3.69, 8192 x 2944
+// 4.35 / 4.82, 8192 x 5504 5.6 / 5.4, 12288 x 2432 4.7 / 5.1, 22016 x 4096 8.2 / 8.1; W4A8 7424 x 2944 4.40 / 5.14.  The same one tile at
+// more than eight waves (4096 x 11008 on 11: 0.95 to 0.98 of the speed), 4-bit weights on two tiles and more than a round of
+// workgroups (9216 x 4608 0.94), 4-bit blocks of four K tiles (4096 x 4096 0.97 to 0.98).  Two to four rows: 2-bit weights level
+// or ahead up to K = 4096, 4-bit ones to 2048, behind beyond (2 x 4096 x 6144 W4A8 0.93); 8-bit weights behind but for one row of K up
+// to 2048 (4096 x 2432 0.95).
+constexpr bool dtg_once(int p, int t, int s, int b, int xm, bool crowded)
+{
+    if (xm == 1)
+        return p == 2   ? t == 1 ? !(b == 2 && crowded) : b == 2 || t == 6 || (t == 4 && s % 2 == 0)
+               : p == 4 ? t == 1 ? (b == 2 ? !crowded : s < 4) : (t == 2 && b == 2 && !crowded) || (t == 4 && s < 3)
+                        : t == 1 && s < 3;
+    if (xm == 4)
+        return b == 1 && (p == 2 || (p == 4 && s < 3));
+    return xm == 8;
+}
+
+template <int Q, int P, bool SIGNED, int T, int B, int S, int XM, int XL, int FE, bool G64, bool ONCE>
 static hipError_t launch_dtg_instance(const GemmArgs &a, hipStream_t stream)
 {
     if constexpr (!dtg_built(P, T, B, G64)) {
@@ -591,7 +613,7 @@ static hipError_t launch_dtg_instance(const GemmArgs &a, hipStream_t stream)
         size_t lds = dtg_lds(nw, T, B, S, rows, G64) + (!XM && XL ? (size_t)nw * 2 * Q * 256 : 0);
         if (XM)
             lds += (size_t)nw * ((nblocks + nw - 1) / nw) * S * rows * 128 + (size_t)rows * 128;
-        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_decode_tiled_grouped<Q, P, SIGNED, T, B, S, XM, XL, FE, G64>),
+        static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_decode_tiled_grouped<Q, P, SIGNED, T, B, S, XM, XL, FE, G64, ONCE>),
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (attr != hipSuccess)
             return attr;
@@ -599,7 +621,7 @@ static hipError_t launch_dtg_instance(const GemmArgs &a, hipStream_t stream)
             return hipErrorInvalidValue;
         const int tiles = (a.N + 15) / 16;
         const dim3 grid((tiles + T - 1) / T, (a.M + 15) / 16);
-        hipLaunchKernelGGL((gemm_decode_tiled_grouped<Q, P, SIGNED, T, B, S, XM, XL, FE, G64>), grid, dim3(64 * nw), lds, stream, a);
+        hipLaunchKernelGGL((gemm_decode_tiled_grouped<Q, P, SIGNED, T, B, S, XM, XL, FE, G64, ONCE>), grid, dim3(64 * nw), lds, stream, a);
         return hipGetLastError();
     }
 }
@@ -668,26 +690,30 @@ template <int Q, int P, bool SIGNED, bool XDYN, bool G64> static hipError_t laun
     auto go = [&](auto tt, auto bb, auto ss) -> hipError_t {
         constexpr int TT = decltype(tt)::value, BB = decltype(bb)::value, SS = decltype(ss)::value;
         if constexpr (XDYN) {
-            if (xm == 1)
-                return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 1, 0, 1, false>(a, stream);
+            if (xm == 1) {
+                constexpr bool sparse_once = dtg_once(P, TT, SS, BB, 1, false), crowded_once = dtg_once(P, TT, SS, BB, 1, true);
+                if (sparse_once != crowded_once && (TT == 1 ? nw > 8 : (tiles + TT - 1) / TT > 256))
+                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 1, 0, 1, false, crowded_once>(a, stream);
+                return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 1, 0, 1, false, sparse_once>(a, stream);
+            }
             if constexpr (TT <= 2) {
                 if (xm == 4)
-                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 4, 0, 4, false>(a, stream);
+                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 4, 0, 4, false, dtg_once(P, TT, SS, BB, 4, false)>(a, stream);
                 if constexpr (BB == 1)
-                    return launch_dtg_instance<Q, P, SIGNED, TT, 1, SS, 8, 0, 4, false>(a, stream);
+                    return launch_dtg_instance<Q, P, SIGNED, TT, 1, SS, 8, 0, 4, false, dtg_once(P, TT, SS, 1, 8, false)>(a, stream);
             }
             return hipErrorInvalidValue;
         } else {
             if (a.M == 1) {
                 if constexpr (TT <= 2)
-                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 1, 1, G64>(a, stream);
+                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 1, 1, G64, false>(a, stream);
                 return hipErrorInvalidValue;
             }
             if constexpr (Q == 8) {
                 if (a.M > 8)
-                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 2, 4, G64>(a, stream);
+                    return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 2, 4, G64, false>(a, stream);
             }
-            return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 1, 4, G64>(a, stream);
+            return launch_dtg_instance<Q, P, SIGNED, TT, BB, SS, 0, 1, 4, G64, false>(a, stream);
         }
     };
     using std::integral_constant;

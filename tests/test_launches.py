@@ -285,6 +285,20 @@ def test_large_prefills_on_few_columns_of_tiles_launch_the_spread_grid(tmp_path)
         assert r["grid"] == [spread_grid(m_blocks, n_blocks), 1, 1] and r["grid"][0] < 8 * -(-n_blocks // 8) * m_blocks, (c, r)
 
 
+def test_rows_quantised_in_the_group_scale_decode_kernel_take_short_requests_where_those_were_ahead(tmp_path):
+    """(weight bits, rows, N, K) -> whether the weight loads go out without the test for a second block of rows"""
+    ahead = {(2, 1, 3072, 1792): True, (2, 1, 4096, 4096): True, (2, 1, 4096, 8192): True, (2, 1, 4096, 11008): False, (2, 1, 4112, 2944): False,
+             (2, 1, 8192, 4096): False, (2, 1, 8192, 5504): True, (2, 1, 12288, 4096): False, (2, 1, 12288, 5504): True, (2, 1, 16384, 4096): True,
+             (2, 1, 22016, 4096): True, (4, 1, 4096, 2944): True, (4, 1, 4096, 4096): False, (4, 1, 4096, 8192): True, (4, 1, 4096, 8448): False,
+             (4, 1, 7424, 2944): False, (4, 1, 8192, 4608): True, (4, 1, 9216, 4608): False, (8, 1, 4096, 2048): True, (8, 1, 4096, 2432): False,
+             (8, 1, 8192, 1280): False, (2, 4, 4096, 4096): True, (4, 2, 4096, 2048): True, (4, 2, 4096, 6144): False, (8, 3, 4096, 2432): False}
+    calls = [dict(q=8, p=p, signed=1, M=m, N=n, K=k, group=128, dynamic=True) for p, m, n, k in ahead]
+    for c, r, want in zip(calls, launches(tmp_path, calls), ahead.values()):
+        (made,) = r["launches"]
+        assert r["status"] == 0 and re.fullmatch(r"gemm_decode_tiled_grouped<8, %d, true, \d, \d, \d, [148], 0, [14], false, %s>" % (
+            c["p"], "true" if want else "false"), made["kernel"]), (c, r)
+
+
 def test_only_weight_sized_codes_are_packed_past_the_caches(tmp_path):
     lines = {(4096, 4096, 2): True, (22016, 4096, 4): True, (4095, 4096, 2): False, (1966, 4480, 2): False, (12288, 4096, 5): False, (1, 128, 1): False}
     for (rows, k, bits), r in zip(lines, launches(tmp_path, [dict(pack=list(c)) for c in lines])):
