@@ -526,10 +526,9 @@ __device__ __forceinline__ void staged_gemm(const GemmArgs &a, const v4u *xt, co
     // unsigned pair written with the 128 already taken off (abq_relayout_planes_biased), and nothing was flipped here.
     constexpr bool MAY_BE_BIASED = !FP6 && SIGNED && QB == 8 && PB == 8 && !GROUPED;
     if constexpr (FLIP_X || FLIP_W || MAY_BE_BIASED) {
-        // (several parts of K: the sums are those of whole rows, the first part adds them)
-        const bool fix_x = part == 0 && ((FLIP_X && a.flip_x) || (MAY_BE_BIASED && a.w_row_sums != nullptr)); // X was fed as value - 128
-        const bool fix_w = part == 0 && ((FLIP_W && a.flip_w) || (MAY_BE_BIASED && a.x_row_sums != nullptr));
-        if (fix_x || fix_w) {
+        // (which operands: constants where they are known.  Asked of the arguments for each load, the sums came one latency after the
+        // other, W8A8 64x64 tiles 1 to 3 % of the call: 479 x 1024 x 1024 5.75 -> 6.02 us)
+        auto correct = [&](auto fix_x, auto fix_w) {
             int col_fix[TN];
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
@@ -565,6 +564,25 @@ __device__ __forceinline__ void staged_gemm(const GemmArgs &a, const v4u *xt, co
                     for (int j = 0; j < TN; ++j)
                         acc[i][j][e] = (int)((unsigned)acc[i][j][e] + row_fix + (unsigned)col_fix[j]);
                 }
+        };
+        using std::true_type;
+        using std::false_type;
+        // (several parts of K: the sums are those of whole rows, the first part adds them)
+        const bool fix_x = part == 0 && ((FLIP_X && a.flip_x) || (MAY_BE_BIASED && a.w_row_sums != nullptr)); // X was fed as value - 128
+        const bool fix_w = part == 0 && ((FLIP_W && a.flip_w) || (MAY_BE_BIASED && a.x_row_sums != nullptr));
+        if constexpr (FLIP_X && FLIP_W) {
+            if (fix_x && fix_w)
+                correct(true_type{}, true_type{});
+            else if (fix_x || fix_w)
+                correct(fix_x, fix_w);
+        } else if constexpr (FLIP_X) {
+            if (fix_x)
+                correct(true_type{}, false_type{});
+        } else if constexpr (FLIP_W) {
+            if (fix_w)
+                correct(false_type{}, true_type{});
+        } else if (fix_x || fix_w) { // (signed: a second copy of it cost the calls without sums 1 %)
+            correct(fix_x, fix_w);
         }
     }
     auto result = [&](int i, int j, int e) -> int {

@@ -41,3 +41,15 @@ def test_row_sums_of_rows_of_any_length(abq, oracle, q, p):
     for rows, K in [(1, 128), (5, 8192), (3, 8320), (4, 16512)]:
         v = rng.integers(0, 1 << q, (rows, K), dtype=np.int32)
         assert np.array_equal(abq.row_sums(planes_dev(oracle.pack_i32(v, q))).cpu().numpy(), v.sum(1))
+
+
+@pytest.mark.parametrize("bits", [(8, 8), (8, 7), (7, 8), (6, 6)])
+@pytest.mark.parametrize("M,N,K", [(40, 100, 1152), (300, 130, 384), (517, 1030, 256)])
+def test_w8a8_records_of_narrower_codes(abq, oracle, bits, M, N, K):
+    """Either operand, both or none fed as code - 128: the result is corrected by the sums of the one or two that are."""
+    rng = np.random.default_rng(M + bits[0])
+    x, w = (rng.integers(0, 1 << b, (r, K), dtype=np.int32) for b, r in zip(bits, (M, N)))
+    xp, wp = planes_dev(oracle.pack_i32(x, 8)), planes_dev(oracle.pack_i32(w, 8))
+    g = abq.Gemm(abq.relayout_planes(xp), abq.relayout_planes(wp), False, x_tiled=True, w_tiled=True, value_bits=bits,
+                 x_row_sums=abq.row_sums(xp), w_row_sums=abq.row_sums(wp))
+    assert np.array_equal(g.run().cpu().numpy(), oracle.np_gemm(x, w)), g.config_name
