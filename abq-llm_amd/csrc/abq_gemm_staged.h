@@ -197,8 +197,9 @@ __device__ __forceinline__ void staged_gemm(const GemmArgs &a, const v4u *xt, co
     const int flip_x = FLIP_X && a.flip_x ? (int)0x80808080u : 0, flip_w = FLIP_W && a.flip_w ? (int)0x80808080u : 0;
 
     // The scale of the whole result, asked for before anything else: loaded in the epilogue it is a memory latency there (static
-    // scales, a GEMM each of 4096 x 4096, 11008 x 4096, 4096 x 11008: W8A8 512 rows 165.4 -> 164.6 us for two copies, W4A4 2048 rows
-    // 339.0 -> 336.3; W2A8 100 rows of 2048 / 5504 112.4 -> 110.4 for four).  Without such a scale any four bytes do: a branch here
+    // scales, a GEMM each of 4096 x 4096, 11008 x 4096, 4096 x 11008, without the launches that pack the activations: W8A8 512 rows
+    // 165.4 -> 164.6 us for two copies, W4A4 2048 rows 339.0 -> 336.3; W2A8 100 rows of 2048 / 5504 112.4 -> 110.4 for four.  With
+    // the packing, timed in turn, W8A8 190.9 -> 188.5, W4A4 370.8 -> 368.2, no more than its runs differ).  Without such a scale any four bytes do: a branch here
     // would have its wait in front of the tiles' loads.
     float tensor_scale = 0.f;
     if constexpr (!GROUPED && !KP)
