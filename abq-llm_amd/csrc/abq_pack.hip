@@ -1280,12 +1280,16 @@ hipError_t launch_pack_i32(const int32_t *in, uint32_t *planes, int rows, int k,
                            hipStream_t stream)
 {
     const size_t n_units = (size_t)rows * k / 8;
-    // Whole lines per non-temporal load from 16 M elements on, where the codes are weights that a loader reads once (cold, 2 bits: 4096 x
-    // 4096 14.0 -> 12.2 us, 22016 x 4096 73.1 -> 64.6).  Such loads leave nothing in the Infinity Cache: codes that lie there and are
-    // packed again cost more than on the other kernel while they fit (2 bits, the same 8192 x 4096 each time 21.5 / 21.7, 12288 x 4096
-    // 31.4 / 34.8), which is why smaller operands, activations among them, stay off it (1966 x 4480 next to the GEMMs that read
-    // the planes: 0.9 us a call more).  Up to 4 bits: beyond, its arithmetic per plane would come close to the time of the loads.
-    if (bits >= 1 && bits <= 4 && n_units >= ((size_t)1 << 21) && n_units < ((size_t)1 << 30) && (reinterpret_cast<size_t>(in) & 15) == 0) {
+    // Whole lines per non-temporal load where the codes are weights that a loader reads once (cold, 2 bits: 4096 x 4096 14.0 -> 12.2 us,
+    // 22016 x 4096 73.1 -> 64.6).  Such loads leave nothing in the Infinity Cache, so that codes which lie there and are packed again
+    // are read from memory: 1 to 3 bits from 16 M elements on (activations of 8 to 16 M codes next to the GEMMs that read the planes,
+    // W2A2 1966 rows of 4480 and 12032, four copies: 640 / 650 us a pass; loading below 16 M: level).  4 bits from 8 M on: the
+    // planes and records that a loader makes of them are twice as large and stay in that cache in their place (W4 layers of 2304
+    // and 6528, two matrices of four between 8 and 16 M, 323 / 313 us, of 3584 and 9472, one of four, 444 / 437; 4-bit
+    // activations of 1966 x 4480 as above, W2A4 1085 / 1090).
+    // Up to 4 bits: beyond, its arithmetic per plane would come close to the time of the loads.
+    const size_t least_units = (size_t)1 << (bits == 4 ? 20 : 21);
+    if (bits >= 1 && bits <= 4 && n_units >= least_units && n_units < ((size_t)1 << 30) && (reinterpret_cast<size_t>(in) & 15) == 0) {
         const uint32_t quads = (uint32_t)(n_units * 2);
         const dim3 grid(grid_for(n_units / 4));
         const pack_quad *src = reinterpret_cast<const pack_quad *>(in);

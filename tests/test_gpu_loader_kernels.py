@@ -1,5 +1,5 @@
 """The kernels a loader brings weight matrices through, at the sizes where their variants begin and end: packing of int32
-codes by whole lines (from 2^21 units of eight codes on, 1 to 4 bits) and the activation zero point's term."""
+codes by whole lines (from 2^21 units of eight codes on, 4 bits from 2^20) and the activation zero point's term."""
 import numpy as np
 import pytest
 

@@ -300,7 +300,7 @@ def test_rows_quantised_in_the_group_scale_decode_kernel_take_short_requests_whe
 
 
 def test_only_weight_sized_codes_are_packed_past_the_caches(tmp_path):
-    lines = {(4096, 4096, 2): True, (22016, 4096, 4): True, (4095, 4096, 2): False, (1966, 4480, 2): False, (12288, 4096, 5): False, (1, 128, 1): False}
+    lines = {(4096, 4096, 2): True, (22016, 4096, 4): True, (4095, 4096, 2): False, (4095, 4096, 3): False, (2048, 4096, 4): True, (2047, 4096, 4): False, (1966, 4480, 2): False, (12288, 4096, 5): False, (1, 128, 1): False}
     for (rows, k, bits), r in zip(lines, launches(tmp_path, [dict(pack=list(c)) for c in lines])):
         (made,) = r["launches"]
         assert r["status"] == 0 and made["kernel"].startswith("pack_i32_lines_kernel<%d>" % bits if lines[rows, k, bits] else "pack_i32_quads_kernel"), (rows, k, bits, r)
