@@ -1283,7 +1283,7 @@ hipError_t launch_pack_i32(const int32_t *in, uint32_t *planes, int rows, int k,
     // Whole lines per non-temporal load where the codes are weights that a loader reads once (cold, 2 bits: 4096 x 4096 14.0 -> 12.2 us,
     // 22016 x 4096 73.1 -> 64.6).  Such loads leave nothing in the Infinity Cache, so that codes which lie there and are packed again
     // are read from memory: 1 to 3 bits from 16 M elements on (activations of 8 to 16 M codes next to the GEMMs that read the planes,
-    // W2A2 1966 rows of 4480 and 12032, four copies: 640 / 650 us a pass; loading below 16 M: level).  4 bits from 8 M on: the
+    // W2A2 1966 rows of 4480 and 12032, four copies: 638 / 651 us a pass; loading below 16 M: level).  4 bits from 8 M on: the
     // planes and records that a loader makes of them are twice as large and stay in that cache in their place (W4 layers of 2304
     // and 6528, two matrices of four between 8 and 16 M, 323 / 313 us, of 3584 and 9472, one of four, 444 / 437; 4-bit
     // activations of 1966 x 4480 as above, W2A4 1085 / 1090).
